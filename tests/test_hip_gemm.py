@@ -570,3 +570,16 @@ def test_gemm_config3prime_f16_f32(dtype, M):
     want = _oracle(a[rows], w[cols.to(DEV)].cpu().t().contiguous(), None, 32, 16)
     report = close_report(full[rows.to(DEV)][:, cols.to(DEV)], want)
     assert not report, report
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("M,N", [(3, 33), (20, 7), (130, 129)])
+def test_gemm_padded_row_major_b(dtype, M, N):
+    # B [K, N] as a view of wider rows whose stride is a whole number of
+    # 16-byte chunks while N is not: the last chunk of a row is partial
+    K = 200
+    a, b = _int_mats(M, K, N, seed=M + N, dtype=dtype)
+    wide = torch.full((K, -(-N // 8) * 8 + 8), 3.0, dtype=dtype, device=DEV)
+    wide[:, :N] = b.to(DEV)
+    got = KG.gemm_fxp_run(a.to(DEV), wide[:, :N], None, 32, 16).cpu()
+    assert torch.equal(got, _oracle(a, b, None, 32, 16))

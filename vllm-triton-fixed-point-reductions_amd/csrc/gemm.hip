@@ -71,8 +71,10 @@ int gemm_launch(const void* a, const void* b, const float* bias, void* c, int io
 
   const int esz = io_dtype == FXPR_DTYPE_F32 ? 4 : 2;
   const int ch = 16 / esz;
+  // (N-contiguous B: whole 16-byte chunks of columns only. A padded view, N
+  // not a multiple of the chunk under an aligned row stride, loads by element.)
   const bool vec = aligned(a, 16) && aligned(b, 16) && (stride_am % ch == 0 || m == 1) &&
-                   (ldb % ch == 0 || (b_ncontig ? k == 1 : n == 1));
+                   (b_ncontig ? n % ch == 0 && (ldb % ch == 0 || k == 1) : ldb % ch == 0 || n == 1);
 
   GemmArgs args{};
   args.a = a;
