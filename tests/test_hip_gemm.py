@@ -583,3 +583,33 @@ def test_gemm_padded_row_major_b(dtype, M, N):
     wide[:, :N] = b.to(DEV)
     got = KG.gemm_fxp_run(a.to(DEV), wide[:, :N], None, 32, 16).cpu()
     assert torch.equal(got, _oracle(a, b, None, 32, 16))
+
+
+# --- fp32 kernel fed by LDS DMA: 32- and 64-row tiles by 128 columns ---------
+
+
+@pytest.mark.parametrize("b_layout", ["nk", "kn"])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 16), (16, 8)])
+@pytest.mark.parametrize("M,N,K", [(1, 4, 64), (16, 128, 128), (17, 132, 68), (32, 260, 192), (33, 124, 64),
+                                   (64, 384, 132), (65, 128, 256), (130, 516, 200), (257, 1028, 60)])
+def test_gemm_f32_tile_edges(b_layout, bits, frac, M, N, K):
+    # one past and one short of a tile in M, N and K (whole K-tiles, a peeled
+    # partial one, only a partial one), unsplit, split and the automatic
+    # choice: small integers, so every K-tile dot is exact
+    a, b = _int_mats(M, K, N, seed=M + N + K, dtype=torch.float32)
+    bias = torch.arange(N, dtype=torch.float32) / 16
+    want = _oracle(a, b, bias, bits, frac)
+    for split_k in (0, 1, 2):
+        got = _run(a, b, bias, bits, frac, split_k=split_k, b_layout=b_layout)
+        assert torch.equal(got, want), mismatch_report(got, want)
+
+
+@pytest.mark.parametrize("b_layout", ["nk", "kn"])
+def test_gemm_f32_rows_do_not_depend_on_the_batch(b_layout):
+    # a row's bits are the same from the skinny, the 32- and the 64-row tiles
+    g = torch.Generator("cpu").manual_seed(8)
+    a = torch.randn(300, 1000, generator=g)
+    b = torch.randn(1000, 640, generator=g) * 0.05
+    whole = _run(a, b, b_layout=b_layout)
+    for m in (1, 16, 17, 40, 200):
+        assert torch.equal(_run(a[:m], b, b_layout=b_layout), whole[:m])

@@ -141,3 +141,15 @@ def test_gemm_workspace_follows_the_split(lib):
     assert lib.fxpr_gemm_workspace_bytes(1, 4096, 4096, BF16, 32, 0) == 0
     assert lib.fxpr_gemm_workspace_bytes(1, 4096, 4096, BF16, 32, 3) == 3 * 4096 * 4
     assert lib.fxpr_gemm_workspace_bytes(8192, 128256, 4096, BF16, 32, 0) == 0
+
+
+def test_gemm_f32_split_fills_whole_rounds(lib):
+    # fp32 beyond M = 32: the count whose 32- or 64-row tiles fall most evenly
+    # on 256 CUs (f32_plan); rows that cannot be 16-byte aligned (K not a
+    # multiple of 4) keep 512 / (output tiles)
+    assert gemm_splits(lib, 256, 4096, 4096, F32) == 4       # 256 tiles of 32 rows: 4 on every CU
+    assert gemm_splits(lib, 64, 6144, 4096, F32) == 8        # 96: 3 on every CU
+    assert gemm_splits(lib, 130, 4096, 14336, F32) == 8      # 160: 5 on every CU
+    assert gemm_splits(lib, 777, 14336, 4096, F32) == 1
+    assert gemm_splits(lib, 130, 4096, 4098, F32) == 8       # 64 tiles of 128 x 128
+    assert gemm_splits(lib, 130, 4096, 100, F32) <= 2        # 2 K-tiles

@@ -1,5 +1,5 @@
 // Fixed-point GEMM kernels instantiated for f32 inputs (see gemm_impl.h).
-#include "gemm_impl.h"
+#include "gemm_f32_impl.h"
 
 namespace fxpr {
 namespace gemm {

@@ -1252,39 +1252,64 @@ template <int DT, int BITS> int launch_stream(const GemmArgs& a, hipStream_t st)
   return launch_stream_tile<DT, BITS, StreamTile<1, 4, 4>>(a, st);
 }
 
-// Tile configuration by M. Only speed depends on it: every config issues the
-// same MFMA chain per output element.
-enum class TileId { M16, M32, M64, Big };
-inline TileId pick_tile(int64_t M) {
-  if (M <= 16) return TileId::M16;
-  if (M <= 32) return TileId::M32;
-  if (M <= 64) return TileId::M64;
-  return TileId::Big;
-}
+// Register-staged tiles: skinny rows, and a square tile for everything that
+// the DMA kernels do not take. Only speed depends on the choice: every config
+// issues the same MFMA chain per output element.
 using T16 = Tile<16, 256, 16, 64>;
-using T32 = Tile<32, 256, 32, 64>;
-using T64 = Tile<64, 256, 64, 64>;
 using TBig = Tile<128, 128, 64, 64>;
 
 // rows for which 16-bit K-contiguous operands take gemm_big_kernel
 inline bool big_rows(int64_t M) { return M > 16; }
 
-inline void tile_dims(TileId t, int& bm, int& bn) {
-  switch (t) {
-    case TileId::M16: bm = T16::BM; bn = T16::BN; break;
-    case TileId::M32: bm = T32::BM; bn = T32::BN; break;
-    case TileId::M64: bm = T64::BM; bn = T64::BN; break;
-    default: bm = TBig::BM; bn = TBig::BN; break;
-  }
+// fp32 kernel (gemm_f32_impl.h), instantiated in gemm_f32.hip only
+template <int BITS> int launch_f32(const GemmArgs& a, bool b_ncontig, int splits, hipStream_t st);
+
+// fp32 operands the DMA kernel takes: 16-byte aligned, and strides whose tile
+// rows span less than 2^31 bytes of its 32-bit lane offsets. At M <= 16 a
+// K-contiguous B streams as fast from the skinny tile (27 against 28 us at
+// N = 6144, K = 4096), an N-contiguous one does not (46 against 26 us).
+inline bool f32_dma_ok(const GemmArgs& a, bool b_ncontig, bool vec) {
+  return vec && (b_ncontig || a.M > 16) && a.lda <= (int64_t(1) << 21) && a.ldb <= (int64_t(1) << 21);
 }
 
-// Instantiation matrix: the vectorised K-contiguous-B path (weights as
-// stored by the vLLM glue) gets every tile; the N-contiguous-B path gets a
-// skinny and a square tile; misaligned / ragged operands (scalar loads) use
+// Rows per tile (32 or 64, by 128 columns) and split count of the fp32 DMA
+// kernel beyond M = 32. The kernel is matrix-core bound, so what decides is
+// how evenly tiles x splits fall on the 256 CUs, against the partials' way
+// through memory. The estimate, in us: every CU runs r = ceil(workgroups /
+// 256) workgroups, each 0.9 us per K-tile and 32 x 128 outputs, over the
+// share of the matrix cores that r workgroups in flight keep busy; splits add
+// a reduce launch and 1.6e-6 us per partial. Fitted to 450 timings (M 33 to
+// 1000, N 1601 to 14336, K 4096 to 14336, 1 to 16 splits): within 2 % of the
+// fastest choice on average, 17 % at worst.
+struct F32Plan {
+  int bm, splits;
+};
+inline F32Plan f32_plan(int64_t M, int64_t N, int ktiles, int requested) {
+  constexpr double busy[4] = {0.6, 0.85, 0.95, 1.0};
+  F32Plan best{64, 1};
+  double best_us = 0.0;
+  for (int bm = 32; bm <= 64; bm += 32) {
+    const int64_t tiles = cdiv(M, bm) * cdiv(N, 128);
+    const int lo = requested >= 1 ? requested : 1;
+    const int hi = requested >= 1 ? requested : (ktiles < 16 ? ktiles : 16);
+    for (int s = lo; s <= hi; ++s) {
+      const int64_t r = cdiv(tiles * s, 256);
+      double us = double(r) * (double(cdiv(ktiles, s)) * (bm / 32) * 0.9 / busy[(r < 4 ? r : 4) - 1] + 0.5);
+      if (s > 1) us += 3.0 + 1.6e-6 * double(s) * double(M) * double(N);
+      if (best_us == 0.0 || us < best_us) {
+        best_us = us;
+        best = {bm, s};
+      }
+    }
+  }
+  return best;
+}
+
+// Instantiation matrix of the register-staged tiles: the vectorised paths get
+// a skinny and a square tile; misaligned / ragged operands (scalar loads) use
 // the square tile only. Tile choice never changes bits.
 template <int DT, int BITS>
 int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipStream_t st) {
-  const TileId t = pick_tile(a.M);
   // gemm_big_kernel's 32-bit lane offsets span up to 256 rows of A or B.
   // From M = 17 its tiles (rows past M clamped, never stored) beat the skinny
   // tiles: 183 / 187 us against 215 / 244 at M = 32 / 64 on the lm_head with
@@ -1318,16 +1343,17 @@ int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipSt
     if (big_ok && ts64_rows(a.M, BITS)) return launch_big<DT, BITS, TS64>(a, splits, st);
     if (big_ok) return launch_big<DT, BITS, TB2>(a, splits, st);
   }
+  if constexpr (DT == FXPR_DTYPE_F32) {
+    if (f32_dma_ok(a, b_ncontig, vec)) return launch_f32<BITS>(a, b_ncontig, splits, st);
+  }
   if (vec && !b_ncontig) {
-    switch (t) {
-      case TileId::M16: return launch_cfg<DT, BITS, T16, false, true>(a, splits, st);
-      case TileId::M32: return launch_cfg<DT, BITS, T32, false, true>(a, splits, st);
-      case TileId::M64: return launch_cfg<DT, BITS, T64, false, true>(a, splits, st);
-      default: return launch_cfg<DT, BITS, TBig, false, true>(a, splits, st);
-    }
+    if (a.M <= 16) return launch_cfg<DT, BITS, T16, false, true>(a, splits, st);
+    return launch_cfg<DT, BITS, TBig, false, true>(a, splits, st);
   }
   if (vec) {
-    if (t == TileId::M16) return launch_cfg<DT, BITS, T16, true, true>(a, splits, st);
+    if constexpr (DT != FXPR_DTYPE_F32) {
+      if (a.M <= 16) return launch_cfg<DT, BITS, T16, true, true>(a, splits, st);
+    }
     return launch_cfg<DT, BITS, TBig, true, true>(a, splits, st);
   }
   if (b_ncontig) return launch_cfg<DT, BITS, TBig, true, false>(a, splits, st);
@@ -1362,12 +1388,15 @@ inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int
   } else {
     // 16-bit decode shapes take the streaming kernel, which needs no split
     if (io_dtype != FXPR_DTYPE_F32 && stream_shape(M, N)) return 1;
-    int bm, bn;
-    tile_dims(pick_tile(M), bm, bn);
-    if (big_rows(M) && io_dtype != FXPR_DTYPE_F32) {
-      const bool s64 = ts64_rows(M, int_bits);
-      bm = s64 ? TS64::BM : TB2::BM;  // TB64 has TB2's tile
-      bn = s64 ? TS64::BN : TB2::BN;
+    // fp32 beyond M = 32 (K a multiple of a chunk: other rows cannot be
+    // 16-byte aligned and take the register-staged tiles)
+    if (io_dtype == FXPR_DTYPE_F32 && M > 32 && K % 4 == 0) return f32_plan(M, N, ktiles, 0).splits;
+    int bm = 128, bn = 128;  // TB2, TB64, TBig
+    if (io_dtype != FXPR_DTYPE_F32 && ts64_rows(M, int_bits)) {
+      bm = TS64::BM;
+      bn = TS64::BN;
+    } else if (M <= 16 || (io_dtype == FXPR_DTYPE_F32 && M <= 64)) {
+      bn = 256;  // one row of tiles: the skinny tile (fp32: and twice as many 32 x 128 ones)
     }
     const int64_t tiles = cdiv(M, bm) * cdiv(N, bn);
     if (tiles >= 256) return 1;
