@@ -613,3 +613,38 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(b_layout):
     whole = _run(a, b, b_layout=b_layout)
     for m in (1, 16, 17, 40, 200):
         assert torch.equal(_run(a[:m], b, b_layout=b_layout), whole[:m])
+
+
+# --- row-major (N-contiguous) 16-bit B on the large-M kernel's tiles ---------
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 16), (64, 32), (16, 8)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 128), (5, 4096, 256), (16, 264, 136), (17, 120, 384), (64, 256, 72),
+                                   (65, 128, 128), (130, 392, 520), (257, 136, 256)])
+def test_gemm_row_major_b_tile_edges(dtype, bits, frac, M, N, K):
+    # one past and one short of a tile in M, N and K (whole K-tiles, a peeled
+    # partial one, only a partial one), unsplit, split and the automatic choice
+    a, b = _int_mats(M, K, N, seed=M + N + K, dtype=dtype)
+    bias = (torch.arange(N, dtype=torch.float32) / 16).to(dtype)
+    want = _oracle(a, b, bias, bits, frac)
+    for split_k in (0, 1, 2):
+        got = _run(a, b, bias, bits, frac, split_k=split_k, b_layout="kn")
+        assert torch.equal(got, want), mismatch_report(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 16), (16, 8)])
+@pytest.mark.parametrize("M", [9, 40, 300])
+def test_gemm_row_major_b_equals_k_contiguous(dtype, bits, frac, M):
+    # both layouts run the same chains: the same bits, on ordinary values and
+    # where a K-tile leaves the rounding constant's range (recomputed exactly,
+    # or with 64-bit sums by the second pass), with inf and NaN among them
+    g = torch.Generator("cpu").manual_seed(M)
+    a = torch.randn(M, 648, generator=g).to(dtype)
+    b = (torch.randn(648, 400, generator=g) * 0.05).to(dtype)
+    assert torch.equal(_run(a, b, bits=bits, frac=frac, b_layout="kn"), _run(a, b, bits=bits, frac=frac, b_layout="nk"))
+    a[M // 2, 5] = 3000.0
+    a[0, 200], b[300, 17], b[640, 399] = float("inf"), float("nan"), 900.0
+    kn = _run(a, b, bits=bits, frac=frac, b_layout="kn")
+    assert nan_aware_equal(kn, _run(a, b, bits=bits, frac=frac, b_layout="nk"))

@@ -458,8 +458,8 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs args, 
 }
 
 // ---------------------------------------------------------------------------
-// Large-M kernel for 16-bit inputs with K-contiguous A and B (the lm_head /
-// linear layout). Same per-output MFMA chain as gemm_fxp_kernel (16x16x32,
+// Large-M kernel for 16-bit inputs with a K-contiguous A (the lm_head / linear
+// layout, B K-contiguous; BNC: a row-major B). Same per-output MFMA chain as gemm_fxp_kernel (16x16x32,
 // increasing k, zero C at each 128-wide K-tile), so results are bitwise
 // identical to every other configuration; only the schedule differs.
 //
@@ -540,7 +540,33 @@ __device__ __forceinline__ void lgkm_wait_for(u32x4& a, u32x4& b, u32x4& c, u32x
 // stores nothing but a NaN at C[m0][n0] for the 64-bit kernel's REDO pass,
 // which computes exactly those tiles (a NaN there from a NaN bias costs a
 // redundant, bit-identical recompute).
-template <int DT, int BITS, class BT, bool SPLIT, bool WIDEN = false, bool REDO = false>
+//
+// BNC: B is N-contiguous ([K][N] rows). Its stage is kept as it lies, 64 k
+// rows of BN columns (chunk c of row r at slot c ^ bnc_swz(r)), and a fragment
+// (16 columns x 32 k) is two transposing reads (ds_read_b64_tr_b16: 16 lanes
+// take 4 k rows x 16 columns and get one column each) instead of one
+// ds_read_b128. bnc_swz spreads the 16 k rows of a read over all banks.
+// It runs within 1-8 % of the K-contiguous form (twelve reads per half stage
+// instead of eight); the register-staged tiles that served this layout wrote
+// B into LDS element by element, one wave per SIMD: f16 M = 1000, N = 6144,
+// K = 4096: 392 -> 70 us; M = 4096: 237 us (868 TFLOP/s); M = 1: 471 -> 21 us.
+__device__ __forceinline__ int bnc_swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+// the two 4-k halves of an N-contiguous B fragment
+struct TrFrag {
+  uint64_t lo, hi;
+};
+template <int N>
+__device__ __forceinline__ void lgkm_wait_for(u32x4& a, TrFrag& b, TrFrag& c, TrFrag& d, TrFrag& e) {
+  asm volatile("s_waitcnt lgkmcnt(%9)"
+               : "+v"(a), "+v"(b.lo), "+v"(b.hi), "+v"(c.lo), "+v"(c.hi), "+v"(d.lo), "+v"(d.hi), "+v"(e.lo), "+v"(e.hi)
+               : "n"(N)
+               : "memory");
+}
+template <int OFF> __device__ __forceinline__ void read_tr16(unsigned addr, uint64_t& x) {
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=&v"(x) : "v"(addr), "n"(OFF) : "memory");
+}
+
+template <int DT, int BITS, class BT, bool SPLIT, bool WIDEN = false, bool REDO = false, bool BNC = false>
 __global__ __launch_bounds__(BT::THREADS, BT::WPE) void gemm_big_kernel(GemmArgs args) {
   using M_ = Mma<DT>;
   using T = typename M_::T;
@@ -557,6 +583,15 @@ __global__ __launch_bounds__(BT::THREADS, BT::WPE) void gemm_big_kernel(GemmArgs
   constexpr int NIB = BN / 8 / NW;        // B DMA instructions per wave per stage
   constexpr int NDMA = NIA + NIB;         // vector memory instructions per wave per stage
   static_assert(NIA * 8 * NW == BM && NIB * 8 * NW == BN, "tile / wave mismatch");
+  // BNC: bytes and 16-byte chunks per k row of a B stage
+  constexpr int ROWB = BN * 2, CPRB = BN / CH;
+  static_assert(!BNC || (CPRB >= 16 && CPRB <= 64 && 64 % CPRB == 0), "whole k rows per DMA instruction");
+  // BNC: a wave's instructions lie NW * 64 / CPRB rows apart; after 16 rows the
+  // swizzle repeats, so VP lane offsets serve them all, 16 rows further on in
+  // the scalar offset
+  constexpr int VP = BNC ? 16 * CPRB / (64 * NW) : NIB;
+  static_assert(VP >= 1 && NIB % VP == 0, "swizzle period");
+  using BFrag = std::conditional_t<BNC, TrFrag, u32x4>;
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(smem_raw));
@@ -613,13 +648,23 @@ redo_next:
   // a scalar.
   const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
       uniform_ptr(A + m0 * args.lda + kb0), short(0), -1, kBufferDword3);
-  const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(
-      uniform_ptr(B + n0 * args.ldb + kb0), short(0), -1, kBufferDword3);
-  uint32_t voff[NDMA];
+  // (BNC: instruction i covers 1 KB of k rows, lane l chunk l % CPRB of row
+  // l / CPRB of them; columns past N clamped by whole chunks, and the stage
+  // offset, which may pass 2^31 bytes, in the 64-bit base)
+  const T* const b_base = BNC ? B + kb0 * args.ldb + n0 : B + n0 * args.ldb + kb0;
+  const __amdgpu_buffer_rsrc_t brsrc =
+      __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(b_base), short(0), -1, kBufferDword3);
+  uint32_t voff[NIA + VP];
 #pragma unroll
-  for (int q = 0; q < NDMA; ++q) {
+  for (int q = 0; q < NIA + VP; ++q) {
     const bool isa = q < NIA;
     const int i = wave + NW * (isa ? q : q - NIA);
+    if (BNC && !isa) {
+      const int r = (64 / CPRB) * i + lane / CPRB;
+      const int c = (lane % CPRB) ^ bnc_swz(r);
+      voff[q] = uint32_t((r * args.ldb + (min<int64_t>(n0 + c * CH, args.N - CH) - n0)) * int64_t(sizeof(T)));
+      continue;
+    }
     const int r = 8 * i + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     const int64_t row = isa ? min<int64_t>(m0 + r, args.M - 1) - m0 : min<int64_t>(n0 + r, args.N - 1) - n0;
@@ -629,6 +674,14 @@ redo_next:
   auto dma = [&](bool isb, int s, int q) {
     const int soff = s * (BKS * int(sizeof(T)));
     const unsigned slot = isb ? B_RING + (q % NSB) * B_SLOT : (q % NSA) * A_SLOT;
+    if (BNC && isb) {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          uniform_ptr(b_base + int64_t(s) * BKS * args.ldb), short(0), -1, kBufferDword3);
+#pragma unroll
+      for (int q = 0; q < NIB; ++q)
+        buffer_to_lds(r, lds0 + slot + (wave + NW * q) * 1024, voff[NIA + q % VP], q / VP * 16 * int(args.ldb) * int(sizeof(T)));
+      return;
+    }
 #pragma unroll
     for (int q = isb ? NIA : 0; q < (isb ? NDMA : NIA); ++q) {
       const int i = wave + NW * (isb ? q - NIA : q);
@@ -658,31 +711,58 @@ redo_next:
     const unsigned slot = isb ? B_RING + (s % NSB) * B_SLOT : (s % NSA) * A_SLOT;
     return lds0 + slot + ((((h << 2) + kg) ^ sw) << 4) + (isb ? brow : arow);
   };
+  // BNC fragment of column block j: lane (j16 = lane % 16) of k group kg takes
+  // row 8 kg + j16 / 4 (+ 4 for the second half, whose swizzle differs in bit
+  // 0 only) and the 8-byte piece j16 % 4 of the block's 32 bytes; its h half
+  // lies 32 rows further on (same swizzle).
+  const int trow = 8 * kg + ((lane & 15) >> 2);
+  const unsigned tr_row = trow * ROWB + (lane & 1) * 8;
+  const unsigned tr_chunk = unsigned((wn * (BT::WN / CH) + ((lane & 3) >> 1)) ^ bnc_swz(trow)) << 4;
+  auto tr_addr = [&](int s, int j, int half) -> unsigned {
+    return lds0 + B_RING + (s % NSB) * B_SLOT + tr_row + half * 4 * ROWB + (tr_chunk ^ unsigned((j << 5) | (half << 4)));
+  };
   auto read_frag = [&](unsigned addr, u32x4& x, auto off_tag) {
     constexpr int OFF = decltype(off_tag)::value;
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(x) : "v"(addr), "n"(OFF) : "memory");
   };
   // Issue order A0, B0..B3, A1..A3: the stage loop starts on block row 0 as
   // soon as the first five have landed.
-  auto read_frags = [&](int st, int h, u32x4 (&fa)[MB], u32x4 (&fb)[NB]) {
-    const unsigned aa = frag_addr(st, h, false), bb = frag_addr(st, h, true);
+  auto read_frags = [&](int st, auto h_tag, u32x4 (&fa)[MB], BFrag (&fb)[NB]) __attribute__((always_inline)) {
+    constexpr int h = decltype(h_tag)::value;
+    const unsigned aa = frag_addr(st, h, false);
     read_frag(aa, fa[0], std::integral_constant<int, 0>{});
-    read_frag(bb, fb[0], std::integral_constant<int, 0>{});
-    read_frag(bb, fb[1], std::integral_constant<int, 2048>{});
-    read_frag(bb, fb[2], std::integral_constant<int, 4096>{});
-    read_frag(bb, fb[3], std::integral_constant<int, 6144>{});
+    if constexpr (BNC) {
+      static_for<NB>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        read_tr16<h * 32 * ROWB>(tr_addr(st, j, 0), fb[j].lo);
+        read_tr16<h * 32 * ROWB>(tr_addr(st, j, 1), fb[j].hi);
+      });
+    } else {
+      const unsigned bb = frag_addr(st, h, true);
+      read_frag(bb, fb[0], std::integral_constant<int, 0>{});
+      read_frag(bb, fb[1], std::integral_constant<int, 2048>{});
+      read_frag(bb, fb[2], std::integral_constant<int, 4096>{});
+      read_frag(bb, fb[3], std::integral_constant<int, 6144>{});
+    }
     read_frag(aa, fa[1], std::integral_constant<int, 2048>{});
     read_frag(aa, fa[2], std::integral_constant<int, 4096>{});
     read_frag(aa, fa[3], std::integral_constant<int, 6144>{});
   };
-  auto lds_wait = [&](u32x4 (&fa)[MB], u32x4 (&fb)[NB]) {
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]),
-                   "+v"(fb[3])
-                 :
-                 : "memory");
+  auto lds_wait = [&](u32x4 (&fa)[MB], BFrag (&fb)[NB]) __attribute__((always_inline)) {
+    if constexpr (BNC)
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0].lo), "+v"(fb[0].hi),
+                     "+v"(fb[1].lo), "+v"(fb[1].hi), "+v"(fb[2].lo), "+v"(fb[2].hi), "+v"(fb[3].lo), "+v"(fb[3].hi)
+                   :
+                   : "memory");
+    else
+      asm volatile("s_waitcnt lgkmcnt(0)"
+                   : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]),
+                     "+v"(fb[3])
+                   :
+                   : "memory");
   };
-  auto mma = [&](int i, int j, const u32x4& a, const u32x4& b, bool zero_c) {
+  auto mma = [&](int i, int j, const u32x4& a, const BFrag& b, bool zero_c) {
     P[i][j] = M_::mma(__builtin_bit_cast(uint4, a), __builtin_bit_cast(uint4, b), zero_c ? zero4 : P[i][j]);
   };
   auto quantize_block = [&](int i, int j) {
@@ -750,16 +830,16 @@ redo_next:
   };
   // Plain (unpipelined) stage, used for the peeled tail tile.
   auto compute = [&](int st, bool first) {
-    u32x4 fa[MB], fb[NB];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      read_frags(st, h, fa, fb);
+    u32x4 fa[MB];
+    BFrag fb[NB];
+    static_for<2>([&](auto hc) {
+      read_frags(st, hc, fa, fb);
       lds_wait(fa, fb);
 #pragma unroll
       for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) mma(i, j, fa[i], fb[j], first && h == 0);
-    }
+        for (int j = 0; j < NB; ++j) mma(i, j, fa[i], fb[j], first && decltype(hc)::value == 0);
+    });
   };
 
   // P holds the fp32 partial of the K-tile in progress; it is quantised into
@@ -778,6 +858,14 @@ redo_next:
     const int64_t kt0 = int64_t(kt) * 128;
     for (int e = tid; e < 2 * (BM + BN) * 8; e += BT::THREADS) {
       const int st = e / ((BM + BN) * 8), rem = e % ((BM + BN) * 8);
+      if (BNC && rem >= BM * 8) {
+        const int r = (rem - BM * 8) / CPRB, c = (rem - BM * 8) % CPRB;
+        const int64_t k = kt0 + st * BKS + r, col = n0 + c * CH;
+        const int valid = k < args.K && col < args.N ? CH : 0;  // N is a whole number of chunks
+        const uint4 v = load_chunk<false>(B + (valid ? k * args.ldb + col : 0), valid);
+        *reinterpret_cast<uint4*>(smem_raw + B_RING + st * B_SLOT + r * ROWB + ((c ^ bnc_swz(r)) << 4)) = v;
+        continue;
+      }
       const int r = rem / 8, c = rem % 8;
       const int64_t k = kt0 + st * BKS + c * CH;
       const bool isa = r < BM;
@@ -809,7 +897,8 @@ redo_next:
   // stage's h = 0 fragment reads, which complete while the MFMAs drain.
   const int nst = 2 * nfull;
   if (nst > 0) {
-    u32x4 fa0[MB], fb0[NB], fa1[MB], fb1[NB];
+    u32x4 fa0[MB], fa1[MB];
+    BFrag fb0[NB], fb1[NB];
     constexpr bool B_DEEP = NSB > NSA;
     constexpr int NSS = B_DEEP ? NSA : NSB, NSD = B_DEEP ? NSB : NSA;  // shallow, deep depth
     constexpr int NID = B_DEEP ? NIB : NIA;                             // deep ring's DMAs per stage
@@ -826,7 +915,7 @@ redo_next:
     for (int j = 1 - NSD; j < 0; ++j) dma_group(j);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAITN) : "memory");
     __builtin_amdgcn_s_barrier();
-    read_frags(0, 0, fa0, fb0);
+    read_frags(0, std::integral_constant<int, 0>{}, fa0, fb0);
     // Landed before the loop: the compiler may move the loop's fragment
     // registers into place here, and an inline-asm read's output looks ready
     // to it at issue.
@@ -837,7 +926,8 @@ redo_next:
     auto stage = [&](int s, auto tile_start_tag) {
       constexpr bool tile_start = decltype(tile_start_tag)::value;
       dma_group(s);
-      const unsigned aa1 = frag_addr(s, 1, false), bb1 = frag_addr(s, 1, true);
+      const unsigned aa1 = frag_addr(s, 1, false);
+      [[maybe_unused]] const unsigned bb1 = BNC ? 0 : frag_addr(s, 1, true);
       __builtin_amdgcn_sched_barrier(0);
       // Block row i: its quantisation (at a K-tile start; registers only, so
       // it runs while the row's fragments land), a wait for them (LDS
@@ -859,7 +949,8 @@ redo_next:
         } else if constexpr (i == 0) {
           lgkm_wait_for<3>(fa0[0], fb0[0], fb0[1], fb0[2], fb0[3]);
         } else {
-          lgkm_wait_for<3 + i>(fa0[i]);
+          // A(i + 1 .. 3), and the two (BNC: three) h = 1 reads of each row so far
+          lgkm_wait_for<3 + (BNC ? 2 : 1) * i>(fa0[i]);
         }
       };
       // compile-time block index: every read and wait at a fixed place (a
@@ -869,7 +960,19 @@ redo_next:
         constexpr int b = decltype(bc)::value, i = b / NB, j = b % NB;
         if constexpr (j == 0) row_prologue(std::integral_constant<int, i>{});
         mma(i, j, fa0[i], fb0[j], tile_start);
-        if constexpr (b % 2 == 0) {
+        if constexpr (BNC) {
+          // twelve h = 1 reads, three per row: A 0..3, then the halves of B 0..3
+          if constexpr (j < 3) {
+            constexpr int g = 3 * i + j;
+            if constexpr (g < MB) {
+              read_frag(aa1, fa1[g], std::integral_constant<int, 2048 * g>{});
+            } else {
+              constexpr int fj = (g - MB) / 2;
+              if constexpr ((g - MB) % 2 == 0) read_tr16<32 * ROWB>(tr_addr(s, fj, 0), fb1[fj].lo);
+              else read_tr16<32 * ROWB>(tr_addr(s, fj, 1), fb1[fj].hi);
+            }
+          }
+        } else if constexpr (b % 2 == 0) {
           constexpr int f = b / 2;  // h = 1 fragment f: A 0..3, then B 0..3
           if constexpr (f < MB)
             read_frag(aa1, fa1[f], std::integral_constant<int, 2048 * f>{});
@@ -896,7 +999,7 @@ redo_next:
       // s_barrier: __syncthreads() would also fence, i.e. wait for every DMA.
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAITN) : "memory");
       __builtin_amdgcn_s_barrier();
-      read_frags(s + 1, 0, fa0, fb0);
+      read_frags(s + 1, std::integral_constant<int, 0>{}, fa0, fb0);
     };
     for (int s = 0; s < nst; s += 2) {
       stage(s, std::true_type{});
@@ -1188,7 +1291,7 @@ int launch_tile(const GemmArgs& a, int splits, hipStream_t st) {
   return launch_status();
 }
 
-template <int DT, int BITS, class BT, bool WIDEN = false, bool REDO = false>
+template <int DT, int BITS, class BT, bool BNC, bool WIDEN = false, bool REDO = false>
 int launch_big(GemmArgs a, int splits, hipStream_t st) {
   a.tiles_m = int(cdiv(a.M, BT::BM));
   a.tiles_n = int(cdiv(a.N, BT::BN));
@@ -1206,12 +1309,12 @@ int launch_big(GemmArgs a, int splits, hipStream_t st) {
     return launch_status();
   };
   if constexpr (REDO) {
-    return go(gemm_big_kernel<DT, BITS, BT, false, false, true>);
+    return go(gemm_big_kernel<DT, BITS, BT, false, false, true, BNC>);
   } else if constexpr (WIDEN) {
-    return go(gemm_big_kernel<DT, BITS, BT, false, true>);
+    return go(gemm_big_kernel<DT, BITS, BT, false, true, false, BNC>);
   } else {
-    if (splits > 1 || a.mode == kPartial) return go(gemm_big_kernel<DT, BITS, BT, true>);
-    return go(gemm_big_kernel<DT, BITS, BT, false>);
+    if (splits > 1 || a.mode == kPartial) return go(gemm_big_kernel<DT, BITS, BT, true, false, false, BNC>);
+    return go(gemm_big_kernel<DT, BITS, BT, false, false, false, BNC>);
   }
 }
 
@@ -1314,34 +1417,36 @@ int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipSt
   // From M = 17 its tiles (rows past M clamped, never stored) beat the skinny
   // tiles: 183 / 187 us against 215 / 244 at M = 32 / 64 on the lm_head with
   // 128 x 128 tiles (64-bit sums: 189 / 192 against 245 / 362), and the
-  // 64 x 256 ones of M <= 64 more; at M <= 16 the skinny tile streams B
-  // faster (153 against 176 us).
-  const bool big_ok = vec && !b_ncontig && big_rows(a.M) && a.lda <= (int64_t(1) << 22) &&
+  // 64 x 256 ones of M <= 64 more; at M <= 16 the skinny tile streams a
+  // K-contiguous B faster (153 against 176 us). An N-contiguous B takes it at
+  // every M (the register-staged tiles transpose it element by element).
+  const bool big_ok = vec && (b_ncontig || big_rows(a.M)) && a.lda <= (int64_t(1) << 22) &&
                       a.ldb <= (int64_t(1) << 22);
   const bool full = a.mode == kFull;
   if constexpr (DT != FXPR_DTYPE_F32) {
     // decode shapes: stream B once, no split-K partials
     if (full && splits <= 1 && stream_ok(a, vec, b_ncontig)) return launch_stream<DT, BITS>(a, st);
-  }
-  if constexpr (DT != FXPR_DTYPE_F32 && BITS == 64) {
-    if (big_ok) {
-      // Unsplit, fewer than 512 K-tiles: 32-bit sums in the two-workgroups-
-      // per-CU schedule (the 64-bit state of the exact kernel leaves it one
-      // wave per SIMD), then the exact kernel on the tiles that pass marked (a
-      // K-tile outside the rounding-constant range). Only for f <= 20 (|P| < 4
-      // per K-tile stays in range; at larger f most tiles would be computed
-      // twice). 1.4-1.8x faster than the exact kernel alone from M = 65 up.
-      if (full && splits <= 1 && a.ktiles < 512 && a.fast_lim >= 4.0f) {
-        const int rc = launch_big<DT, 32, TB2, true>(a, 1, st);
-        if (rc != FXPR_OK) return rc;
-        return launch_big<DT, BITS, TB64, false, true>(a, 1, st);
+    auto big = [&](auto bnc_tag) -> int {
+      constexpr bool BNC = decltype(bnc_tag)::value;
+      if constexpr (BITS == 64) {
+        // Unsplit, fewer than 512 K-tiles: 32-bit sums in the two-workgroups-
+        // per-CU schedule (the 64-bit state of the exact kernel leaves it one
+        // wave per SIMD), then the exact kernel on the tiles that pass marked (a
+        // K-tile outside the rounding-constant range). Only for f <= 20 (|P| < 4
+        // per K-tile stays in range; at larger f most tiles would be computed
+        // twice). 1.4-1.8x faster than the exact kernel alone from M = 65 up.
+        if (full && splits <= 1 && a.ktiles < 512 && a.fast_lim >= 4.0f) {
+          const int rc = launch_big<DT, 32, TB2, BNC, true>(a, 1, st);
+          if (rc != FXPR_OK) return rc;
+          return launch_big<DT, BITS, TB64, BNC, false, true>(a, 1, st);
+        }
+        return launch_big<DT, BITS, TB64, BNC>(a, splits, st);
+      } else {
+        if (ts64_rows(BNC && a.M <= 16 ? 17 : a.M, BITS)) return launch_big<DT, BITS, TS64, BNC>(a, splits, st);
+        return launch_big<DT, BITS, TB2, BNC>(a, splits, st);
       }
-      return launch_big<DT, BITS, TB64>(a, splits, st);
-    }
-  }
-  if constexpr (DT != FXPR_DTYPE_F32 && BITS != 64) {
-    if (big_ok && ts64_rows(a.M, BITS)) return launch_big<DT, BITS, TS64>(a, splits, st);
-    if (big_ok) return launch_big<DT, BITS, TB2>(a, splits, st);
+    };
+    if (big_ok) return b_ncontig ? big(std::true_type{}) : big(std::false_type{});
   }
   if constexpr (DT == FXPR_DTYPE_F32) {
     if (f32_dma_ok(a, b_ncontig, vec)) return launch_f32<BITS>(a, b_ncontig, splits, st);
@@ -1350,12 +1455,7 @@ int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipSt
     if (a.M <= 16) return launch_cfg<DT, BITS, T16, false, true>(a, splits, st);
     return launch_cfg<DT, BITS, TBig, false, true>(a, splits, st);
   }
-  if (vec) {
-    if constexpr (DT != FXPR_DTYPE_F32) {
-      if (a.M <= 16) return launch_cfg<DT, BITS, T16, true, true>(a, splits, st);
-    }
-    return launch_cfg<DT, BITS, TBig, true, true>(a, splits, st);
-  }
+  if (vec) return launch_cfg<DT, BITS, TBig, true, true>(a, splits, st);
   if (b_ncontig) return launch_cfg<DT, BITS, TBig, true, false>(a, splits, st);
   return launch_cfg<DT, BITS, TBig, false, false>(a, splits, st);
 }

@@ -59,6 +59,11 @@ def gemm_fxp_run(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, in
 
     lib = _hip.load()
     code = _hip.DTYPE_CODE[a.dtype]
+    if split_k == 0 and M <= 16 and b.stride(0) != 1 and K > 1:
+        # a row-major B runs on the large-M kernel's tiles at every M: the
+        # split count its policy gives a row of them, not the streaming
+        # kernel's (none)
+        split_k = lib.fxpr_gemm_splits(17, N, K, code, int(int_bits), 0)
     ws_bytes = lib.fxpr_gemm_workspace_bytes(M, N, K, code, int(int_bits), int(split_k))
     ws = torch.empty(ws_bytes, device=a.device, dtype=torch.uint8) if ws_bytes > 0 else None
     _hip.call(
