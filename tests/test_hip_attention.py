@@ -18,6 +18,7 @@ import pytest
 import torch
 
 import fxpr_vllm  # noqa: F401
+from fxpr_vllm._kernels import attention as KA
 from oracle import attention as A
 from tests._util import IO_NAME, close_report, from_np, to_np
 
@@ -596,3 +597,80 @@ def test_page_sizes_decode_and_prefill(ps):
     for s in (0, 3):
         assert torch.equal(attend(q, kv, qsl, sl, bt, max(q_lens), s, scale=scale), one), s
     assert close(one, oracle(q, kv, qsl, sl, bt, scale=scale))
+
+
+# --- long and short requests of one batch split apart from each other ---------
+
+
+def _ragged(reqs, hq, hkv, d, ps, dtype, seed):
+    """Paged inputs for [(new tokens, context after them)], pages shuffled."""
+    g = torch.Generator("cpu").manual_seed(seed)
+    pages = [-(-ctx // ps) for _, ctx in reqs]
+    bt = torch.zeros(len(reqs), max(pages), dtype=torch.int32)
+    perm = torch.randperm(sum(pages), generator=g).to(torch.int32)
+    at = 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = perm[at:at + n]
+        at += n
+    qsl = torch.tensor([0] + [n for n, _ in reqs], dtype=torch.int32).cumsum(0).to(torch.int32)
+    sl = torch.tensor([c for _, c in reqs], dtype=torch.int32)
+    q = torch.randn(int(qsl[-1]), hq, d, generator=g).to(dtype).cuda()
+    kv = torch.randn(sum(pages), 2, ps, hkv, d, generator=g).to(dtype).cuda()
+    return q, kv, qsl.cuda(), sl.cuda(), bt.cuda(), max(n for n, _ in reqs)
+
+
+def _attend(inp, splits, bits=32, frac=16, window=0, softcap=0.0, causal=True):
+    q, kv, qsl, sl, bt, max_q = inp
+    o = torch.full_like(q, 7.0)
+    KA.unified_attention_fxp_run(q, kv, o, qsl, sl, bt, max_q, None, causal, None, bits, frac, softcap, window, splits)
+    return o
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,hq,hkv", [(128, 8, 2), (64, 4, 4), (128, 28, 4)])
+@pytest.mark.parametrize("reqs", [
+    [(1, 700), (130, 2300), (1, 2600), (3, 513), (1, 1), (12, 40)],   # one prompt chunk among decode steps
+    [(600, 2700)],                                                    # one long prompt, cached prefix
+    [(64, 2100), (1, 64), (70, 70), (48, 2049)],                      # rows on both sides of a 64-row tile
+    [(1, 3000)] * 40 + [(90, 90)],                                    # flat grid: short requests mostly
+])
+@pytest.mark.parametrize("opts", [dict(), dict(window=600), dict(softcap=30.0), dict(bits=16, frac=8)])
+def test_mixed_batch_equals_each_request_alone(dtype, d, hq, hkv, reqs, opts):
+    # automatic (prefill workgroups and short requests split apart), unsplit
+    # and explicit splits give the same bits, and the same as each request in
+    # a launch of its own; rows of no request keep their contents
+    inp = _ragged(reqs, hq, hkv, d, 16, dtype, seed=len(reqs) + d)
+    q, kv, qsl, sl, bt, max_q = inp
+    base = _attend(inp, 1, **opts)
+    for splits in (0, 2, 3, 5):
+        assert torch.equal(_attend(inp, splits, **opts), base), splits
+    at = qsl.tolist()
+    for i in range(min(len(reqs), 4)):
+        one = (q[at[i]:at[i + 1]].contiguous(), kv, torch.tensor([0, at[i + 1] - at[i]], dtype=torch.int32, device="cuda"),
+               sl[i:i + 1].contiguous(), bt[i:i + 1].contiguous(), at[i + 1] - at[i])
+        assert torch.equal(_attend(one, 0, **opts), base[at[i]:at[i + 1]]), i
+    pad = torch.cat([q, torch.zeros_like(q[:5])])
+    o = _attend((pad, kv, qsl, sl, bt, max_q), 0, **opts)
+    assert torch.equal(o[:-5], base) and bool((o[-5:] == 7.0).all())
+
+
+def test_mixed_batch_wide_block_table_and_graph():
+    # a block table far wider than the contexts (slots past them stay
+    # untouched), replayed from a graph with the eager bits each time
+    reqs = [(200, 1500), (1, 4000), (1, 17), (2, 2500)]
+    q, kv, qsl, sl, bt, max_q = _ragged(reqs, 8, 2, 128, 16, torch.bfloat16, 5)
+    wide = torch.zeros(len(reqs), 2048, dtype=torch.int32, device="cuda")
+    wide[:, :bt.shape[1]] = bt
+    base = _attend((q, kv, qsl, sl, bt, max_q), 1)
+    inp = (q, kv, qsl, sl, wide, max_q)
+    assert torch.equal(_attend(inp, 0), base)
+    o = torch.zeros_like(q)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        KA.unified_attention_fxp_run(q, kv, o, qsl, sl, wide, max_q, None, True, None, 32, 16, 0.0, 0, 0)
+    for _ in range(3):
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, base)
+        torch.randn(1 << 20, device="cuda").sum()

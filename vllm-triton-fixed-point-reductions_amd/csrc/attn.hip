@@ -32,10 +32,11 @@ struct WsLayout {
   int64_t crange = -1, pmax = -1, den = -1, wv = -1, total = 0;
 };
 
-WsLayout ws_layout(int64_t num_tokens, int num_heads, int head_dim, int int_bits, int splits, int64_t slots) {
+// (ws_rows: the query tokens that hold records, AttnArgs' W)
+WsLayout ws_layout(int64_t ws_rows, int num_heads, int head_dim, int int_bits, bool split, int64_t slots) {
   WsLayout w;
-  if (splits <= 1) return w;
-  const int64_t rows = num_tokens * num_heads;
+  if (!split) return w;
+  const int64_t rows = ws_rows * num_heads;
   w.crange = 0;
   w.total = align256(rows * 8);
   w.pmax = w.total;
@@ -93,10 +94,77 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
   SplitPlan sp = plan_splits(num_requests, num_kv_heads, num_heads / num_kv_heads, max_query_len, max_blocks,
                              page_size, requested);
   if (sp.splits > 1 &&
-      ws_layout(num_tokens, num_heads, head_dim, int_bits, sp.splits, chunk_slots(max_blocks, page_size)).total >
+      ws_layout(num_tokens, num_heads, head_dim, int_bits, true, chunk_slots(max_blocks, page_size)).total >
           kSplitWsMax)
     sp = {1, 0};
   return sp;
+}
+
+// Launches that may hold requests of kPrefillRows rows or more, where the DMA
+// kernels can take them (16- / 32-bit sums; the rest of their conditions is
+// known at the launch, which otherwise runs launch_plan's): the two kinds of
+// requests are split apart from each other.
+//   * Prefill workgroups (64 rows each): about tokens x heads / 64 of them.
+//     Below 512 (two per CU) their keys are split until there are about
+//     kLongWgs; a chunk is the least a split can hold.
+//   * Short requests: one chunk per split, as in launches of their own, when
+//     their contexts can be long (more than 32 tiles).
+// Explicit requests split both that many times. Records need a workspace: per
+// token when the prefill rows are split, else only for the short requests'
+// tokens; above kLongWsMax (explicit: kSplitWsMax) the launch runs unsplit.
+constexpr int64_t kFullWgs = 512, kLongWgs = 2048;
+constexpr int64_t kLongWsMax = int64_t(1) << 29;
+
+struct LongLayout {
+  LongPlan plan;
+  WsLayout ws;
+};
+
+LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int num_kv_heads, int head_dim, int int_bits,
+                     int max_query_len, int max_blocks, int page_size, int requested) {
+  LongLayout l;
+  const int group = num_heads / num_kv_heads;
+  const int64_t max_rows = int64_t(max_query_len > 1 ? max_query_len : 1) * group;
+  if (int_bits == 64 || max_rows < kPrefillRows || (head_dim != 64 && head_dim != 128)) return l;
+  l.plan.use = true;
+  const int64_t slots = chunk_slots(max_blocks, page_size);
+  const int64_t tiles = cdiv(int64_t(max_blocks > 0 ? max_blocks : 1) * page_size, TILE);
+  int64_t ps = 1, ds = 1;
+  if (requested >= 1) {
+    ps = ds = std::min<int64_t>({int64_t(requested), std::max<int64_t>(slots, 1), kMaxGridZ});
+  } else {
+    const int64_t wgs = std::max<int64_t>(cdiv(num_tokens * num_heads, PQROWS), 1);
+    if (wgs < kFullWgs && tiles > 32) ps = std::min<int64_t>(cdiv(kLongWgs, wgs), slots);
+    if (tiles > 32 && int64_t(num_requests) * num_kv_heads <= 8 * 256)
+      ds = std::min<int64_t>(slots, kMaxSplits);
+  }
+  auto layout = [&](int64_t rows) { return ws_layout(rows, num_heads, head_dim, int_bits, true, slots); };
+  const int64_t most = requested >= 1 ? kSplitWsMax : kLongWsMax;
+  if (ps > 1) {
+    l.ws = layout(num_tokens);
+    if (l.ws.total > most) {
+      ps = 1;
+      if (requested >= 1) ds = 1;
+    }
+  }
+  if (ps <= 1) {
+    l.ws = WsLayout{};
+    if (ds > 1) {
+      // a short request holds fewer than kPrefillRows rows
+      const int64_t cap = std::min<int64_t>(max_query_len, std::max<int64_t>((kPrefillRows - 1) / group, 1));
+      l.plan.tok_cap = int(cap);
+      l.ws = layout(int64_t(num_requests) * cap);
+      if (l.ws.total > most) {
+        ds = 1;
+        l.plan.tok_cap = 0;
+        l.ws = WsLayout{};
+      }
+    }
+  }
+  l.plan.pq_splits = int(ps);
+  l.plan.splits = int(ds);
+  l.plan.chunks_per_split = requested >= 1 || ds <= 1 ? 0 : int(cdiv(slots, ds));
+  return l;
 }
 }  // namespace
 
@@ -116,9 +184,12 @@ extern "C" int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_
     return 0;
   const SplitPlan sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
                                    max_query_len, max_blocks_per_seq, page_size, num_kv_splits);
-  return ws_layout(num_tokens, num_heads, head_dim, int_bits, sp.splits,
-                   chunk_slots(max_blocks_per_seq, page_size))
-      .total;
+  const int64_t plain = ws_layout(num_tokens, num_heads, head_dim, int_bits, sp.splits > 1,
+                                  chunk_slots(max_blocks_per_seq, page_size))
+                            .total;
+  return std::max(plain, long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
+                                   max_blocks_per_seq, page_size, num_kv_splits)
+                             .ws.total);
 }
 
 extern "C" int fxpr_unified_attention(
@@ -156,8 +227,11 @@ extern "C" int fxpr_unified_attention(
     if (sv < 0 || sv > int64_t(0xffffffff)) return FXPR_E_ARG;
   const int64_t slots = chunk_slots(max_blocks_per_seq, page_size);
   if (slots > 0x7fffffff) return FXPR_E_SHAPE;
-  const WsLayout wl = ws_layout(num_tokens, num_heads, head_dim, int_bits, num_splits, slots);
-  if (wl.total > 0 && (!workspace || workspace_bytes < wl.total)) return FXPR_E_WORKSPACE;
+  const WsLayout wl = ws_layout(num_tokens, num_heads, head_dim, int_bits, num_splits > 1, slots);
+  LongLayout ll = long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
+                            max_blocks_per_seq, page_size, num_kv_splits);
+  const int64_t need = std::max(wl.total, ll.ws.total);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return FXPR_E_WORKSPACE;
 
   AttnArgs a{};
   a.q = q;
@@ -173,6 +247,12 @@ extern "C" int fxpr_unified_attention(
   if (wl.pmax >= 0) a.pmax = reinterpret_cast<float*>(base + wl.pmax);
   if (wl.den >= 0) a.den_ws = base + wl.den;
   if (wl.wv >= 0) a.wv_ws = base + wl.wv;
+  if (ll.ws.crange >= 0) {
+    ll.plan.crange = reinterpret_cast<int*>(base + ll.ws.crange);
+    ll.plan.pmax = reinterpret_cast<float*>(base + ll.ws.pmax);
+    ll.plan.den_ws = base + ll.ws.den;
+    ll.plan.wv_ws = base + ll.ws.wv;
+  }
   a.chunk_slots = int(slots);
   a.sq_t = stride_q_token;
   a.sq_h = stride_q_head;
@@ -207,9 +287,9 @@ extern "C" int fxpr_unified_attention(
   const int max_qtiles = int(cdiv(int64_t(max_query_len > 1 ? max_query_len : 1) * a.group, QROWS));
   hipStream_t st = as_stream(stream);
   switch (io_dtype) {
-    case FXPR_DTYPE_BF16: return run_attn_bf16(a, int_bits, num_requests, max_qtiles, num_tokens, st);
-    case FXPR_DTYPE_F16: return run_attn_f16(a, int_bits, num_requests, max_qtiles, num_tokens, st);
-    default: return run_attn_f32(a, int_bits, num_requests, max_qtiles, num_tokens, st);
+    case FXPR_DTYPE_BF16: return run_attn_bf16(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
+    case FXPR_DTYPE_F16: return run_attn_f16(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
+    default: return run_attn_f32(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
   }
 }
 
@@ -276,9 +356,19 @@ extern "C" int fxpr_unified_attention_noalloc(
     int64_t stride_v_head, int64_t stride_o_token, int64_t stride_o_head, int64_t stride_bt_row,
     int is_causal, float softmax_scale_log2, float softcap_log2, int window_size, int int_bits,
     int frac_bits, int num_kv_splits, void* stream) {
-  const int64_t need = fxpr_attention_workspace_bytes(num_requests, num_tokens, num_heads, num_kv_heads,
-                                                      head_dim, int_bits, num_kv_splits, max_query_len,
-                                                      max_blocks_per_seq, page_size);
+  auto ws_need = [&](int splits) {
+    return fxpr_attention_workspace_bytes(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
+                                          splits, max_query_len, max_blocks_per_seq, page_size);
+  };
+  int64_t need = ws_need(num_kv_splits);
+  if (need > kStaticScratchBytes && num_kv_splits == 0) {
+    // the records of an automatic split of long requests may not fit where
+    // the batch's plain split count does (often none): run that (same bits)
+    num_kv_splits = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
+                                max_blocks_per_seq, page_size, 0)
+                        .splits;
+    need = ws_need(num_kv_splits);
+  }
   if (need > kStaticScratchBytes) return FXPR_E_WORKSPACE;
   void* ws = nullptr;
   if (need > 0) {

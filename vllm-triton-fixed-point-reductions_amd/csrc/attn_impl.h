@@ -59,22 +59,41 @@ struct AttnArgs {
   const int32_t* seq_lens;
   const int32_t* bt;
   const float* alibi;  // per q head, already multiplied by log2(e); or null
-  float* pmax;         // [T, Hq, chunk_slots] per-chunk row maxima         (split launches)
-  void* den_ws;        // [T, Hq, chunk_slots] denominators, int32 / int64  (split launches)
-  void* wv_ws;         // [T, Hq, chunk_slots, D] weighted V, int32 / int64 (split launches)
-  int* crange;         // [T, Hq, 2] chunk range [first, end) of the row    (split launches)
+  // split launches: records of W workspace rows (see ws_row)
+  float* pmax;         // [W, Hq, chunk_slots] per-chunk row maxima
+  void* den_ws;        // [W, Hq, chunk_slots] denominators, int32 / int64
+  void* wv_ws;         // [W, Hq, chunk_slots, D] weighted V, int32 / int64
+  int* crange;         // [W, Hq, 2] chunk range [first, end) of the row
   int64_t sq_t, sq_h, sk_b, sk_s, sk_h, sv_b, sv_s, sv_h, so_t, so_h, sbt;
   int num_heads, num_kv_heads, group, head_dim, page_size, num_splits, window, causal;
   int max_blocks;       // block-table row length
   int chunks_per_split;  // > 0: fixed chunks per split (work-balanced); 0: even division
   int chunk_slots;       // chunks per row in the split workspace
-  int pq_rows;           // > 0: requests with at least this many rows go to attn_prefill_kernel
+  int pq_rows;           // > 0: requests with at least this many rows go to the prefill kernels
+  int pq_splits;         // key splits of the prefill workgroups (their chunks dealt evenly)
+  int pq_blocks;         // > 0: 64-row blocks of a flat prefill grid (see flat_block)
+  int tok_cap;           // > 0: workspace rows for requests of at most this many tokens only
   int num_requests;
   int64_t num_blocks;   // physical blocks in the cache
   int64_t num_tokens;   // rows of q / o
   int64_t lmax;         // key capacity of a block-table row (max_blocks * page_size)
   int ps_shift;         // log2(page_size) if a power of two, else -1
   float scale_log2, softcap_log2, fxp_scale, fxp_inv;
+};
+
+// Host plan of a launch that holds requests of kPrefillRows rows or more, for
+// shapes the DMA kernels take: key splits of the prefill workgroups and of the
+// short requests' 16-row ones, and the workspace records of the split rows.
+struct LongPlan {
+  bool use = false;
+  int pq_splits = 1;       // prefill workgroups
+  int splits = 1;          // short requests
+  int chunks_per_split = 0;
+  int tok_cap = 0;         // AttnArgs::tok_cap
+  float* pmax = nullptr;
+  void* den_ws = nullptr;
+  void* wv_ws = nullptr;
+  int* crange = nullptr;
 };
 
 template <int DT> struct Traits;
@@ -146,6 +165,13 @@ __device__ __forceinline__ RowInfo row_info(const AttnArgs& a, int g, int q_star
   ri.kend = a.causal ? min(seq_len, ri.qpos + 1) : seq_len;
   ri.kstart = a.window > 0 ? max(0, ri.qpos - a.window + 1) : 0;
   return ri;
+}
+
+// Workspace row of a query token: the token itself, or (tok_cap) a slot among
+// tok_cap per request, where only short requests are split and the long ones'
+// many tokens need no records.
+__device__ __forceinline__ int64_t ws_row(const AttnArgs& a, int r, int q_start, int64_t token) {
+  return a.tok_cap > 0 ? int64_t(r) * a.tok_cap + (token - q_start) : token;
 }
 
 // Per-row statistics of key chunks are folded in fixed point: an accumulator
@@ -1162,7 +1188,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
         for (int e = 0; e < 4; ++e) {
           const RowInfo ri = row_info(a, g, q_start, q_len, ctx, seq_len, row0 + 4 * kg + e);
           if (!ri.valid) continue;
-          const int64_t slot = (ri.token * a.num_heads + ri.head) * a.chunk_slots + c;
+          const int64_t slot = (ws_row(a, r, q_start, ri.token) * a.num_heads + ri.head) * a.chunk_slots + c;
           if ((lane & 15) == 0 && wave == 0) {
             a.pmax[slot] = mc[e];
             static_cast<AccT*>(a.den_ws)[slot] = dc[e];
@@ -1204,7 +1230,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
   if (SPLIT && split == 0 && tid < QROWS) {
     const RowInfo ri = row_info(a, g, q_start, q_len, ctx, seq_len, row0 + tid);
     if (ri.valid) {
-      int* cr = a.crange + 2 * (ri.token * a.num_heads + ri.head);
+      int* cr = a.crange + 2 * (ws_row(a, r, q_start, ri.token) * a.num_heads + ri.head);
       cr[0] = c_lo;
       cr[1] = c_lo + nch;
     }
@@ -1642,7 +1668,36 @@ template <int OFF> __device__ __forceinline__ void lds_read_b128_off(unsigned ad
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(addr), "n"(OFF) : "memory");
 }
 
-template <int DT, int BITS, int DMAX>
+//
+// SPLIT: the chunks of a row tile are dealt evenly to pq_splits workgroups
+// (blockIdx.z), for batches whose row tiles are too few to give every CU two
+// workgroups: one alone waits on each step's DMAs and barriers (512 new tokens
+// after 3500 cached, 32 heads: 256 workgroups took 310 us at one per CU). The
+// first split folds its chunks as the unsplit kernel does and leaves the
+// folded state as one record (the fold is sequential from chunk c_lo, and
+// folding an empty state with a record gives the record, so the combine
+// continues from it with the same bits); the others leave a record per chunk.
+//
+// flat_block: with a flat grid (pq_blocks), block b -> request and row tile.
+// Request r owns blocks [start(r), start(r + 1)), start(r) = floor(qsl[r] *
+// group / 64) + r: at least one per row tile, so the grid follows the batch's
+// tokens and not requests x the longest one (which starts mostly workgroups
+// that exit at once when decode steps share the batch). Wave-uniform; -1 if b
+// belongs to no request.
+__device__ __forceinline__ int flat_block(const AttnArgs& a, int b, int& tile) {
+  const int lane = threadIdx.x & 63;
+  int owned = 0;  // requests whose first block is at or before b
+  for (int r0 = 0; r0 < a.num_requests; r0 += 64) {
+    const int r = min(r0 + lane, a.num_requests - 1);
+    const int64_t start = ((int64_t(a.qsl[r]) * a.group) >> 6) + r;
+    owned += __builtin_popcountll(__builtin_amdgcn_ballot_w64(r0 + lane < a.num_requests && start <= b));
+  }
+  const int r = owned - 1;
+  if (r >= 0) tile = b - int(((int64_t(a.qsl[r]) * a.group) >> 6) + r);
+  return r;
+}
+
+template <int DT, int BITS, int DMAX, bool SPLIT>
 __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs a) {
   static_assert(DT != FXPR_DTYPE_F32, "16-bit inputs only");
   using TR = Traits<DT>;
@@ -1664,16 +1719,22 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
 
   const int tid = threadIdx.x, lane = tid & 63, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = blockIdx.x / a.num_kv_heads, g = blockIdx.x % a.num_kv_heads;
+  const int g = blockIdx.x % a.num_kv_heads;
+  // Row tiles last to first: under causal masking the later rows attend the
+  // most keys, so the longest workgroups start first and the short ones fill
+  // the tail (B = 4 x 2048 tokens: -6 %, one 8192-token prompt: -9 %).
+  int r = blockIdx.x / a.num_kv_heads, rtile = int(gridDim.y - 1 - blockIdx.y);
+  if (a.pq_blocks > 0) {
+    r = __builtin_amdgcn_readfirstlane(flat_block(a, a.pq_blocks - 1 - r, rtile));
+    rtile = __builtin_amdgcn_readfirstlane(rtile);
+    if (r < 0 || rtile < 0) return;  // uniform
+  }
   const int q_start = a.qsl[r];
   const int q_len = a.qsl[r + 1] - q_start;
   const int seq_len = a.seq_lens[r];
   const int ctx = seq_len - q_len;
   const int rows_total = q_len * a.group;
-  // Row tiles last to first: under causal masking the later rows attend the
-  // most keys, so the longest workgroups start first and the short ones fill
-  // the tail (B = 4 x 2048 tokens: -6 %, one 8192-token prompt: -9 %).
-  const int row0 = int(gridDim.y - 1 - blockIdx.y) * PQROWS;
+  const int row0 = rtile * PQROWS;
   if (row0 >= rows_total || rows_total < a.pq_rows) return;  // uniform; short requests: the 16-row kernels
   const int wrow0 = row0 + 16 * wave;
 
@@ -1683,8 +1744,15 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
   const int lo = a.window > 0 ? max(0, ctx + i_min - a.window + 1) : 0;
   const int t_lo = lo / TILE;
   const int t_hi = hi > lo ? (hi + TILE - 1) / TILE : t_lo;
-  const int c_lo = t_lo / CT;
-  const int c_hi = t_hi > t_lo ? (t_hi + CT - 1) / CT : c_lo;
+  const int c_first = t_lo / CT;
+  int c_end = t_hi > t_lo ? (t_hi + CT - 1) / CT : c_first;
+  if constexpr (SPLIT) c_end = min(c_end, a.chunk_slots);
+  // this workgroup's chunks
+  const int nch = max(0, c_end - c_first);
+  const int split = SPLIT ? int(blockIdx.z) : 0;
+  const int per = SPLIT ? (nch + a.pq_splits - 1) / a.pq_splits : nch;
+  const int c_lo = c_first + min(nch, split * per);
+  const int c_hi = min(c_first + nch, c_lo + per);
 
   const ConstI32Ptr bt_row = (ConstI32Ptr)(a.bt + int64_t(r) * a.sbt);
   const int last_block = int(a.num_blocks - 1 < 0x7fffffff ? a.num_blocks - 1 : 0x7fffffff);
@@ -1891,6 +1959,20 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
   for (int b = 0; b < DBLK; ++b)
 #pragma unroll
     for (int e = 0; e < 4; ++e) Wr[b][e] = 0;
+
+  // the row's record of chunk c (or the folded state, as chunk c's)
+  auto store_record = [&](int c, float m, AccT den, const AccT (&w)[DBLK][4]) __attribute__((always_inline)) {
+    if (!me.valid) return;
+    const int64_t slot = (ws_row(a, r, q_start, me.token) * a.num_heads + me.head) * a.chunk_slots + c;
+    if (kg == 0) {
+      a.pmax[slot] = m;
+      static_cast<AccT*>(a.den_ws)[slot] = den;
+    }
+    typedef AccT acc4 __attribute__((ext_vector_type(4)));
+    acc4* wp = reinterpret_cast<acc4*>(static_cast<AccT*>(a.wv_ws) + slot * DMAX + 4 * kg);
+#pragma unroll
+    for (int b = 0; b < DBLK; ++b) wp[4 * b] = acc4{w[b][0], w[b][1], w[b][2], w[b][3]};
+  };
 
   // Fast variant (same bits): no softcap or ALiBi and a positive scale, so a
   // score is fl(acc * scale) and the chunk maximum is fl(max(acc) * scale)
@@ -2158,7 +2240,9 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
       // the chunk's denominator over the row's four lanes, then the fold
       den = wadd<BITS>(den, __shfl_xor(den, 16, 64));
       den = wadd<BITS>(den, __shfl_xor(den, 32, 64));
-      if (__builtin_amdgcn_ballot_w64(Mr != -__builtin_inff()) == 0) {
+      if (SPLIT && split > 0) {  // uniform
+        store_record(c, mx, den, wv);
+      } else if (__builtin_amdgcn_ballot_w64(Mr != -__builtin_inff()) == 0) {
         // no row of the wave has folded a chunk yet (W = D = 0, M = -inf):
         // the fold gives the chunk's own sums (rescale(0, 0) + rescale(x, 1));
         // a row without a key here has zero sums (its weights are 0 and a
@@ -2210,7 +2294,16 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
     }
   }
 
-  if (me.valid) {
+  if constexpr (SPLIT) {
+    if (split == 0) {
+      if (c_lo < c_hi) store_record(c_hi - 1, Mr, Dr, Wr);
+      if (me.valid && kg == 0) {
+        int* cr = a.crange + 2 * (ws_row(a, r, q_start, me.token) * a.num_heads + me.head);
+        cr[0] = c_lo < c_hi ? c_hi - 1 : c_first;
+        cr[1] = c_end;
+      }
+    }
+  } else if (me.valid) {
     // the row's 32 quotients over one denominator (in [1e-6, 2^31]; the
     // numerators are fixed-point values below 2^31): by its rounded
     // reciprocal, the same bits as div_rn
@@ -2232,13 +2325,23 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t n
   using T = typename Traits<DT>::T;
   using AccT = typename AccOf<BITS>::T;
   const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  // tokens past query_start_loc[num_requests] belong to no request (e.g. graph
-  // padding) and are left untouched, as in the single-pass path
-  const int64_t used = min<int64_t>(num_tokens, a.qsl[a.num_requests]);
-  const int64_t total = used * a.num_heads * a.head_dim;
-  if (idx >= total) return;
   const int d = int(idx % a.head_dim);
-  const int64_t th = idx / a.head_dim;  // token * Hq + head
+  const int64_t th = idx / a.head_dim;  // workspace row * Hq + head
+  int64_t token = th / a.num_heads;
+  if (a.tok_cap > 0) {
+    // tok_cap rows per request, of requests short of the prefill workgroups
+    const int64_t r = token / a.tok_cap;
+    if (r >= a.num_requests) return;
+    const int i = int(token % a.tok_cap), q0 = a.qsl[r], q_len = a.qsl[r + 1] - q0;
+    if (i >= q_len || q_len * a.group >= a.pq_rows) return;
+    token = q0 + i;
+    if (token < 0 || token >= num_tokens) return;
+  } else {
+    // tokens past query_start_loc[num_requests] belong to no request (e.g. graph
+    // padding) and are left untouched, as in the single-pass path
+    const int64_t used = min<int64_t>(num_tokens, a.qsl[a.num_requests]);
+    if (token >= used) return;
+  }
   float M = -__builtin_inff();
   AccT D = 0, W = 0;
   // batches of NB chunks: every load of a batch is issued (clamped to the
@@ -2294,7 +2397,6 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t n
     }
   }
   const float den_f = fmaxf(acc_f32<BITS>(D, a.fxp_inv), 1.0e-6f);
-  const int64_t token = th / a.num_heads;
   const int head = int(th % a.num_heads);
   static_cast<T*>(a.o)[token * a.so_t + int64_t(head) * a.so_h + d] =
       Io<DT>::store(div_rn(acc_f32<BITS>(W, a.fxp_inv), den_f));
@@ -2332,10 +2434,10 @@ int launch_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
   return 0;
 }
 
-template <int DT, int BITS, int DMAX>
+template <int DT, int BITS, int DMAX, bool SPLIT>
 int launch_prefill_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
   if constexpr (DT != FXPR_DTYPE_F32 && (DMAX == 64 || DMAX == 128)) {
-    auto kern = attn_prefill_dma_kernel<DT, BITS, DMAX>;
+    auto kern = attn_prefill_dma_kernel<DT, BITS, DMAX, SPLIT>;
     constexpr size_t lds = prefill_dma_lds_bytes<DMAX>();
     static bool attr_done = false;  // benign race: the attribute is idempotent
     if (!attr_done) {
@@ -2349,41 +2451,83 @@ int launch_prefill_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
   return 0;
 }
 
+template <int DT, int BITS> int launch_combine(const AttnArgs& a, int64_t ws_rows, int64_t num_tokens, hipStream_t st) {
+  const int64_t total = ws_rows * a.num_heads * a.head_dim;
+  attn_combine_kernel<DT, BITS><<<dim3(unsigned(cdiv(total, 256))), 256, 0, st>>>(a, num_tokens);
+  return launch_status();
+}
+
+// 16-row workgroups of the short requests (fewer than kPrefillRows rows) span
+// at most this many query tiles: a grid over every tile of the longest request
+// would only start workgroups that exit at once
+constexpr int kShortTiles = (kPrefillRows - 1 + QROWS - 1) / QROWS;
+
+// Requests of at least kPrefillRows rows in 64-row workgroups, the others
+// (decode steps, short prompts) in 16-row ones; both kernels see the whole
+// batch and each skips the other's requests. Same bits per row either way.
+// empty workgroups of the request-by-tile prefill grid from which the flat one
+// is taken: it costs a load of the token bounds per workgroup and the
+// longest-first order across requests (three prompts of 921 tokens among four
+// decode steps, 1500 empty workgroups: 53 us flat, 47 not; one of 512 among 31,
+// 7700 empty: the launch 8 us shorter)
+constexpr int64_t kFlatEmpty = 4096;
+
 template <int DT, int BITS, int DMAX>
-int launch_attn(const AttnArgs& a, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st) {
+int launch_long(AttnArgs a, const LongPlan& lp, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st) {
+  a.pq_rows = kPrefillRows;
+  a.pq_splits = lp.pq_splits;
+  a.num_splits = lp.splits;
+  a.chunks_per_split = lp.chunks_per_split;
+  a.tok_cap = lp.tok_cap;
+  a.pmax = lp.pmax;
+  a.den_ws = lp.den_ws;
+  a.wv_ws = lp.wv_ws;
+  a.crange = lp.crange;
+  const int64_t ptiles = cdiv(int64_t(max_qtiles) * QROWS, PQROWS);
+  // a flat grid over the tokens where requests x the longest one's tiles
+  // would be mostly empty (continuous batching: one prompt chunk, many
+  // decode steps); else request by tile, longest tiles first across requests
+  const int64_t flat = num_tokens * a.group / PQROWS + num_requests;
+  dim3 pgrid(unsigned(num_requests * a.num_kv_heads), unsigned(ptiles), unsigned(lp.pq_splits));
+  if ((num_requests * ptiles - flat) * a.num_kv_heads * lp.pq_splits > kFlatEmpty) {
+    a.pq_blocks = int(flat);
+    pgrid = dim3(unsigned(flat * a.num_kv_heads), 1, unsigned(lp.pq_splits));
+  }
+  const bool prefill_split = lp.pq_splits > 1;
+  int e = prefill_split ? launch_prefill_dma<DT, BITS, DMAX, true>(a, pgrid, st)
+                        : launch_prefill_dma<DT, BITS, DMAX, false>(a, pgrid, st);
+  if (e) return e;
+  // (split prefill rows are combined with the short ones: those then leave
+  // records too, whatever their split count)
+  const bool split = prefill_split || lp.splits > 1;
+  const dim3 sgrid(unsigned(num_requests * a.num_kv_heads), unsigned(max_qtiles < kShortTiles ? max_qtiles : kShortTiles),
+                   unsigned(lp.splits));
+  e = split ? launch_dma<DT, BITS, DMAX, true>(a, sgrid, st) : launch_dma<DT, BITS, DMAX, false>(a, sgrid, st);
+  if (e) return e;
+  if (split)
+    return launch_combine<DT, BITS>(a, a.tok_cap > 0 ? int64_t(num_requests) * a.tok_cap : num_tokens, num_tokens, st);
+  return launch_status();
+}
+
+template <int DT, int BITS, int DMAX>
+int launch_attn(const AttnArgs& a, const LongPlan& lp, int num_requests, int max_qtiles, int64_t num_tokens,
+                hipStream_t st) {
   dim3 grid(unsigned(num_requests * a.num_kv_heads), unsigned(max_qtiles), unsigned(a.num_splits));
   const bool dma = dma_ok<DT, DMAX>(a);
-  if (a.num_splits <= 1) {
-    if constexpr (DT != FXPR_DTYPE_F32 && BITS <= 32 && DMAX <= 128) {
-      // Requests of at least kPrefillRows rows run in 64-row workgroups,
-      // the others (decode steps, short prompts) in attn_kernel's 16-row
-      // ones; both kernels see the whole batch and each skips the other's
-      // requests. Same bits per row either way.
-      if (int64_t(max_qtiles) * QROWS >= kPrefillRows) {
-        AttnArgs b = a;
-        b.pq_rows = kPrefillRows;
-        const int ptiles = int(cdiv(int64_t(max_qtiles) * QROWS, PQROWS));
-        const dim3 pgrid(grid.x, unsigned(ptiles), 1);
-        if (dma) {
-          const int e = launch_prefill_dma<DT, BITS, DMAX>(b, pgrid, st);
-          if (e) return e;
-        } else {
-          attn_prefill_kernel<DT, BITS, DMAX><<<pgrid, kPThreads, 0, st>>>(b);
-        }
-        // the short requests (fewer than kPrefillRows rows) span at most
-        // this many 16-row tiles: a grid over every tile of the longest
-        // request would only start workgroups that exit at once
-        const int64_t short_tiles = cdiv(kPrefillRows - 1, QROWS);
-        const dim3 sgrid(grid.x, unsigned(max_qtiles < short_tiles ? max_qtiles : short_tiles), 1);
-        if (dma) {
-          const int e = launch_dma<DT, BITS, DMAX, false>(b, sgrid, st);
-          if (e) return e;
-        } else {
-          attn_kernel<DT, BITS, DMAX, false><<<sgrid, kThreads, 0, st>>>(b);
-        }
-        return launch_status();
-      }
+  if constexpr (DT != FXPR_DTYPE_F32 && BITS <= 32 && DMAX <= 128) {
+    if (lp.use && dma) return launch_long<DT, BITS, DMAX>(a, lp, num_requests, max_qtiles, num_tokens, st);
+    if (a.num_splits <= 1 && int64_t(max_qtiles) * QROWS >= kPrefillRows) {
+      // as launch_long, on the register-load kernels
+      AttnArgs b = a;
+      b.pq_rows = kPrefillRows;
+      const dim3 pgrid(grid.x, unsigned(cdiv(int64_t(max_qtiles) * QROWS, PQROWS)), 1);
+      attn_prefill_kernel<DT, BITS, DMAX><<<pgrid, kPThreads, 0, st>>>(b);
+      const dim3 sgrid(grid.x, unsigned(max_qtiles < kShortTiles ? max_qtiles : kShortTiles), 1);
+      attn_kernel<DT, BITS, DMAX, false><<<sgrid, kThreads, 0, st>>>(b);
+      return launch_status();
     }
+  }
+  if (a.num_splits <= 1) {
     if (dma) {
       const int e = launch_dma<DT, BITS, DMAX, false>(a, grid, st);
       if (e) return e;
@@ -2398,22 +2542,23 @@ int launch_attn(const AttnArgs& a, int num_requests, int max_qtiles, int64_t num
   } else {
     attn_kernel<DT, BITS, DMAX, true><<<grid, kThreads, 0, st>>>(a);
   }
-  const int64_t total = num_tokens * a.num_heads * a.head_dim;
-  attn_combine_kernel<DT, BITS><<<dim3(unsigned(cdiv(total, 256))), 256, 0, st>>>(a, num_tokens);
-  return launch_status();
+  return launch_combine<DT, BITS>(a, num_tokens, num_tokens, st);
 }
 
 template <int DT, int BITS>
-int dispatch_dmax(const AttnArgs& a, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st) {
-  if (a.head_dim <= 64) return launch_attn<DT, BITS, 64>(a, num_requests, max_qtiles, num_tokens, st);
-  if (a.head_dim <= 128) return launch_attn<DT, BITS, 128>(a, num_requests, max_qtiles, num_tokens, st);
+int dispatch_dmax(const AttnArgs& a, const LongPlan& lp, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st) {
+  if (a.head_dim <= 64) return launch_attn<DT, BITS, 64>(a, lp, num_requests, max_qtiles, num_tokens, st);
+  if (a.head_dim <= 128) return launch_attn<DT, BITS, 128>(a, lp, num_requests, max_qtiles, num_tokens, st);
   if constexpr (DT == FXPR_DTYPE_F32) return FXPR_E_SHAPE;  // fp32 tiles beyond 128 exceed LDS
-  else return launch_attn<DT, BITS, 256>(a, num_requests, max_qtiles, num_tokens, st);
+  else return launch_attn<DT, BITS, 256>(a, lp, num_requests, max_qtiles, num_tokens, st);
 }
 
-int run_attn_bf16(const AttnArgs& a, int bits, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st);
-int run_attn_f16(const AttnArgs& a, int bits, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st);
-int run_attn_f32(const AttnArgs& a, int bits, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st);
+int run_attn_bf16(const AttnArgs& a, const LongPlan& lp, int bits, int num_requests, int max_qtiles,
+                 int64_t num_tokens, hipStream_t st);
+int run_attn_f16(const AttnArgs& a, const LongPlan& lp, int bits, int num_requests, int max_qtiles,
+                 int64_t num_tokens, hipStream_t st);
+int run_attn_f32(const AttnArgs& a, const LongPlan& lp, int bits, int num_requests, int max_qtiles,
+                 int64_t num_tokens, hipStream_t st);
 
 }  // namespace attn
 }  // namespace fxpr
