@@ -3,7 +3,7 @@
     python check_lds_reads.py [source.hip ...]
 
 The kernels that stage tiles with LDS DMA (gemm_big_kernel, gemm_f32_kernel, attn_dma_kernel,
-attn_prefill_dma_kernel) read LDS with inline-asm ds_read instructions and
+attn_prefill_dma_kernel, attn_mix_dma_kernel) read LDS with inline-asm ds_read instructions and
 wait for them with explicit s_waitcnt lgkmcnt(N): the compiler would otherwise
 wait for every DMA in flight before each LDS read it can see. To the compiler
 an inline-asm read's destination is ready at issue, so nothing but the kernel's
@@ -55,7 +55,7 @@ sys.path.insert(0, str(HERE))
 from build import COMMON_FLAGS, CSRC, FILE_FLAGS, hipcc  # noqa: E402
 
 DEFAULT_SOURCES = ["gemm_bf16.hip", "gemm_f16.hip", "gemm_f32.hip", "attn_bf16.hip", "attn_f16.hip"]
-KERNELS = re.compile(r"^(_ZN4fxpr\w*(gemm_big_kernel|gemm_f32_kernel|attn_dma_kernel|attn_prefill_dma_kernel)\w*):")
+KERNELS = re.compile(r"^(_ZN4fxpr\w*(gemm_big_kernel|gemm_f32_kernel|attn_dma_kernel|attn_prefill_dma_kernel|attn_mix_dma_kernel)\w*):")
 ALL_KERNELS = re.compile(r"^(_ZN4fxpr\w+):")
 MFMA_WAIT_STATES = 19
 

@@ -279,6 +279,8 @@ extern "C" int fxpr_unified_attention(
   a.num_blocks = num_blocks;
   a.num_tokens = num_tokens;
   a.lmax = int64_t(max_blocks_per_seq) * page_size;
+  const int esz = io_dtype == FXPR_DTYPE_F32 ? 4 : 2;
+  a.o_vec = stride_o_token % kCombineVec == 0 && stride_o_head % kCombineVec == 0 && aligned(o, kCombineVec * esz);
   a.ps_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(unsigned(page_size)) : -1;
   a.scale_log2 = softmax_scale_log2;
   a.softcap_log2 = softcap_log2;

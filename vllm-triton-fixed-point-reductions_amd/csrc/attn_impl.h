@@ -28,6 +28,7 @@
 // order: no atomics, nothing to pre-zero.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -59,7 +60,7 @@ struct AttnArgs {
   const int32_t* seq_lens;
   const int32_t* bt;
   const float* alibi;  // per q head, already multiplied by log2(e); or null
-  // split launches: records of W workspace rows (see ws_row)
+  // split launches: records of W workspace rows (tokens, or tok_cap per request)
   float* pmax;         // [W, Hq, chunk_slots] per-chunk row maxima
   void* den_ws;        // [W, Hq, chunk_slots] denominators, int32 / int64
   void* wv_ws;         // [W, Hq, chunk_slots, D] weighted V, int32 / int64
@@ -77,6 +78,7 @@ struct AttnArgs {
   int64_t num_blocks;   // physical blocks in the cache
   int64_t num_tokens;   // rows of q / o
   int64_t lmax;         // key capacity of a block-table row (max_blocks * page_size)
+  int o_vec;            // output rows aligned for kCombineVec elements at a time
   int ps_shift;         // log2(page_size) if a power of two, else -1
   float scale_log2, softcap_log2, fxp_scale, fxp_inv;
 };
@@ -165,13 +167,6 @@ __device__ __forceinline__ RowInfo row_info(const AttnArgs& a, int g, int q_star
   ri.kend = a.causal ? min(seq_len, ri.qpos + 1) : seq_len;
   ri.kstart = a.window > 0 ? max(0, ri.qpos - a.window + 1) : 0;
   return ri;
-}
-
-// Workspace row of a query token: the token itself, or (tok_cap) a slot among
-// tok_cap per request, where only short requests are split and the long ones'
-// many tokens need no records.
-__device__ __forceinline__ int64_t ws_row(const AttnArgs& a, int r, int q_start, int64_t token) {
-  return a.tok_cap > 0 ? int64_t(r) * a.tok_cap + (token - q_start) : token;
 }
 
 // Per-row statistics of key chunks are folded in fixed point: an accumulator
@@ -771,8 +766,14 @@ template <int K, int NDMA> __device__ __forceinline__ void dma_wait(int later) {
   }
 }
 
-template <int DT, int BITS, int DMAX, bool SPLIT>
-__global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
+// (bx, qt, split: the workgroup's place in a (request x kv head, query tile,
+// key split) grid)
+// CAP (split): the workspace row of a token is not the token but one of tok_cap
+// per request: only short requests leave records, and the long ones' many
+// tokens need no room. (An instance of its own: the shift's scalar registers
+// cost spills in the plain one.)
+template <int DT, int BITS, int DMAX, bool SPLIT, bool CAP>
+__device__ __forceinline__ void attn_dma_body(const AttnArgs& a, const unsigned bx, const int qt, const int split) {
   static_assert(DT != FXPR_DTYPE_F32, "16-bit inputs only");
   using TR = Traits<DT>;
   using T = typename TR::T;
@@ -795,11 +796,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
   const unsigned lds0 = (__builtin_amdgcn_groupstaticsize() + 15u) & ~15u;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kg = lane >> 4;
-  const int g = blockIdx.x % a.num_kv_heads;
+  const int g = bx % a.num_kv_heads;
   // (the request index is wave-uniform: its bounds are scalar loads, issued
   // together and waited for once)
-  const int r = __builtin_amdgcn_readfirstlane(request_by_length(a, blockIdx.x / a.num_kv_heads));
-  const int qt = blockIdx.y, split = blockIdx.z;
+  const int r = __builtin_amdgcn_readfirstlane(request_by_length(a, bx / a.num_kv_heads));
   const ConstI32Ptr bt_row = (ConstI32Ptr)(a.bt + int64_t(r) * a.sbt);
   // Without a window, with a fixed chunk count per split (or one split),
   // the first chunk and so the pages of the first NS steps (its first K
@@ -824,6 +824,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
   const int ctx = seq_len - q_len;
   const int rows_total = q_len * a.group;
   const int row0 = qt * QROWS;
+  [[maybe_unused]] auto ws_row = [&](int64_t token) { return CAP ? int64_t(r) * a.tok_cap + (token - q_start) : token; };
   if (row0 >= rows_total) return;  // uniform
   if (a.pq_rows > 0 && rows_total >= a.pq_rows) return;  // attn_prefill_kernel's request
 
@@ -1188,7 +1189,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
         for (int e = 0; e < 4; ++e) {
           const RowInfo ri = row_info(a, g, q_start, q_len, ctx, seq_len, row0 + 4 * kg + e);
           if (!ri.valid) continue;
-          const int64_t slot = (ws_row(a, r, q_start, ri.token) * a.num_heads + ri.head) * a.chunk_slots + c;
+          const int64_t slot = (ws_row(ri.token) * a.num_heads + ri.head) * a.chunk_slots + c;
           if ((lane & 15) == 0 && wave == 0) {
             a.pmax[slot] = mc[e];
             static_cast<AccT*>(a.den_ws)[slot] = dc[e];
@@ -1230,7 +1231,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
   if (SPLIT && split == 0 && tid < QROWS) {
     const RowInfo ri = row_info(a, g, q_start, q_len, ctx, seq_len, row0 + tid);
     if (ri.valid) {
-      int* cr = a.crange + 2 * (ws_row(a, r, q_start, ri.token) * a.num_heads + ri.head);
+      int* cr = a.crange + 2 * (ws_row(ri.token) * a.num_heads + ri.head);
       cr[0] = c_lo;
       cr[1] = c_lo + nch;
     }
@@ -1254,6 +1255,11 @@ __global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
       }
     }
   }
+}
+
+template <int DT, int BITS, int DMAX, bool SPLIT, bool CAP>
+__global__ __launch_bounds__(kThreads, 2) void attn_dma_kernel(AttnArgs a) {
+  attn_dma_body<DT, BITS, DMAX, SPLIT, CAP>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 template <int DMAX> constexpr size_t dma_lds_bytes() {
@@ -1697,8 +1703,11 @@ __device__ __forceinline__ int flat_block(const AttnArgs& a, int b, int& tile) {
   return r;
 }
 
+// (bx, ytile, zsplit: the workgroup's place in a (request or flat block x kv
+// head, row tile counted from the last, key split) grid of ytiles row tiles)
 template <int DT, int BITS, int DMAX, bool SPLIT>
-__global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs a) {
+__device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const unsigned bx, const int ytile, const int ytiles,
+                                                      const int zsplit) {
   static_assert(DT != FXPR_DTYPE_F32, "16-bit inputs only");
   using TR = Traits<DT>;
   using T = typename TR::T;
@@ -1719,11 +1728,11 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
 
   const int tid = threadIdx.x, lane = tid & 63, kg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = blockIdx.x % a.num_kv_heads;
+  const int g = bx % a.num_kv_heads;
   // Row tiles last to first: under causal masking the later rows attend the
   // most keys, so the longest workgroups start first and the short ones fill
   // the tail (B = 4 x 2048 tokens: -6 %, one 8192-token prompt: -9 %).
-  int r = blockIdx.x / a.num_kv_heads, rtile = int(gridDim.y - 1 - blockIdx.y);
+  int r = bx / a.num_kv_heads, rtile = ytiles - 1 - ytile;
   if (a.pq_blocks > 0) {
     r = __builtin_amdgcn_readfirstlane(flat_block(a, a.pq_blocks - 1 - r, rtile));
     rtile = __builtin_amdgcn_readfirstlane(rtile);
@@ -1749,7 +1758,7 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
   if constexpr (SPLIT) c_end = min(c_end, a.chunk_slots);
   // this workgroup's chunks
   const int nch = max(0, c_end - c_first);
-  const int split = SPLIT ? int(blockIdx.z) : 0;
+  const int split = SPLIT ? zsplit : 0;
   const int per = SPLIT ? (nch + a.pq_splits - 1) / a.pq_splits : nch;
   const int c_lo = c_first + min(nch, split * per);
   const int c_hi = min(c_first + nch, c_lo + per);
@@ -1963,7 +1972,7 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
   // the row's record of chunk c (or the folded state, as chunk c's)
   auto store_record = [&](int c, float m, AccT den, const AccT (&w)[DBLK][4]) __attribute__((always_inline)) {
     if (!me.valid) return;
-    const int64_t slot = (ws_row(a, r, q_start, me.token) * a.num_heads + me.head) * a.chunk_slots + c;
+    const int64_t slot = (me.token * a.num_heads + me.head) * a.chunk_slots + c;
     if (kg == 0) {
       a.pmax[slot] = m;
       static_cast<AccT*>(a.den_ws)[slot] = den;
@@ -2298,7 +2307,7 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
     if (split == 0) {
       if (c_lo < c_hi) store_record(c_hi - 1, Mr, Dr, Wr);
       if (me.valid && kg == 0) {
-        int* cr = a.crange + 2 * (ws_row(a, r, q_start, me.token) * a.num_heads + me.head);
+        int* cr = a.crange + 2 * (me.token * a.num_heads + me.head);
         cr[0] = c_lo < c_hi ? c_hi - 1 : c_first;
         cr[1] = c_end;
       }
@@ -2318,21 +2327,62 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs
   }
 }
 
+template <int DT, int BITS, int DMAX, bool SPLIT>
+__global__ __launch_bounds__(kPThreads, 2) void attn_prefill_dma_kernel(AttnArgs a) {
+  attn_prefill_dma_body<DT, BITS, DMAX, SPLIT>(a, blockIdx.x, blockIdx.y, gridDim.y, blockIdx.z);
+}
+
+// The prefill workgroups and the short requests' 16-row ones of one unsplit
+// launch in one grid, prefill first, for batches whose workgroups all fit on
+// the GPU at once (two per CU): both kinds then wait on their own DMA latency
+// side by side instead of one launch after the other (four prompts of 95
+// tokens beside six decode steps: 14 + 24 -> 26 us). Larger batches keep two
+// launches: with each kind saturating its own resource, a shared CU serves
+// both worse (512 new tokens over 3500 cached beside 31 decode steps: 370 us
+// interleaved in one grid, 105 + 125 apart).
+struct MixGrid {
+  int pq_x, pq_y;  // prefill grid
+  int sh_x, sh_y;  // short requests' grid
+};
+template <int DT, int BITS, int DMAX>
+__global__ __launch_bounds__(kPThreads, 2) void attn_mix_dma_kernel(AttnArgs a, MixGrid m) {
+  static_assert(kPThreads == kThreads, "one workgroup shape");
+  const int b = blockIdx.x, np = m.pq_x * m.pq_y;
+  if (b < np) {
+    const int y = b / m.pq_x;
+    attn_prefill_dma_body<DT, BITS, DMAX, false>(a, b - y * m.pq_x, y, m.pq_y, 0);
+  } else {
+    const int y = (b - np) / m.sh_x;
+    attn_dma_body<DT, BITS, DMAX, false, false>(a, b - np - y * m.sh_x, y, 0);
+  }
+}
+
 // Fold the per-chunk partials of each (token, head) in ascending chunk order
-// (the kernel's single-pass fold, step for step) and divide.
-template <int DT, int BITS>
+// (the kernel's single-pass fold, step for step) and divide. A thread takes V
+// consecutive d. Decode launches (V = 1) are bound by their two dependent round
+// trips (range, then records: 6.6 us at 64 x 32 rows; 7.6 with V = 4); those
+// with split prefill rows (V = 4) by reading the records, so there a record is
+// one 16-byte load, the row's maximum and denominator are folded once for the
+// four, and no record is loaded before its row's range is known (543 tokens x
+// 32 heads of 8 records: 34 -> 21 us; 478 x 28 heads: 58 -> 27 us).
+constexpr int kCombineVec = 4;
+template <int DT, int BITS, int V>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t num_tokens) {
   using T = typename Traits<DT>::T;
   using AccT = typename AccOf<BITS>::T;
-  const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  const int d = int(idx % a.head_dim);
-  const int64_t th = idx / a.head_dim;  // workspace row * Hq + head
-  int64_t token = th / a.num_heads;
+  typedef AccT accv __attribute__((ext_vector_type(V)));
+  // (32-bit indices: kSplitWsMax keeps the workspace rows' elements below 2^28)
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x, per_row = uint32_t(a.head_dim) / V;
+  const uint32_t th = idx / per_row;  // workspace row * Hq + head
+  const int d = int(idx - th * per_row) * V;
+  const uint32_t wrow = th / uint32_t(a.num_heads);
+  const int head = int(th - wrow * uint32_t(a.num_heads));
+  int64_t token = wrow;
   if (a.tok_cap > 0) {
     // tok_cap rows per request, of requests short of the prefill workgroups
-    const int64_t r = token / a.tok_cap;
-    if (r >= a.num_requests) return;
-    const int i = int(token % a.tok_cap), q0 = a.qsl[r], q_len = a.qsl[r + 1] - q0;
+    const uint32_t r = wrow / uint32_t(a.tok_cap);
+    if (r >= uint32_t(a.num_requests)) return;
+    const int i = int(wrow - r * uint32_t(a.tok_cap)), q0 = a.qsl[r], q_len = a.qsl[r + 1] - q0;
     if (i >= q_len || q_len * a.group >= a.pq_rows) return;
     token = q0 + i;
     if (token < 0 || token >= num_tokens) return;
@@ -2343,52 +2393,62 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t n
     if (token >= used) return;
   }
   float M = -__builtin_inff();
-  AccT D = 0, W = 0;
+  AccT D = 0, W[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) W[v] = 0;
   // batches of NB chunks: every load of a batch is issued (clamped to the
   // range) before the sequential fold, so the loads overlap
   constexpr int NB = 16;
-  const AccT* den_p = static_cast<const AccT*>(a.den_ws) + th * a.chunk_slots;
-  const AccT* wv_p = static_cast<const AccT*>(a.wv_ws) + th * a.chunk_slots * a.head_dim + d;
-  const float* pm_p = a.pmax + th * a.chunk_slots;
+  const AccT* den_p = static_cast<const AccT*>(a.den_ws) + int64_t(th) * a.chunk_slots;
+  const AccT* wv_p = static_cast<const AccT*>(a.wv_ws) + int64_t(th) * a.chunk_slots * a.head_dim + d;
+  const float* pm_p = a.pmax + int64_t(th) * a.chunk_slots;
   float mc[NB];
-  AccT dc[NB], wc[NB];
+  AccT dc[NB];
+  accv wc[NB];
   auto load = [&](int cb, int c_end) __attribute__((always_inline)) {
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
       const int c = min(cb + k, c_end - 1);
       mc[k] = pm_p[c];
       dc[k] = den_p[c];
-      wc[k] = wv_p[int64_t(c) * a.head_dim];
+      wc[k] = *reinterpret_cast<const accv*>(wv_p + int64_t(c) * a.head_dim);
     }
   };
   // Mn is M or mc[k], so fa or fb is 2^0 = 1 (unless both maxima are +inf:
   // inf - inf is NaN), and rescale(x, 1) = x for 16- and 32-bit sums (exact
-  // in fp64): those rescale one side only. The side is the same for the
-  // whole (token, head), i.e. for every lane of the wave.
+  // in fp64): those rescale one side only.
   auto fold = [&](int cb, int c_end) __attribute__((always_inline)) {
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
       if (cb + k >= c_end || mc[k] == -__builtin_inff()) continue;
       float Mn, fa, fb;
       merge_factors(M, mc[k], Mn, fa, fb);
-      if (BITS != 64 && fa == 1.0f) {
+      const bool one_a = fa == 1.0f;
+      if (BITS != 64 && V == 1 && one_a) {  // V = 1: a wave is one row (or two)
         D = wadd<BITS>(D, rescale<BITS>(dc[k], fb));
-        W = wadd<BITS>(W, rescale<BITS>(wc[k], fb));
-      } else if (BITS != 64 && fb == 1.0f) {
+        W[0] = wadd<BITS>(W[0], rescale<BITS>(wc[k][0], fb));
+      } else if (BITS != 64 && V == 1 && fb == 1.0f) {
         D = wadd<BITS>(rescale<BITS>(D, fa), dc[k]);
-        W = wadd<BITS>(rescale<BITS>(W, fa), wc[k]);
+        W[0] = wadd<BITS>(rescale<BITS>(W[0], fa), wc[k][0]);
+      } else if (BITS != 64 && (one_a || fb == 1.0f)) {
+        const float f = one_a ? fb : fa;
+        D = wadd<BITS>(rescale<BITS>(one_a ? dc[k] : D, f), one_a ? D : dc[k]);
+#pragma unroll
+        for (int v = 0; v < V; ++v) W[v] = wadd<BITS>(rescale<BITS>(one_a ? wc[k][v] : W[v], f), one_a ? W[v] : wc[k][v]);
       } else {
         D = wadd<BITS>(rescale<BITS>(D, fa), rescale<BITS>(dc[k], fb));
-        W = wadd<BITS>(rescale<BITS>(W, fa), rescale<BITS>(wc[k], fb));
+#pragma unroll
+        for (int v = 0; v < V; ++v) W[v] = wadd<BITS>(rescale<BITS>(W[v], fa), rescale<BITS>(wc[k][v], fb));
       }
       M = Mn;
     }
   };
-  // The first batch goes out with the range loads (the range of a row
+  // V = 1: the first batch goes out with the range loads (the range of a row
   // usually starts at chunk 0 and fits one batch): one round trip, not two.
-  if (a.chunk_slots > 0) load(0, a.chunk_slots);
-  const int c0 = max(0, a.crange[2 * th]), c1 = min(a.chunk_slots, a.crange[2 * th + 1]);
-  if (c0 == 0 && c1 <= NB) {
+  const bool early = V == 1 && a.chunk_slots > 0;  // uniform
+  if (early) load(0, a.chunk_slots);
+  const int c0 = max(0, a.crange[2 * int64_t(th)]), c1 = min(a.chunk_slots, a.crange[2 * int64_t(th) + 1]);
+  if (early && c0 == 0 && c1 <= NB) {
     fold(0, c1);
   } else {
     for (int cb = c0; cb < c1; cb += NB) {
@@ -2397,9 +2457,17 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t n
     }
   }
   const float den_f = fmaxf(acc_f32<BITS>(D, a.fxp_inv), 1.0e-6f);
-  const int head = int(th % a.num_heads);
-  static_cast<T*>(a.o)[token * a.so_t + int64_t(head) * a.so_h + d] =
-      Io<DT>::store(div_rn(acc_f32<BITS>(W, a.fxp_inv), den_f));
+  T* o = static_cast<T*>(a.o) + token * a.so_t + int64_t(head) * a.so_h + d;
+  if (V > 1 && a.o_vec) {  // uniform
+    typedef T outv __attribute__((ext_vector_type(V)));
+    outv y;
+#pragma unroll
+    for (int v = 0; v < V; ++v) y[v] = Io<DT>::store(div_rn(acc_f32<BITS>(W[v], a.fxp_inv), den_f));
+    *reinterpret_cast<outv*>(o) = y;
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; ++v) o[v] = Io<DT>::store(div_rn(acc_f32<BITS>(W[v], a.fxp_inv), den_f));
+  }
 }
 
 // attn_dma_kernel serves a launch when each wave's 16 key rows of a tile lie
@@ -2417,10 +2485,10 @@ template <int DT, int DMAX> bool dma_ok(const AttnArgs& a) {
   }
 }
 
-template <int DT, int BITS, int DMAX, bool SPLIT>
+template <int DT, int BITS, int DMAX, bool SPLIT, bool CAP = false>
 int launch_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
   if constexpr (DT != FXPR_DTYPE_F32 && (DMAX == 64 || DMAX == 128)) {
-    auto kern = attn_dma_kernel<DT, BITS, DMAX, SPLIT>;
+    auto kern = attn_dma_kernel<DT, BITS, DMAX, SPLIT, CAP>;
     constexpr size_t lds = dma_lds_bytes<DMAX>();
     static bool attr_done = false;  // benign race: the attribute is idempotent
     if (!attr_done) {
@@ -2430,6 +2498,23 @@ int launch_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
       attr_done = true;
     }
     kern<<<grid, kThreads, lds, st>>>(a);
+  }
+  return 0;
+}
+
+template <int DT, int BITS, int DMAX>
+int launch_mix(const AttnArgs& a, const MixGrid& m, hipStream_t st) {
+  if constexpr (DT != FXPR_DTYPE_F32 && DMAX == 128) {
+    auto kern = attn_mix_dma_kernel<DT, BITS, DMAX>;
+    constexpr size_t lds = std::max(prefill_dma_lds_bytes<DMAX>(), dma_lds_bytes<DMAX>());
+    static bool attr_done = false;  // benign race: the attribute is idempotent
+    if (!attr_done) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+      if (e != hipSuccess) return int(e);
+      attr_done = true;
+    }
+    kern<<<dim3(unsigned(m.pq_x * m.pq_y + m.sh_x * m.sh_y)), kThreads, lds, st>>>(a, m);
   }
   return 0;
 }
@@ -2453,7 +2538,14 @@ int launch_prefill_dma(const AttnArgs& a, dim3 grid, hipStream_t st) {
 
 template <int DT, int BITS> int launch_combine(const AttnArgs& a, int64_t ws_rows, int64_t num_tokens, hipStream_t st) {
   const int64_t total = ws_rows * a.num_heads * a.head_dim;
-  attn_combine_kernel<DT, BITS><<<dim3(unsigned(cdiv(total, 256))), 256, 0, st>>>(a, num_tokens);
+  if constexpr (BITS <= 32 && DT != FXPR_DTYPE_F32) {
+    if (a.pq_splits > 1) {
+      attn_combine_kernel<DT, BITS, kCombineVec>
+          <<<dim3(unsigned(cdiv(total / kCombineVec, 256))), 256, 0, st>>>(a, num_tokens);
+      return launch_status();
+    }
+  }
+  attn_combine_kernel<DT, BITS, 1><<<dim3(unsigned(cdiv(total, 256))), 256, 0, st>>>(a, num_tokens);
   return launch_status();
 }
 
@@ -2493,16 +2585,25 @@ int launch_long(AttnArgs a, const LongPlan& lp, int num_requests, int max_qtiles
     a.pq_blocks = int(flat);
     pgrid = dim3(unsigned(flat * a.num_kv_heads), 1, unsigned(lp.pq_splits));
   }
-  const bool prefill_split = lp.pq_splits > 1;
+  // (split prefill rows are combined with the short ones: those then leave
+  // records too, whatever their split count)
+  const bool prefill_split = lp.pq_splits > 1, split = prefill_split || lp.splits > 1;
+  const dim3 sgrid(unsigned(num_requests * a.num_kv_heads), unsigned(max_qtiles < kShortTiles ? max_qtiles : kShortTiles),
+                   unsigned(lp.splits));
+  // (head_dim 128 only: at 64 the prefill workgroups fit four per CU, which
+  // the other body's registers would halve)
+  if (DMAX == 128 && !split && num_requests > 1 &&
+      cdiv(num_tokens * a.num_heads, PQROWS) + int64_t(num_requests) * a.num_kv_heads <= 512) {
+    const MixGrid m{int(pgrid.x), int(pgrid.y), int(sgrid.x), int(sgrid.y)};
+    const int rc = launch_mix<DT, BITS, DMAX>(a, m, st);
+    return rc ? rc : launch_status();
+  }
   int e = prefill_split ? launch_prefill_dma<DT, BITS, DMAX, true>(a, pgrid, st)
                         : launch_prefill_dma<DT, BITS, DMAX, false>(a, pgrid, st);
   if (e) return e;
-  // (split prefill rows are combined with the short ones: those then leave
-  // records too, whatever their split count)
-  const bool split = prefill_split || lp.splits > 1;
-  const dim3 sgrid(unsigned(num_requests * a.num_kv_heads), unsigned(max_qtiles < kShortTiles ? max_qtiles : kShortTiles),
-                   unsigned(lp.splits));
-  e = split ? launch_dma<DT, BITS, DMAX, true>(a, sgrid, st) : launch_dma<DT, BITS, DMAX, false>(a, sgrid, st);
+  e = !split          ? launch_dma<DT, BITS, DMAX, false>(a, sgrid, st)
+      : a.tok_cap > 0 ? launch_dma<DT, BITS, DMAX, true, true>(a, sgrid, st)
+                      : launch_dma<DT, BITS, DMAX, true>(a, sgrid, st);
   if (e) return e;
   if (split)
     return launch_combine<DT, BITS>(a, a.tok_cap > 0 ? int64_t(num_requests) * a.tok_cap : num_tokens, num_tokens, st);
