@@ -674,3 +674,22 @@ def test_mixed_batch_wide_block_table_and_graph():
         torch.cuda.synchronize()
         assert torch.equal(o, base)
         torch.randn(1 << 20, device="cuda").sum()
+
+
+@pytest.mark.parametrize("softcap", [0.5, 50.0])
+def test_prefill_softcap_extreme_scores(softcap):
+    # the prefill workgroups take a chunk's maximum before the softcap; rows
+    # whose raw scores overflow to +-inf, or that see one key only, get the bits
+    # of the 16-row kernels, which cap every score first (group 1, 47 rows)
+    g = torch.Generator("cpu").manual_seed(2)
+    n, L = 130, 700
+    q, kv, qsl, sl, bt, max_q = _ragged([(n, L)], 2, 2, 128, 16, torch.bfloat16, 9)
+    q[5] *= 1e30
+    q[60, 0] = -q[60, 0] * 1e36
+    kv[:, 0, 3] *= 1e8
+    whole = _attend((q, kv, qsl, sl, bt, max_q), 1, softcap=softcap)
+    for lo in range(0, n, 47):
+        m = min(47, n - lo)
+        part = (q[lo:lo + m].contiguous(), kv, torch.tensor([0, m], dtype=torch.int32, device="cuda"),
+                torch.tensor([L - n + lo + m], dtype=torch.int32, device="cuda"), bt, m)
+        assert torch.equal(_attend(part, 1, softcap=softcap), whole[lo:lo + m]), lo

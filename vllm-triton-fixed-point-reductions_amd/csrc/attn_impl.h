@@ -136,6 +136,8 @@ template <int BITS> __device__ __forceinline__ float acc_f32(typename AccOf<BITS
   else return fixed_to_f32(v, inv);
 }
 
+constexpr float kFltMax = 3.402823466e38f;
+
 __device__ __forceinline__ float tanh_approx(float x) {
   // tanh(x) = sign(x) (1 - 2 / (2^(2|x| log2 e) + 1)); tolerance path only
   const float e = __builtin_amdgcn_exp2f(2.0f * 1.44269504088896341f * __builtin_fabsf(x));
@@ -1990,10 +1992,16 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
   // its range, see fast_den); P is packed without the canonical-NaN rule (any
   // NaN weight yields a NaN weighted V either way, which quantises to 0).
   const bool fast_den = BITS != 64 && a.fxp_scale <= (BITS == 16 ? 16384.0f : 4194304.0f);
-  const bool fast = fast_den && !(a.softcap_log2 > 0.0f) && !a.alibi && a.scale_log2 > 0.0f;
+  // With a softcap the same holds around it (CAP): tanh_approx is monotone
+  // (checked over every fp32 value), so the chunk maximum is the capped maximum
+  // of the raw scores, and only phase 1 computes a score's tanh and divisions
+  // (3 x up to 1018 tokens after up to 5643, 32 heads: 1.24 -> 0.73 ms).
+  const bool cap = a.softcap_log2 > 0.0f;
+  const bool fast = fast_den && !a.alibi && a.scale_log2 > 0.0f;
   const float vlim = (BITS == 16 ? 32767.0f : 4194304.0f) / a.fxp_scale;  // 2^f: exact
-  auto run = [&](auto fast_tag) __attribute__((always_inline)) {
-    constexpr bool FAST = decltype(fast_tag)::value;
+  auto run = [&](auto fast_tag, auto cap_tag) __attribute__((always_inline)) {
+    constexpr bool FAST = decltype(fast_tag)::value, CAP = decltype(cap_tag)::value;
+    auto capped = [&](float x) { return a.softcap_log2 * tanh_approx(x / a.softcap_log2); };
     // A step consumes C ring entries (1: a K tile of phase 0; 2: a tile's K
     // and V in phase 1) and issues C more: the cursor stays NS - 2 entries
     // ahead, so the two slots a 2-entry step refills are free. Returns the
@@ -2077,14 +2085,18 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
     // Scores of chain q of tile t for the lane's row and keys
     // t * TILE + 32 (q >> 1) + 8 kg + 4 (q & 1) + e; whole: the wave's rows see
     // the whole tile.
-    auto chain_scores = [&](const f32x4& acc, int t, int q, bool whole, float (&sc)[4]) __attribute__((always_inline)) {
+    // (RAW: before the softcap; the mask is -inf, a score of -inf is not.)
+    auto chain_scores = [&](const f32x4& acc, int t, int q, bool whole, auto raw_tag, float (&sc)[4]) __attribute__((always_inline)) {
+      constexpr bool RAW = decltype(raw_tag)::value;
       const int key0 = t * TILE + 32 * (q >> 1) + 8 * kg + 4 * (q & 1);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         float x = __fmul_rn(acc[e], a.scale_log2);
         if constexpr (!FAST) {
-          if (a.softcap_log2 > 0.0f) x = a.softcap_log2 * tanh_approx(x / a.softcap_log2);
+          if (a.softcap_log2 > 0.0f) x = capped(x);
           if (a.alibi) x = x + slope * static_cast<float>(key0 + e - qp);
+        } else if constexpr (CAP) {
+          x = RAW ? fmaxf(x, -kFltMax) : capped(x);
         }
         sc[e] = (whole || (key0 + e >= ks && key0 + e < ke)) ? x : -__builtin_inff();
       }
@@ -2103,17 +2115,23 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
           key_groups(base, [&](auto, const f32x4& acc) __attribute__((always_inline)) {
             mraw = fmaxf(fmaxf(mraw, fmaxf(acc[0], acc[1])), fmaxf(acc[2], acc[3]));
           });
+          if constexpr (CAP) mraw = fmaxf(mraw, -kFltMax);  // keys were seen
         } else {
           key_groups(base, [&](auto qc, const f32x4& acc) __attribute__((always_inline)) {
             float sc[4];
-            chain_scores(acc, t, decltype(qc)::value, false, sc);
+            chain_scores(acc, t, decltype(qc)::value, false, std::true_type{}, sc);
             mx = fmaxf(fmaxf(mx, fmaxf(sc[0], sc[1])), fmaxf(sc[2], sc[3]));
           });
         }
       }
-      if constexpr (FAST) mx = fmaxf(mx, __fmul_rn(mraw, a.scale_log2));
+      if constexpr (FAST) {
+        float m1 = __fmul_rn(mraw, a.scale_log2);
+        if constexpr (CAP) m1 = mraw != -__builtin_inff() ? fmaxf(m1, -kFltMax) : m1;
+        mx = fmaxf(mx, m1);
+      }
       mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if constexpr (CAP) mx = mx != -__builtin_inff() ? capped(mx) : mx;
       const float m = mx != -__builtin_inff() ? mx : 0.0f;  // no key: pin to 0
       // phase 1: weights and weighted V, tile by tile
       AccT den = 0;
@@ -2136,7 +2154,7 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
             key_groups(base, [&](auto qc, const f32x4& acc) __attribute__((always_inline)) {
               constexpr int q = decltype(qc)::value, s = q >> 1, h = q & 1;
               float sc[4];
-              chain_scores(acc, t, q, WHOLE, sc);
+              chain_scores(acc, t, q, WHOLE, std::false_type{}, sc);
               float w[4];
 #pragma unroll
               for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_exp2f(sc[i] - m);
@@ -2294,12 +2312,14 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
   };
   if (c_lo < c_hi) {
     if constexpr (BITS != 64) {
-      if (fast)
-        run(std::true_type{});
+      if (fast && cap)
+        run(std::true_type{}, std::true_type{});
+      else if (fast)
+        run(std::true_type{}, std::false_type{});
       else
-        run(std::false_type{});
+        run(std::false_type{}, std::false_type{});
     } else {
-      run(std::false_type{});
+      run(std::false_type{}, std::false_type{});
     }
   }
 
