@@ -1,10 +1,13 @@
-"""Build libfxpr_hip.so (the gfx950 kernels + C ABI) in-tree with hipcc.
+"""Build libfxpr_hip.so (the gfx950 kernels + C ABI) and libfxpr_torch.so (the
+torch.ops.fxpr launchers) in-tree.
 
     python build.py [--jobs N] [--verbose]
 
 Each csrc/*.hip file is compiled to an object under _build/ and the objects
 are linked into fxpr_vllm/libfxpr_hip.so, which fxpr_vllm/_hip.py loads with
-ctypes. hipcc cross-compiles for gfx950, so this works without a GPU.
+ctypes; csrc/torch_ops.cpp is compiled by the host compiler against torch's
+headers and linked to it. hipcc cross-compiles for gfx950, so this works
+without a GPU.
 """
 
 from __future__ import annotations
@@ -22,6 +25,7 @@ REPO = HERE.parent
 CSRC = HERE / "csrc"
 BUILD = HERE / "_build"
 OUT = HERE / "fxpr_vllm" / "libfxpr_hip.so"
+TORCH_OUT = HERE / "fxpr_vllm" / "libfxpr_torch.so"
 ARCH = os.environ.get("FXPR_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32.
@@ -91,6 +95,23 @@ def _check_defined(lib: Path) -> None:
         raise RuntimeError(f"{lib.name}: undefined symbols of the library's own code: {missing[:4]}")
 
 
+def torch_commands(obj: Path, hip_lib: Path, out: Path) -> tuple[list[str], list[str]]:
+    """Compile and link commands of the torch launchers. (torch's own headers
+    for ROCm are plain C++: no device code here, so any host compiler.)"""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    cxx = shutil.which("g++") or shutil.which("c++") or hipcc()
+    compile_ = [cxx, "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{REPO / 'include'}",
+                f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+                f"-I{Path(os.environ.get('ROCM_PATH', '/opt/rocm')) / 'include'}",
+                "-c", str(CSRC / "torch_ops.cpp"), "-o", str(obj)]
+    link = [cxx, "-shared", "-fPIC", str(obj), str(hip_lib), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_hip", "-ltorch", "-Wl,-rpath,$ORIGIN", "-o", str(out)]
+    return compile_, link
+
+
 def build(jobs: int | None = None, verbose: bool = False) -> Path:
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
@@ -98,19 +119,25 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     BUILD.mkdir(exist_ok=True)
     cc = hipcc()
     objs = [BUILD / (s.stem + ".o") for s in sources]
-    jobs = jobs or min(8, len(sources))
+    jobs = jobs or min(8, len(sources) + 1)
+    torch_obj, torch_tmp = BUILD / "torch_ops.o", TORCH_OUT.with_suffix(".so.tmp")
+    torch_cc, torch_ld = torch_commands(torch_obj, OUT, torch_tmp)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = [
             ex.submit(_run, [cc, *COMMON_FLAGS, *FILE_FLAGS.get(s.name, []), "-c", str(s), "-o", str(o)], verbose)
             for s, o in zip(sources, objs)
         ]
+        futs.append(ex.submit(_run, torch_cc, verbose))
         for f in futs:
             f.result()
     tmp = OUT.with_suffix(".so.tmp")
-    _run([cc, "-shared", f"--offload-arch={ARCH}", "-fPIC", *map(str, objs), "-o", str(tmp)],
+    # (the soname is how libfxpr_torch.so finds it, beside itself)
+    _run([cc, "-shared", f"--offload-arch={ARCH}", "-fPIC", f"-Wl,-soname,{OUT.name}", *map(str, objs), "-o", str(tmp)],
          verbose)
     _check_defined(tmp)
     os.replace(tmp, OUT)
+    _run(torch_ld, verbose)
+    os.replace(torch_tmp, TORCH_OUT)
     return OUT
 
 

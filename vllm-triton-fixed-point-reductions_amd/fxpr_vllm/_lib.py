@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import torch
 
+from . import _hip
 from ._kernels import attention as _attention
 from ._kernels import cache as _cache
 from ._kernels import casts as _casts
@@ -181,17 +182,36 @@ def _log_softmax_fxp_shard_finish_cuda(x, row_max, row_sum, fxp_frac_bits, out_d
     return _rows.log_softmax_shard_finish_run(x, row_max, row_sum, int(fxp_frac_bits), out_dtype)
 
 
-# Register after definition so the functions stay importable by name.
-_lib.impl("float_to_fixed", _float_to_fixed_cuda, "CUDA")
-_lib.impl("fixed_to_float", _fixed_to_float_cuda, "CUDA")
-_lib.impl("rms_norm_fxp", _rms_norm_fxp_cuda, "CUDA")
-_lib.impl("rms_norm_fxp_residual", _rms_norm_fxp_residual_cuda, "CUDA")
-_lib.impl("gemm_fxp", _gemm_fxp_cuda, "CUDA")
-_lib.impl("unified_attention_fxp", _unified_attention_fxp_cuda, "CUDA")
-_lib.impl("fixed_row_sum", _fixed_row_sum_cuda, "CUDA")
-_lib.impl("log_softmax_fxp", _log_softmax_fxp_cuda, "CUDA")
-_lib.impl("reshape_and_cache", _reshape_and_cache_cuda, "CUDA")
-_lib.impl("sample_greedy_fxp", _sample_greedy_fxp_cuda, "CUDA")
+# The launchers of the hot ops are native (csrc/torch_ops.cpp, beside the
+# kernel library): they register themselves for the "CUDA" key when loaded. The
+# Python launchers below serve the remaining ops, and every op where the native
+# library has not been built (they raise without the kernel library).
+_NATIVE_PATH = _hip.LIB_PATH.with_name("libfxpr_torch.so")
+_NATIVE = _NATIVE_PATH.exists()
+if _NATIVE:
+    try:
+        torch.ops.load_library(str(_NATIVE_PATH))
+    except OSError as e:
+        raise RuntimeError(
+            f"fxpr: {_NATIVE_PATH} does not load with this torch ({torch.__version__}): {e}; rebuild it "
+            "(`python build.py` in the package directory)") from e
+
+# op -> Python launcher, native counterpart in csrc/torch_ops.cpp
+_WITH_NATIVE = {
+    "float_to_fixed": _float_to_fixed_cuda,
+    "fixed_to_float": _fixed_to_float_cuda,
+    "rms_norm_fxp": _rms_norm_fxp_cuda,
+    "rms_norm_fxp_residual": _rms_norm_fxp_residual_cuda,
+    "gemm_fxp": _gemm_fxp_cuda,
+    "unified_attention_fxp": _unified_attention_fxp_cuda,
+    "fixed_row_sum": _fixed_row_sum_cuda,
+    "log_softmax_fxp": _log_softmax_fxp_cuda,
+    "reshape_and_cache": _reshape_and_cache_cuda,
+    "sample_greedy_fxp": _sample_greedy_fxp_cuda,
+}
+for _name, _fn in _WITH_NATIVE.items():
+    if not _NATIVE:
+        _lib.impl(_name, _fn, "CUDA")
 _lib.impl("gemm_fxp_partial", _gemm_fxp_partial_cuda, "CUDA")
 _lib.impl("gemm_fxp_finish", _gemm_fxp_finish_cuda, "CUDA")
 _lib.impl("log_softmax_fxp_shard_max", _log_softmax_fxp_shard_max_cuda, "CUDA")
