@@ -204,3 +204,31 @@ def test_multi_workgroup_threshold(dtype, vocab_off):
     for k in (0, 7):
         one, multi = _sample_both_paths(x.to(DEV), k, 32, 16)
         _paths_equal(one, multi)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 32), (16, 8)])
+@pytest.mark.parametrize("cols", [1, 3, 7, 9, 15, 100, 2051, 4105, 33001])
+def test_ragged_widths_equal_element_loads(dtype, bits, frac, cols):
+    # widths that are no whole number of 16-byte vectors: rows start at every
+    # offset of a vector, and share their first and last with their neighbours.
+    # An input whose base is not 16-byte aligned loads element by element: the
+    # same bits, with infinite, NaN, flat and tied rows among them
+    rows = 19
+    g = torch.Generator("cpu").manual_seed(cols)
+    x = torch.randn(rows, cols, generator=g) * 4
+    x[1] = float("-inf")
+    x[2, cols // 2] = float("inf")
+    x[3, cols - 1] = float("nan")
+    x[4] = 1.0
+    x[5] = torch.randint(0, 3, (cols,), generator=g).float()
+    x[6, 0], x[6, 1:] = 2.0, float("-inf")
+    x = x.to(dtype).cuda()
+    off = torch.empty(rows * cols + 1, dtype=dtype, device="cuda")[1:].view(rows, cols).copy_(x)
+    assert off.data_ptr() % 16 and x.data_ptr() % 16 == 0
+    for out in (None, torch.float32):
+        a, b = (torch.ops.fxpr.log_softmax_fxp(t, bits, frac, out) for t in (x, off))
+        assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)) and torch.equal(a.isnan(), b.isnan())
+    for k in {0, min(5, cols), min(64, cols)}:
+        for a, b in zip(*(torch.ops.fxpr.sample_greedy_fxp(t, k, bits, frac) for t in (x, off))):
+            assert torch.equal(a.double().nan_to_num(7.0), b.double().nan_to_num(7.0))

@@ -314,7 +314,7 @@ int launch_rms(const void* x, void* r, const void* w, void* y, int64_t rows, int
 
 // One workgroup per row: row_lse, then y_j = OUT(fl32(x_j) - lse) from the
 // chunks kept in registers (later chunks re-read).
-template <int XDT, int YDT, int VEC, int NREG, int BITS, bool WIDE>
+template <int XDT, int YDT, int VEC, int NREG, int BITS, bool WIDE, bool RAG>
 __global__ __launch_bounds__(kLsmThreads) void log_softmax_kernel(
     const typename Io<XDT>::T* __restrict__ x, typename Io<YDT>::T* __restrict__ y, int64_t cols,
     int frac, float inv_scale, int fast_sum) {
@@ -324,27 +324,34 @@ __global__ __launch_bounds__(kLsmThreads) void log_softmax_kernel(
   __shared__ LseSum<WIDE> ired[kLsmThreads / 64];
 
   const int64_t row = blockIdx.x;
-  const int64_t nchunks = cols / VEC;
   const int nthr = blockDim.x;
   const int tid = threadIdx.x;
-  const XV* xr = reinterpret_cast<const XV*>(x + row * cols);
-  YV* yr = reinterpret_cast<YV*>(y + row * cols);
+  const RowVecs<XDT, VEC, RAG> xr(x, row, cols);
+  const int64_t nchunks = xr.n;
+  // (RAG: the vectors of y are those of x)
+  YV* yr = reinterpret_cast<YV*>(y + (row * cols - xr.head));
 
   XV keep[NREG];
-  const float lse = row_lse<XDT, VEC, NREG, BITS, WIDE>(xr, keep, nchunks, frac, inv_scale, fast_sum, fred, ired);
+  const float lse = row_lse<XDT, VEC, NREG, BITS, WIDE>(xr, keep, frac, inv_scale, fast_sum, fred, ired);
 
   auto emit = [&](int64_t c, const XV& xv) {
     YV yv;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) yv.v[j] = Io<YDT>::store(__fsub_rn(Io<XDT>::load(xv.v[j]), lse));
-    yr[c] = yv;
+    if (xr.whole(c)) {
+      yr[c] = yv;
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        if (xr.in_row(c, j)) y[row * cols + xr.index(c, j)] = yv.v[j];
+    }
   };
 #pragma unroll
   for (int i = 0; i < NREG; ++i) {
     const int64_t c = tid + static_cast<int64_t>(i) * nthr;
     if (c < nchunks) emit(c, keep[i]);
   }
-  for (int64_t c = tid + static_cast<int64_t>(NREG) * nthr; c < nchunks; c += nthr) emit(c, xr[c]);
+  for (int64_t c = tid + static_cast<int64_t>(NREG) * nthr; c < nchunks; c += nthr) emit(c, xr.load(c));
 }
 
 // ---------------------------------------------------------------------------
@@ -702,7 +709,7 @@ bool try_lsm_split(const void* x, void* y, int64_t rows, int64_t cols, int frac,
   return true;
 }
 
-template <int XDT, int YDT, int VEC>
+template <int XDT, int YDT, int VEC, bool RAG>
 int launch_lsm_vec(const void* x, void* y, int64_t rows, int64_t cols, int bits, int frac,
                    hipStream_t st) {
   using XT = typename Io<XDT>::T;
@@ -710,7 +717,7 @@ int launch_lsm_vec(const void* x, void* y, int64_t rows, int64_t cols, int bits,
   constexpr int NREG = VEC == 1 ? 8 : 32;
   const LseShape sh = lse_shape(cols, VEC, NREG, bits, frac);
   // (128-bit sums, for near-flat rows at large f, keep the one-workgroup kernel)
-  if constexpr (VEC > 1) {
+  if constexpr (VEC > 1 && !RAG) {
     int rc = FXPR_OK;
     bool done = false;
     if (bits == 16) done = try_lsm_split<XDT, YDT, VEC, 16, false>(x, y, rows, cols, frac, st, &rc);
@@ -724,13 +731,13 @@ int launch_lsm_vec(const void* x, void* y, int64_t rows, int64_t cols, int bits,
   YT* yp = static_cast<YT*>(y);
   const int n = sh.threads;
   if (bits == 16)
-    log_softmax_kernel<XDT, YDT, VEC, NREG, 16, false><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, sh.fast_sum);
+    log_softmax_kernel<XDT, YDT, VEC, NREG, 16, false, RAG><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, sh.fast_sum);
   else if (bits == 32)
-    log_softmax_kernel<XDT, YDT, VEC, NREG, 32, false><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, sh.fast_sum);
+    log_softmax_kernel<XDT, YDT, VEC, NREG, 32, false, RAG><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, sh.fast_sum);
   else if (!sh.wide)
-    log_softmax_kernel<XDT, YDT, VEC, NREG, 64, false><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, 0);
+    log_softmax_kernel<XDT, YDT, VEC, NREG, 64, false, RAG><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, 0);
   else
-    log_softmax_kernel<XDT, YDT, VEC, NREG, 64, true><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, 0);
+    log_softmax_kernel<XDT, YDT, VEC, NREG, 64, true, RAG><<<grid, n, 0, st>>>(xp, yp, cols, frac, inv, 0);
   return launch_status();
 }
 
@@ -739,9 +746,11 @@ int launch_lsm(const void* x, void* y, int64_t rows, int64_t cols, int bits, int
   using XT = typename Io<XDT>::T;
   using YT = typename Io<YDT>::T;
   constexpr int VEC = 16 / sizeof(XT);
-  if (cols % VEC == 0 && aligned(x, 16) && aligned(y, sizeof(YT) * VEC))
-    return launch_lsm_vec<XDT, YDT, VEC>(x, y, rows, cols, bits, frac, st);
-  return launch_lsm_vec<XDT, YDT, 1>(x, y, rows, cols, bits, frac, st);
+  if (aligned(x, 16) && aligned(y, sizeof(YT) * VEC)) {
+    if (cols % VEC == 0) return launch_lsm_vec<XDT, YDT, VEC, false>(x, y, rows, cols, bits, frac, st);
+    return launch_lsm_vec<XDT, YDT, VEC, true>(x, y, rows, cols, bits, frac, st);
+  }
+  return launch_lsm_vec<XDT, YDT, 1, false>(x, y, rows, cols, bits, frac, st);
 }
 
 // ---------------------------------------------------------------------------

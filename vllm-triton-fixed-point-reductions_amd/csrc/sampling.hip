@@ -41,7 +41,7 @@ __device__ __forceinline__ uint64_t order_key(float v, int64_t j) {
   return (static_cast<uint64_t>(value_order(v)) << 32) | (0xfffffffeu - static_cast<uint32_t>(j));
 }
 
-template <int XDT, int VEC, int NREG, int BITS, bool WIDE>
+template <int XDT, int VEC, int NREG, int BITS, bool WIDE, bool RAG>
 __global__ __launch_bounds__(kLsmThreads) void sample_greedy_kernel(
     const typename Io<XDT>::T* __restrict__ x, int64_t cols, int rounds, int frac, float inv_scale,
     int fast_sum, int64_t* __restrict__ sampled, float* __restrict__ sampled_logprob,
@@ -53,15 +53,15 @@ __global__ __launch_bounds__(kLsmThreads) void sample_greedy_kernel(
   __shared__ uint64_t kred[2][kLsmThreads / 64];
 
   const int64_t row = blockIdx.x;
-  const int64_t nchunks = cols / VEC;
+  const RowVecs<XDT, VEC, RAG> xr(x, row, cols);
+  const int64_t nchunks = xr.n;
   const int nthr = blockDim.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6, nwaves = nthr >> 6;
   const XT* xrow = x + row * cols;
-  const XV* xr = reinterpret_cast<const XV*>(xrow);
 
   XV keep[NREG];
-  const float lse = row_lse<XDT, VEC, NREG, BITS, WIDE>(xr, keep, nchunks, frac, inv_scale, fast_sum, fred, ired);
+  const float lse = row_lse<XDT, VEC, NREG, BITS, WIDE>(xr, keep, frac, inv_scale, fast_sum, fred, ired);
 
   // the thread's two largest keys below `below` (0: none; keys are never 0)
   uint64_t h1 = 0, h2 = 0;
@@ -80,8 +80,8 @@ __global__ __launch_bounds__(kLsmThreads) void sample_greedy_kernel(
     auto consider = [&](int64_t c, const XV& xv) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        uint64_t key = order_key(Io<XDT>::load(xv.v[j]), c * VEC + j);
-        key = key < below ? key : 0;
+        uint64_t key = order_key(Io<XDT>::load(xv.v[j]), xr.index(c, j));
+        key = key < below && xr.in_row(c, j) ? key : 0;
         const bool gt1 = key > h1, gt2 = key > h2;
         h2 = gt1 ? h1 : (gt2 ? key : h2);
         h1 = gt1 ? key : h1;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kLsmThreads) void sample_greedy_kernel(
       const int64_t c = t + static_cast<int64_t>(i) * nthr;
       if (c < nchunks) consider(c, keep[i]);
     }
-    for (int64_t c = t + static_cast<int64_t>(NREG) * nthr; c < nchunks; c += nthr) consider(c, xr[c]);
+    for (int64_t c = t + static_cast<int64_t>(NREG) * nthr; c < nchunks; c += nthr) consider(c, xr.load(c));
   };
   scan(~uint64_t(0));
 
@@ -140,9 +140,6 @@ constexpr int kSpanThreads = 256;
 constexpr int kSpanNreg = 8;
 constexpr int kMaxSpans = 16;
 constexpr int kMultiMaxRows = 128;   // from here the one-workgroup kernel fills the CUs
-constexpr int kFinalThreads = 256;   // kMaxSpans * kMaxLogprobs keys, four per thread
-static_assert(kFinalThreads == kSpanThreads, "block_max_key's shared slots are sized for kSpanThreads");
-static_assert(kMaxSpans * kMaxLogprobs % kFinalThreads == 0, "whole keys per thread");
 
 __device__ __forceinline__ float block_maximum(float v, float* smem) {
 #pragma unroll
@@ -167,7 +164,7 @@ __device__ __forceinline__ uint64_t block_max_key(uint64_t v, uint64_t (&kred)[2
   return best;
 }
 
-template <int XDT, int VEC>
+template <int XDT, int VEC, bool RAG>
 __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
     const typename Io<XDT>::T* __restrict__ x, int64_t cols, int spans, int64_t span_chunks, int rounds,
     float* __restrict__ maxima, uint64_t* __restrict__ cand) {
@@ -178,11 +175,10 @@ __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
   __shared__ uint64_t kred[2][kSpanThreads / 64];
 
   const int64_t row = blockIdx.x / spans;
-  const int64_t nchunks = cols / VEC;
+  const RowVecs<XDT, VEC, RAG> xr(x, row, cols);
   const int64_t c0 = (blockIdx.x % spans) * span_chunks;
-  const int64_t c1 = min(nchunks, c0 + span_chunks);
+  const int64_t c1 = min(xr.n, c0 + span_chunks);
   const int nthr = blockDim.x, tid = threadIdx.x;
-  const XV* xr = reinterpret_cast<const XV*>(x + row * cols);
 
   XV keep[NREG];
   float m = -__builtin_inff();
@@ -190,13 +186,13 @@ __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
   for (int i = 0; i < NREG; ++i) {
     const int64_t c = c0 + tid + static_cast<int64_t>(i) * nthr;
     if (c < c1) {
-      keep[i] = xr[c];
+      keep[i] = xr.load(c);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) m = __builtin_elementwise_maximum(m, Io<XDT>::load(keep[i].v[j]));
     }
   }
   for (int64_t c = c0 + tid + static_cast<int64_t>(NREG) * nthr; c < c1; c += nthr) {
-    const XV xv = xr[c];
+    const XV xv = xr.load(c);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) m = __builtin_elementwise_maximum(m, Io<XDT>::load(xv.v[j]));
   }
@@ -217,8 +213,8 @@ __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
     auto consider = [&](int64_t c, const XV& xv) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        uint64_t key = order_key(Io<XDT>::load(xv.v[j]), c * VEC + j);
-        key = key < below ? key : 0;
+        uint64_t key = order_key(Io<XDT>::load(xv.v[j]), xr.index(c, j));
+        key = key < below && xr.in_row(c, j) ? key : 0;
         const bool gt1 = key > h1, gt2 = key > h2;
         h2 = gt1 ? h1 : (gt2 ? key : h2);
         h1 = gt1 ? key : h1;
@@ -229,7 +225,7 @@ __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
       const int64_t c = c0 + t + static_cast<int64_t>(i) * nthr;
       if (c < c1) consider(c, keep[i]);
     }
-    for (int64_t c = c0 + t + static_cast<int64_t>(NREG) * nthr; c < c1; c += nthr) consider(c, xr[c]);
+    for (int64_t c = c0 + t + static_cast<int64_t>(NREG) * nthr; c < c1; c += nthr) consider(c, xr.load(c));
   };
   scan(~uint64_t(0));
   for (int r = 0; r < rounds; ++r) {
@@ -243,7 +239,17 @@ __global__ __launch_bounds__(kSpanThreads) void sample_span_kernel(
   }
 }
 
-template <int XDT, int VEC, int BITS, bool WIDE>
+// The maximum of a row's span maxima (every lane of the wave).
+__device__ __forceinline__ float spans_maximum(const float* p, int spans) {
+  static_assert(kMaxSpans <= 16, "a span per lane of 16");
+  const int t = threadIdx.x & 15;
+  float m = p[t < spans ? t : 0];
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) m = __builtin_elementwise_maximum(m, __shfl_xor(m, o, 64));
+  return m;
+}
+
+template <int XDT, int VEC, int BITS, bool WIDE, bool RAG>
 __global__ __launch_bounds__(kSpanThreads) void sample_sum_kernel(
     const typename Io<XDT>::T* __restrict__ x, int64_t cols, int spans, int64_t span_chunks, int frac,
     int fast_sum, const float* __restrict__ maxima, LseSum<WIDE>* __restrict__ sums) {
@@ -253,59 +259,61 @@ __global__ __launch_bounds__(kSpanThreads) void sample_sum_kernel(
   __shared__ SumT ired[kSpanThreads / 64];
 
   const int64_t row = blockIdx.x / spans;
-  const int64_t nchunks = cols / VEC;
+  const RowVecs<XDT, VEC, RAG> xr(x, row, cols);
   const int64_t c0 = (blockIdx.x % spans) * span_chunks;
-  const int64_t c1 = min(nchunks, c0 + span_chunks);
-  const XV* xr = reinterpret_cast<const XV*>(x + row * cols);
-  float m = -__builtin_inff();
-  for (int t = 0; t < spans; ++t) m = __builtin_elementwise_maximum(m, maxima[row * spans + t]);
+  const int64_t c1 = min(xr.n, c0 + span_chunks);
+  // (one lane per span maximum: a loop over them waits for a load per span)
+  const float m = spans_maximum(maxima + row * spans, spans);
 
   SumT acc = 0;
   if (BITS != 64 && fast_sum) {
     const float zero_below = exp_zero_below(frac);
     uint32_t acc32 = 0;
-    for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) add_terms_rc<XDT, VEC>(xr[c], m, frac, zero_below, acc32);
+    for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) add_terms_rc<XDT, VEC>(xr.load(c), m, frac, zero_below, acc32);
     acc = acc32;
   } else {
-    for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) add_terms_exact<XDT, VEC, BITS>(xr[c], m, frac, acc);
+    for (int64_t c = c0 + threadIdx.x; c < c1; c += blockDim.x) add_terms_exact<XDT, VEC, BITS>(xr.load(c), m, frac, acc);
   }
   const SumT total = block_exact_sum(acc, ired);
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-template <int XDT, bool WIDE>
-__global__ __launch_bounds__(kFinalThreads) void sample_final_kernel(
+// One wave per row: the spans' maxima and sums one per lane, the keys KPT per
+// lane, and each round one wave maximum (no barriers: as a workgroup of four
+// waves whose threads each looped over the spans' sums this took 6.8 us at
+// 32 rows x 16 spans x 5 keys, now 5.2; the launch itself is most of it).
+template <int XDT, bool WIDE, int KPT>
+__global__ __launch_bounds__(64) void sample_final_kernel(
     const typename Io<XDT>::T* __restrict__ x, int64_t cols, int spans, int rounds, float inv_scale,
     const float* __restrict__ maxima, const LseSum<WIDE>* __restrict__ sums, const uint64_t* __restrict__ cand,
     int64_t* __restrict__ sampled, float* __restrict__ sampled_logprob, int64_t* __restrict__ topk_ids,
     float* __restrict__ topk_logprobs, int num_logprobs) {
   using SumT = LseSum<WIDE>;
-  constexpr int KPT = kMaxSpans * kMaxLogprobs / kFinalThreads;  // keys per thread
-  __shared__ uint64_t kred[2][kSpanThreads / 64];
   const int64_t row = blockIdx.x;
-  const int tid = threadIdx.x;
-  float m = -__builtin_inff();
-  SumT total = 0;
-  for (int t = 0; t < spans; ++t) {
-    m = __builtin_elementwise_maximum(m, maxima[row * spans + t]);
-    total += sums[row * spans + t];
-  }
-  const float lse = lse_of(m, total, inv_scale);
-
+  const int lane = threadIdx.x;
   const int n = spans * rounds;
   const uint64_t* rc = cand + row * n;
   uint64_t key[KPT];
 #pragma unroll
-  for (int q = 0; q < KPT; ++q) key[q] = tid + q * kFinalThreads < n ? rc[tid + q * kFinalThreads] : 0;
+  for (int q = 0; q < KPT; ++q) key[q] = lane + 64 * q < n ? rc[lane + 64 * q] : 0;
+  SumT total = (lane & 15) < spans ? sums[row * spans + (lane & 15)] : SumT(0);
+  const float m = spans_maximum(maxima + row * spans, spans);
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    if constexpr (WIDE) total += shfl_xor_u128(total, o);
+    else total += __shfl_xor(total, o, 64);
+  }
+  const float lse = lse_of(m, total, inv_scale);
+
   const auto* xrow = x + row * cols;
   for (int r = 0; r < rounds; ++r) {
     uint64_t mine = 0;
 #pragma unroll
     for (int q = 0; q < KPT; ++q) mine = key[q] > mine ? key[q] : mine;
-    const uint64_t best = block_max_key(mine, kred, r);
+    const uint64_t best = wave_max(mine);
 #pragma unroll
     for (int q = 0; q < KPT; ++q) key[q] = key[q] == best ? 0 : key[q];  // keys are distinct
-    if (tid == 0 && best != 0) {   // k <= cols, so every round finds a key
+    if (lane == 0 && best != 0) {   // k <= cols, so every round finds a key
       const int64_t j = static_cast<int64_t>(0xfffffffeu - static_cast<uint32_t>(best));
       const float lp = __fsub_rn(Io<XDT>::load(xrow[j]), lse);
       if (r == 0) {
@@ -330,11 +338,11 @@ inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 // Launches the multi-workgroup form if the shape suits it and the workspace
 // holds its partials; false: take the one-workgroup kernel (nothing launched).
-template <int XDT, int VEC>
+template <int XDT, int VEC, bool RAG>
 bool try_sample_multi(const void* x, int64_t rows, int64_t cols, int k, int bits, int frac, int64_t* sampled,
                       float* sampled_lp, int64_t* topk_ids, float* topk_lp, void* ws, int64_t ws_bytes,
                       hipStream_t st, int* rc) {
-  const int64_t nchunks = cols / VEC;
+  const int64_t nchunks = cols / VEC + (RAG ? 2 : 0);  // (at most, with partial vectors at both ends)
   if (!ws || rows > kMultiMaxRows || ws_bytes < sample_ws_bytes(rows, k)) return false;
   int spans = kMaxSpans;
   while (spans > 2 && (rows * spans > 1024 || nchunks / spans < kSpanThreads)) spans /= 2;
@@ -351,30 +359,36 @@ bool try_sample_multi(const void* x, int64_t rows, int64_t cols, int k, int bits
   char* sums = base + align_up(rows * spans * 4, 16);
   uint64_t* cand = reinterpret_cast<uint64_t*>(sums + align_up(rows * spans * 16, 16));
   const dim3 sgrid(static_cast<unsigned>(rows * spans));
-  sample_span_kernel<XDT, VEC><<<sgrid, kSpanThreads, 0, st>>>(xp, cols, spans, span_chunks, rounds, maxima, cand);
+  sample_span_kernel<XDT, VEC, RAG><<<sgrid, kSpanThreads, 0, st>>>(xp, cols, spans, span_chunks, rounds, maxima, cand);
+  // a final wave's keys: two per lane (top 8 of 16 spans), or as many as ever needed
+  const bool few = spans * rounds <= 128;
+#define FXPR_SAMPLE_FINAL(W, KPT)                                                                              \
+  sample_final_kernel<XDT, W, KPT><<<dim3(static_cast<unsigned>(rows)), 64, 0, st>>>(                            \
+      xp, cols, spans, rounds, inv, maxima, reinterpret_cast<const LseSum<W>*>(sums), cand, sampled, sampled_lp, \
+      topk_ids, topk_lp, k)
 #define FXPR_SAMPLE_MULTI(B, W, FAST)                                                                        \
   do {                                                                                                       \
-    sample_sum_kernel<XDT, VEC, B, W><<<sgrid, kSpanThreads, 0, st>>>(xp, cols, spans, span_chunks, frac, FAST, \
-                                                                      maxima, reinterpret_cast<LseSum<W>*>(sums)); \
-    sample_final_kernel<XDT, W><<<dim3(static_cast<unsigned>(rows)), kFinalThreads, 0, st>>>(                  \
-        xp, cols, spans, rounds, inv, maxima, reinterpret_cast<const LseSum<W>*>(sums), cand, sampled,          \
-        sampled_lp, topk_ids, topk_lp, k);                                                                   \
+    sample_sum_kernel<XDT, VEC, B, W, RAG><<<sgrid, kSpanThreads, 0, st>>>(                                   \
+        xp, cols, spans, span_chunks, frac, FAST, maxima, reinterpret_cast<LseSum<W>*>(sums));               \
+    if (few) FXPR_SAMPLE_FINAL(W, 2);                                                                        \
+    else FXPR_SAMPLE_FINAL(W, (kMaxSpans * kMaxLogprobs / 64));                                              \
   } while (0)
   if (bits == 16) FXPR_SAMPLE_MULTI(16, false, fast);
   else if (bits == 32) FXPR_SAMPLE_MULTI(32, false, fast);
   else if (!sh.wide) FXPR_SAMPLE_MULTI(64, false, 0);
   else FXPR_SAMPLE_MULTI(64, true, 0);
 #undef FXPR_SAMPLE_MULTI
+#undef FXPR_SAMPLE_FINAL
   *rc = launch_status();
   return true;
 }
 
-template <int XDT, int VEC>
+template <int XDT, int VEC, bool RAG>
 int launch_sample_vec(const void* x, int64_t rows, int64_t cols, int k, int bits, int frac, int64_t* sampled,
                       float* sampled_lp, int64_t* topk_ids, float* topk_lp, void* ws, int64_t ws_bytes,
                       hipStream_t st) {
   int rc = FXPR_OK;
-  if (try_sample_multi<XDT, VEC>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws, ws_bytes,
+  if (try_sample_multi<XDT, VEC, RAG>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws, ws_bytes,
                                  st, &rc))
     return rc;
   using XT = typename Io<XDT>::T;
@@ -386,7 +400,7 @@ int launch_sample_vec(const void* x, int64_t rows, int64_t cols, int k, int bits
   const XT* xp = static_cast<const XT*>(x);
   const int n = sh.threads;
 #define FXPR_SAMPLE(B, W, FAST) \
-  sample_greedy_kernel<XDT, VEC, NREG, B, W><<<grid, n, 0, st>>>(xp, cols, rounds, frac, inv, FAST, sampled, \
+  sample_greedy_kernel<XDT, VEC, NREG, B, W, RAG><<<grid, n, 0, st>>>(xp, cols, rounds, frac, inv, FAST, sampled, \
                                                                   sampled_lp, topk_ids, topk_lp, k)
   if (bits == 16) FXPR_SAMPLE(16, false, sh.fast_sum);
   else if (bits == 32) FXPR_SAMPLE(32, false, sh.fast_sum);
@@ -401,11 +415,15 @@ int launch_sample(const void* x, int64_t rows, int64_t cols, int k, int bits, in
                   float* sampled_lp, int64_t* topk_ids, float* topk_lp, void* ws, int64_t ws_bytes,
                   hipStream_t st) {
   constexpr int VEC = 16 / sizeof(typename Io<XDT>::T);
-  if (cols % VEC == 0 && aligned(x, 16))
-    return launch_sample_vec<XDT, VEC>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws,
-                                       ws_bytes, st);
-  return launch_sample_vec<XDT, 1>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws,
-                                   ws_bytes, st);
+  if (aligned(x, 16)) {
+    if (cols % VEC == 0)
+      return launch_sample_vec<XDT, VEC, false>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp,
+                                                ws, ws_bytes, st);
+    return launch_sample_vec<XDT, VEC, true>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws,
+                                             ws_bytes, st);
+  }
+  return launch_sample_vec<XDT, 1, false>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws,
+                                          ws_bytes, st);
 }
 
 }  // namespace
