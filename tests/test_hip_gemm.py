@@ -648,3 +648,25 @@ def test_gemm_row_major_b_equals_k_contiguous(dtype, bits, frac, M):
     a[0, 200], b[300, 17], b[640, 399] = float("inf"), float("nan"), 900.0
     kn = _run(a, b, bits=bits, frac=frac, b_layout="kn")
     assert nan_aware_equal(kn, _run(a, b, bits=bits, frac=frac, b_layout="nk"))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("b_layout", ["nk", "kn"])
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 1032), (16, 520, 264), (64, 264, 200), (130, 136, 1016), (200, 264, 249)])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 16)])
+def test_gemm_partial_last_k_tile(dtype, b_layout, M, N, K, bits, frac):
+    # a last K-tile of whole 16-byte chunks, of a partial chunk (K = 249 under a
+    # row stride that keeps rows aligned), at every tile family
+    a, b = _int_mats(M, K, N, seed=M + K, dtype=dtype)
+    want = _oracle(a, b, None, bits, frac)
+    wide = torch.full((M, -(-K // 8) * 8), 5.0, dtype=dtype, device=DEV)
+    wide[:, :K] = a.to(DEV)
+    if b_layout == "kn":
+        bd = b.to(DEV)
+    else:
+        wb = torch.full((N, -(-K // 8) * 8), 5.0, dtype=dtype, device=DEV)
+        wb[:, :K] = b.t().to(DEV)
+        bd = wb[:, :K].t()
+    for split_k in (0, 1, 2):
+        got = KG.gemm_fxp_run(wide[:, :K], bd, None, bits, frac, split_k=split_k).cpu()
+        assert torch.equal(got, want), mismatch_report(got, want)

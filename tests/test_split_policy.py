@@ -153,3 +153,10 @@ def test_gemm_f32_split_fills_whole_rounds(lib):
     assert gemm_splits(lib, 777, 14336, 4096, F32) == 1
     assert gemm_splits(lib, 130, 4096, 4098, F32) == 8       # 64 tiles of 128 x 128
     assert gemm_splits(lib, 130, 4096, 100, F32) <= 2        # 2 K-tiles
+
+
+def test_gemm_auto_decode_shapes_with_a_k_tail(lib):
+    # the streaming kernel takes whole K-tiles only; other K split the skinny tile
+    assert gemm_splits(lib, 1, 4096, 4096 + 16) == 16     # 16 tiles of 16 x 256
+    assert gemm_splits(lib, 16, 8192, 10848) == 16        # 32 tiles
+    assert gemm_splits(lib, 1, 4096, 136) == 2            # 2 K-tiles

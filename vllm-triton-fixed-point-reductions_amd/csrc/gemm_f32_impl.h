@@ -218,13 +218,16 @@ __global__ __launch_bounds__(kThreads, FT::WPE) void gemm_f32_kernel(GemmArgs ar
   // masked loads into both slots, zero past K.
   if (has_tail) {
     const int64_t kt0 = int64_t(kt_end - 1) * 64;
+    const bool whole = args.K % CH == 0;
+#pragma unroll 4
     for (int e = tid; e < 2 * BM * 8; e += kThreads) {
       const int st = e / (BM * 8), r = e % (BM * 8) / 8, c = e % 8;
       const int64_t k = kt0 + st * BKS + c * CH, row = m0 + r;
       const int valid = row < args.M && k < args.K ? int(min<int64_t>(CH, args.K - k)) : 0;
       *reinterpret_cast<uint4*>(smem_raw + st * A_SLOT + r * 128 + ((c ^ ((r >> 1) & 7)) << 4)) =
-          load_chunk<false>(A + (valid ? row * args.lda + k : 0), valid);
+          load_chunk_or_zero(A + (valid ? row * args.lda + k : 0), valid, whole);
     }
+#pragma unroll 4
     for (int e = tid; e < 2 * BN * 8; e += kThreads) {
       const int st = e / (BN * 8), w = e % (BN * 8);
       if constexpr (BNC) {
@@ -232,13 +235,13 @@ __global__ __launch_bounds__(kThreads, FT::WPE) void gemm_f32_kernel(GemmArgs ar
         const int64_t k = kt0 + st * BKS + r, col = n0 + c * CH;
         const int valid = k < args.K && col < args.N ? CH : 0;  // N is a multiple of CH
         *reinterpret_cast<uint4*>(smem_raw + B_RING + st * B_SLOT + r * RB + ((c ^ ((r & 3) << 2)) << 4)) =
-            load_chunk<false>(B + (valid ? k * args.ldb + col : 0), valid);
+            load_chunk_or_zero(B + (valid ? k * args.ldb + col : 0), valid, true);
       } else {
         const int r = w / 8, c = w % 8;
         const int64_t k = kt0 + st * BKS + c * CH, col = n0 + r;
         const int valid = col < args.N && k < args.K ? int(min<int64_t>(CH, args.K - k)) : 0;
         *reinterpret_cast<uint4*>(smem_raw + B_RING + st * B_SLOT + r * 128 + ((c ^ ((r >> 1) & 7)) << 4)) =
-            load_chunk<false>(B + (valid ? col * args.ldb + k : 0), valid);
+            load_chunk_or_zero(B + (valid ? col * args.ldb + k : 0), valid, whole);
       }
     }
     __syncthreads();

@@ -124,6 +124,17 @@ __device__ __forceinline__ uint4 load_chunk(const T* p, int valid) {
   return u.v;
 }
 
+// load_chunk<false> where every chunk is whole or absent (`whole`, uniform: K
+// is a number of chunks): one unconditional 16-byte load (an absent chunk's
+// address is the matrix's first), zeroed by a select, so that a batch of them
+// is in flight together. (With a branch per chunk each waits for the last.)
+template <typename T>
+__device__ __forceinline__ uint4 load_chunk_or_zero(const T* p, int valid, bool whole) {
+  if (!whole) return load_chunk<false>(p, valid);
+  const uint4 v = *reinterpret_cast<const uint4*>(p);
+  return valid ? v : make_uint4(0, 0, 0, 0);
+}
+
 // Workgroup tile -> (tm, tn). Hardware hands consecutive workgroup ids to the
 // 8 XCDs round-robin; remap so each XCD gets one contiguous run of logical
 // tiles (L2 reuse), then group GROUP_M row tiles per column sweep.
@@ -854,29 +865,47 @@ redo_next:
   // K-tile kt into ring slots 0 and 1 of A and B by masked register loads
   // (zero past K), in the swizzled layout, and its partials into P: the
   // peeled tail tile, and the exact recomputation.
+  // (Whole chunks as 16-byte loads, a quarter of a thread's issued together.
+  // Loaded element by element, chunk after chunk, the tail tile of K = 1552
+  // cost M = 4096, N = 6144 143 us in all instead of 122, and a launch whose
+  // tiles all leave the rounding constant's range 570-600 us instead of 320
+  // at M = 1000, N = 6144, K = 4096.)
   auto stage_tile = [&](int kt) {
     const int64_t kt0 = int64_t(kt) * 128;
-    for (int e = tid; e < 2 * (BM + BN) * 8; e += BT::THREADS) {
-      const int st = e / ((BM + BN) * 8), rem = e % ((BM + BN) * 8);
-      if (BNC && rem >= BM * 8) {
-        const int r = (rem - BM * 8) / CPRB, c = (rem - BM * 8) % CPRB;
-        const int64_t k = kt0 + st * BKS + r, col = n0 + c * CH;
-        const int valid = k < args.K && col < args.N ? CH : 0;  // N is a whole number of chunks
-        const uint4 v = load_chunk<false>(B + (valid ? k * args.ldb + col : 0), valid);
-        *reinterpret_cast<uint4*>(smem_raw + B_RING + st * B_SLOT + r * ROWB + ((c ^ bnc_swz(r)) << 4)) = v;
-        continue;
+    constexpr int NCH = 2 * (BM + BN) * 8, IT = NCH / BT::THREADS, Q = IT / 4;
+    static_assert(IT * BT::THREADS == NCH && Q * 4 == IT, "whole chunks per thread");
+    const bool whole = args.K % CH == 0;
+#pragma unroll 1
+    for (int e0 = tid; e0 < NCH; e0 += Q * BT::THREADS) {
+      uint4 v[Q];
+      int at[Q];
+#pragma unroll
+      for (int u = 0; u < Q; ++u) {
+        const int e = e0 + u * BT::THREADS;
+        const int st = e / ((BM + BN) * 8), rem = e % ((BM + BN) * 8);
+        const T* src;
+        int valid;
+        if (BNC && rem >= BM * 8) {
+          const int r = (rem - BM * 8) / CPRB, c = (rem - BM * 8) % CPRB;
+          const int64_t k = kt0 + st * BKS + r, col = n0 + c * CH;
+          valid = k < args.K && col < args.N ? CH : 0;  // N is a whole number of chunks
+          src = B + (valid ? k * args.ldb + col : 0);
+          at[u] = B_RING + st * B_SLOT + r * ROWB + ((c ^ bnc_swz(r)) << 4);
+        } else {
+          const int r = rem / 8, c = rem % 8;
+          const int64_t k = kt0 + st * BKS + c * CH;
+          const bool isa = r < BM;
+          const int64_t row = isa ? m0 + r : n0 + (r - BM);
+          const bool ok = isa ? row < args.M : row < args.N;
+          valid = (ok && k < args.K) ? int(min<int64_t>(CH, args.K - k)) : 0;
+          src = isa ? A + (valid ? row * args.lda + k : 0) : B + (valid ? row * args.ldb + k : 0);
+          const int rr = isa ? r : r - BM;
+          at[u] = (isa ? st * A_SLOT : B_RING + st * B_SLOT) + rr * 128 + ((c ^ ((rr >> 1) & 7)) << 4);
+        }
+        v[u] = load_chunk_or_zero(src, valid, whole);
       }
-      const int r = rem / 8, c = rem % 8;
-      const int64_t k = kt0 + st * BKS + c * CH;
-      const bool isa = r < BM;
-      const int64_t row = isa ? m0 + r : n0 + (r - BM);
-      const bool ok = isa ? row < args.M : row < args.N;
-      const int valid = (ok && k < args.K) ? int(min<int64_t>(CH, args.K - k)) : 0;
-      const T* base = isa ? A + (valid ? row * args.lda + k : 0) : B + (valid ? row * args.ldb + k : 0);
-      const uint4 v = load_chunk<false>(base, valid);
-      const int rr = isa ? r : r - BM;
-      *reinterpret_cast<uint4*>(smem_raw + (isa ? st * A_SLOT : B_RING + st * B_SLOT) + rr * 128 +
-                                ((c ^ ((rr >> 1) & 7)) << 4)) = v;
+#pragma unroll
+      for (int u = 0; u < Q; ++u) *reinterpret_cast<uint4*>(smem_raw + at[u]) = v[u];
     }
     __syncthreads();
     compute(0, true);
@@ -1486,8 +1515,10 @@ inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int
   if (requested >= 1) {
     s = requested;
   } else {
-    // 16-bit decode shapes take the streaming kernel, which needs no split
-    if (io_dtype != FXPR_DTYPE_F32 && stream_shape(M, N)) return 1;
+    // 16-bit decode shapes take the streaming kernel, which needs no split. (K
+    // that is no whole number of K-tiles: the skinny tile, split as any other;
+    // unsplit it ran 16 workgroups at N = 4096: M = 1, K = 10848 244 -> 27 us)
+    if (io_dtype != FXPR_DTYPE_F32 && stream_shape(M, N) && K % 128 == 0) return 1;
     // fp32 beyond M = 32 (K a multiple of a chunk: other rows cannot be
     // 16-byte aligned and take the register-staged tiles)
     if (io_dtype == FXPR_DTYPE_F32 && M > 32 && K % 4 == 0) return f32_plan(M, N, ktiles, 0).splits;
