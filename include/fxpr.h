@@ -257,7 +257,10 @@ int64_t fxpr_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k,
  * logit_softcap * log2(e) (0 = off); window_size 0 = off. num_kv_splits:
  * 0 = automatic (fxpr_attention_splits() reports the choice), >= 1 = that
  * many KV splits (a launch whose split partials would exceed 1 GiB runs
- * unsplit; the bits are the same). The launch needs a workspace of
+ * unsplit; the bits are the same). An automatic launch whose max_query_len
+ * allows requests of 48 query rows per kv head or more may split their keys,
+ * and the shorter requests' apart from them, whatever fxpr_attention_splits()
+ * reports; the workspace query covers it. The launch needs a workspace of
  * fxpr_attention_workspace_bytes() bytes when that is non-zero (no zeroing).
  * The output is bitwise independent of num_splits, of the batch the request
  * is in and of max_query_len.
