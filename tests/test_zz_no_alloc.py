@@ -147,3 +147,26 @@ def test_noalloc_first_call_under_capture_is_rejected():
     """)
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=240, cwd=root)
     assert "REJECTED" in res.stdout and "NOT" not in res.stdout, res.stdout + res.stderr[-2000:]
+
+
+def test_noalloc_long_requests_run_the_plain_split():
+    # a prompt chunk over a long context beside decode steps: the automatic
+    # split of long requests keeps records, this entry point runs the plain
+    # (unsplit) count, the same bits, without its scratch array
+    g = torch.Generator("cpu").manual_seed(6)
+    lens, news = [2600] + [3000 - 90 * i for i in range(20)], [120] + [1] * 20
+    kv = torch.randn(400, 2, 16, 8, 128, generator=g).to(torch.bfloat16).cuda()
+    bt = torch.stack([torch.randperm(400, generator=g)[:190] for _ in lens]).to(torch.int32).cuda()
+    q = torch.randn(sum(news), 32, 128, generator=g).to(torch.bfloat16).cuda()
+    qsl = torch.tensor([0] + news).cumsum(0).to(torch.int32).cuda()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    lib = _hip.load()
+    assert lib.fxpr_attention_workspace_bytes(21, 140, 32, 8, 128, 32, 0, 120, 190, 16) > 0
+    assert lib.fxpr_attention_splits(21, 8, 4, 120, 190, 16, 0) == 1
+    outs = []
+    for static in (False, True):
+        o = torch.zeros_like(q)
+        KA.unified_attention_fxp_run(q, kv, o, qsl, sl, bt, 120, None, True, None, 32, 16, 0.0, 0, 0,
+                                     static_scratch=static)
+        outs.append(o)
+    assert torch.equal(*outs)

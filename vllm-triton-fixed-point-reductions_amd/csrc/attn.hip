@@ -363,13 +363,18 @@ extern "C" int fxpr_unified_attention_noalloc(
                                           splits, max_query_len, max_blocks_per_seq, page_size);
   };
   int64_t need = ws_need(num_kv_splits);
-  if (need > kStaticScratchBytes && num_kv_splits == 0) {
-    // the records of an automatic split of long requests may not fit where
-    // the batch's plain split count does (often none): run that (same bits)
-    num_kv_splits = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
-                                max_blocks_per_seq, page_size, 0)
-                        .splits;
-    need = ws_need(num_kv_splits);
+  if (need > 0 && num_kv_splits == 0) {
+    // an automatic split of long requests apart from short ones needs records
+    // where the batch's plain split count (often none) needs fewer or none:
+    // this entry point runs the plain count (same bits), so that such a batch
+    // still needs no scratch array, nor its look-up outside graph capture
+    const int plain = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
+                                  max_blocks_per_seq, page_size, 0)
+                          .splits;
+    if (need > ws_need(plain)) {
+      num_kv_splits = plain;
+      need = ws_need(plain);
+    }
   }
   if (need > kStaticScratchBytes) return FXPR_E_WORKSPACE;
   void* ws = nullptr;
