@@ -260,8 +260,8 @@ int64_t fxpr_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k,
  * unsplit; the bits are the same). An automatic launch whose max_query_len
  * allows requests of 48 query rows per kv head or more may split their keys,
  * and the shorter requests' apart from them, whatever fxpr_attention_splits()
- * reports; the workspace query covers it. The launch needs a workspace of
- * fxpr_attention_workspace_bytes() bytes when that is non-zero (no zeroing).
+ * reports; fxpr_attention_plan() reports that choice. The launch needs a
+ * workspace of fxpr_attention_plan() bytes when that is non-zero (no zeroing).
  * The output is bitwise independent of num_splits, of the batch the request
  * is in and of max_query_len.
  * Replaces unified_attention_fxp_run + _attn_fused_kernel /
@@ -289,7 +289,7 @@ int fxpr_unified_attention(
 /*
  * fxpr_unified_attention without the workspace arguments: allocates nothing.
  * The split partials go to a static device array of FXPR_STATIC_SCRATCH_BYTES
- * per GPU; a launch whose fxpr_attention_workspace_bytes() exceeds that is
+ * per GPU; a launch whose fxpr_attention_plan() bytes exceed that is
  * rejected with FXPR_E_WORKSPACE before anything runs. The array's device
  * address is looked up at the first split call on each device, which must
  * not be under HIP graph capture (FXPR_E_CAPTURE; any eager call that splits
@@ -324,7 +324,21 @@ int fxpr_attention_splits(int num_requests, int num_kv_heads, int group,
 /* Workspace bytes fxpr_unified_attention needs for this launch (0 = none):
  * with more than one split, per (token, head) the chunk range and per
  * (token, head, chunk) the maximum, the integer denominator and the integer
- * weighted-V row. Replaces the per-call scratch of attention.py:839-851. */
+ * weighted-V row. stride_k_slot / stride_v_slot: the caches' key strides, as
+ * the launch gets them. plan: NULL or 4 ints that receive the kernels (0 / 1:
+ * every row in 16-row workgroups, key tiles by register loads / by LDS DMA;
+ * 2 / 3: requests of 48 query rows per kv head or more in 64-row workgroups),
+ * the key splits of those requests and of the shorter ones (equal for 0 to 2),
+ * and the tokens per request that have records (0: every token). Replaces the
+ * per-call scratch of attention.py:839-851. */
+int64_t fxpr_attention_plan(int io_dtype, int num_requests, int64_t num_tokens,
+                            int num_heads, int num_kv_heads, int head_dim,
+                            int page_size, int max_query_len,
+                            int max_blocks_per_seq, int64_t stride_k_slot,
+                            int64_t stride_v_slot, int int_bits,
+                            int num_kv_splits, int32_t* plan);
+
+/* The same without the input type and the cache's strides: enough for any. */
 int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_tokens,
                                        int num_heads, int num_kv_heads,
                                        int head_dim, int int_bits,

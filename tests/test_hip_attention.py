@@ -18,6 +18,7 @@ import pytest
 import torch
 
 import fxpr_vllm  # noqa: F401
+from fxpr_vllm import _hip
 from fxpr_vllm._kernels import attention as KA
 from oracle import attention as A
 from tests._util import IO_NAME, close_report, from_np, to_np
@@ -693,3 +694,20 @@ def test_prefill_softcap_extreme_scores(softcap):
         part = (q[lo:lo + m].contiguous(), kv, torch.tensor([0, m], dtype=torch.int32, device="cuda"),
                 torch.tensor([L - n + lo + m], dtype=torch.int32, device="cuda"), bt, m)
         assert torch.equal(_attend(part, 1, softcap=softcap), whole[lo:lo + m]), lo
+
+
+@pytest.mark.parametrize("dtype,ps", [(torch.float32, 16), (torch.bfloat16, 8)])
+def test_launches_without_records_need_no_workspace(dtype, ps):
+    # fp32 inputs and small pages run unsplit beside long requests, and take
+    # a call without a workspace (the 16-bit DMA kernels' split keeps records)
+    reqs = [(120, 2600)] + [(1, 3000 - 90 * i) for i in range(20)]
+    q, kv, qsl, sl, bt, max_q = _ragged(reqs, 32, 8, 128, ps, dtype, 6)
+    k, v, o = kv.select(1, 0), kv.select(1, 1), torch.zeros_like(q)
+    lib = _hip.load()
+    rc = lib.fxpr_unified_attention(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), _hip.DTYPE_CODE[dtype], qsl.data_ptr(), sl.data_ptr(),
+        bt.data_ptr(), None, len(reqs), q.shape[0], 32, 8, 128, ps, max_q, bt.shape[1], kv.shape[0], q.stride(0),
+        q.stride(1), *k.stride()[:3], *v.stride()[:3], o.stride(0), o.stride(1), bt.stride(0), 1,
+        128 ** -0.5 * 1.4426950408889634, 0.0, 0, 32, 16, 0, None, 0, _hip.stream_ptr(q.device))
+    assert rc == 0, _hip.error_string(rc)
+    assert torch.equal(o, _attend((q, kv, qsl, sl, bt, max_q), 3))

@@ -11,6 +11,8 @@ tests' part (tests/test_hip_attention.py, tests/test_hip_gemm.py).
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 
 from fxpr_vllm import _hip
@@ -78,6 +80,57 @@ def test_attention_policy_is_static(lib):
     # the same arguments always give the same count (graph capture bakes it in)
     first = [attn_splits(lib, b, 8, 4, 1, 8192) for b in (1, 8, 64, 300)]
     assert first == [attn_splits(lib, b, 8, 4, 1, 8192) for b in (1, 8, 64, 300)]
+
+
+# kernels of fxpr_attention_plan: 16-row workgroups by register loads / LDS DMA,
+# long requests apart by register loads / LDS DMA
+ROWS16, ROWS16_DMA, LONG, LONG_DMA = range(4)
+
+
+def attn_plan(lib, requests, tokens, max_q, keys, dt=1, heads=32, kv_heads=8, d=128, page=16, bits=32, stride=None,
+              requested=0):
+    """(kernels, splits of long requests, of short ones, record rows per request, workspace bytes)"""
+    plan = (ctypes.c_int32 * 4)()
+    stride = kv_heads * d if stride is None else stride
+    n = lib.fxpr_attention_plan(dt, requests, tokens, heads, kv_heads, d, page, max_q, -(-keys // page), stride, stride,
+                                bits, requested, plan)
+    return (*plan, n)
+
+
+def record_bytes(rows, keys, heads=32, d=128, acc=4):
+    """Split records of `rows` workspace rows over a table of `keys` (heads and d as attn_plan's)."""
+    slots = -(-keys // 512)
+    up = lambda n: -(-n // 256) * 256  # noqa: E731
+    return sum(map(up, (rows * heads * 8, rows * heads * slots * 4, rows * heads * slots * acc,
+                        rows * heads * slots * d * acc)))
+
+
+def test_attention_workspace_is_the_running_launchs(lib):
+    # a 120-token chunk beside 20 decode steps, contexts up to 3040 keys: the
+    # DMA kernels keep records of the split prefill rows; launches they do not
+    # take (fp32 inputs, pages of 8 or 48 keys, a key stride of 2^20 elements,
+    # 64-bit sums) run unsplit without any
+    mixed = dict(requests=21, tokens=140, max_q=120, keys=3040)
+    want = record_bytes(140, 3040)
+    assert attn_plan(lib, **mixed) == (LONG_DMA, 6, 6, 0, want)
+    assert attn_plan(lib, dt=F16, **mixed)[-1] == want
+    assert attn_plan(lib, dt=F32, **mixed) == (ROWS16, 1, 1, 0, 0)
+    assert attn_plan(lib, page=8, **mixed) == (LONG, 1, 1, 0, 0)
+    assert attn_plan(lib, page=48, **mixed) == (LONG, 1, 1, 0, 0)
+    assert attn_plan(lib, stride=1 << 20, **mixed) == (LONG, 1, 1, 0, 0)
+    assert attn_plan(lib, d=96, **mixed) == (LONG, 1, 1, 0, 0)
+    assert attn_plan(lib, d=256, **mixed) == (ROWS16, 1, 1, 0, 0)
+    assert attn_plan(lib, bits=64, **mixed) == (ROWS16_DMA, 1, 1, 0, 0)
+    # the query without type and strides covers any of them
+    assert lib.fxpr_attention_workspace_bytes(21, 140, 32, 8, 128, 32, 0, 120, 190, 16) == want
+    assert lib.fxpr_attention_workspace_bytes(21, 140, 32, 8, 128, 32, 0, 120, 380, 8) == 0
+    # a decode batch: the plain policy's splits, with either kernel
+    decode = dict(requests=64, tokens=64, max_q=1, keys=8192)
+    assert attn_plan(lib, **decode) == (ROWS16_DMA, 16, 16, 0, record_bytes(64, 8192))
+    assert attn_plan(lib, dt=F32, **decode) == (ROWS16, 16, 16, 0, record_bytes(64, 8192))
+    # one plan's records only: 128 tokens at 16 splits by register loads
+    assert attn_plan(lib, 1, 128, 128, 8192, dt=F32) == (ROWS16, 16, 16, 0, record_bytes(128, 8192))
+    assert attn_plan(lib, 0, 128, 128, 8192) == (0, 0, 0, 0, 0)
 
 
 BF16, F16, F32 = 1, 0, 2

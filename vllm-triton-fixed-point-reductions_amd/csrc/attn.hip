@@ -101,9 +101,8 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
 }
 
 // Launches that may hold requests of kPrefillRows rows or more, where the DMA
-// kernels can take them (16- / 32-bit sums; the rest of their conditions is
-// known at the launch, which otherwise runs launch_plan's): the two kinds of
-// requests are split apart from each other.
+// kernels can take them (Route::kLongDma): the two kinds of requests are split
+// apart from each other.
 //   * Prefill workgroups (64 rows each): about tokens x heads / 64 of them.
 //     Below 512 (two per CU) their keys are split until there are about
 //     kLongWgs; a chunk is the least a split can hold.
@@ -124,9 +123,6 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
                      int max_query_len, int max_blocks, int page_size, int requested) {
   LongLayout l;
   const int group = num_heads / num_kv_heads;
-  const int64_t max_rows = int64_t(max_query_len > 1 ? max_query_len : 1) * group;
-  if (int_bits == 64 || max_rows < kPrefillRows || (head_dim != 64 && head_dim != 128)) return l;
-  l.plan.use = true;
   const int64_t slots = chunk_slots(max_blocks, page_size);
   const int64_t tiles = cdiv(int64_t(max_blocks > 0 ? max_blocks : 1) * page_size, TILE);
   int64_t ps = 1, ds = 1;
@@ -166,6 +162,46 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
   l.plan.chunks_per_split = requested >= 1 || ds <= 1 ? 0 : int(cdiv(slots, ds));
   return l;
 }
+
+// What a launch runs: its kernels, its splits and the records they need.
+struct LaunchPlan {
+  LongPlan lp;        // (splits: kLongDma only)
+  SplitPlan sp{1, 0};  // the other routes' splits
+  WsLayout ws;
+};
+
+LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, int num_heads, int num_kv_heads,
+                          int head_dim, int page_size, int max_query_len, int max_blocks, int64_t stride_k_slot,
+                          int64_t stride_v_slot, int int_bits, int requested) {
+  LaunchPlan p;
+  const bool dma = dma_takes(io_dtype, head_dim, page_size, stride_k_slot, stride_v_slot);
+  const int group = num_heads / num_kv_heads;
+  const int64_t max_rows = int64_t(max_query_len > 1 ? max_query_len : 1) * group;
+  // the 64-row workgroups: 16-bit inputs, 16- / 32-bit sums
+  const bool wide = io_dtype != FXPR_DTYPE_F32 && int_bits != 64 && head_dim <= 128;
+  if (wide && dma && max_rows >= kPrefillRows) {
+    const LongLayout l = long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
+                                   max_blocks, page_size, requested);
+    p.lp = l.plan;
+    p.lp.route = Route::kLongDma;
+    p.ws = l.ws;
+    return p;
+  }
+  p.sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len, max_blocks,
+                     page_size, requested);
+  p.ws = ws_layout(num_tokens, num_heads, head_dim, int_bits, p.sp.splits > 1, chunk_slots(max_blocks, page_size));
+  if (wide && p.sp.splits <= 1 && cdiv(max_rows, QROWS) * QROWS >= kPrefillRows)
+    p.lp.route = Route::kLong;
+  else
+    p.lp.route = dma ? Route::kRows16Dma : Route::kRows16;
+  return p;
+}
+
+bool plan_args_ok(int num_requests, int64_t num_tokens, int num_heads, int num_kv_heads, int head_dim, int page_size,
+                  int max_blocks, int num_kv_splits) {
+  return num_requests > 0 && num_tokens > 0 && num_heads > 0 && num_kv_heads > 0 && head_dim > 0 && max_blocks > 0 &&
+         page_size > 0 && num_heads % num_kv_heads == 0 && num_kv_splits >= 0;
+}
 }  // namespace
 
 extern "C" int fxpr_attention_splits(int num_requests, int num_kv_heads, int group, int max_query_len,
@@ -179,17 +215,33 @@ extern "C" int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_
                                                   int num_kv_heads, int head_dim, int int_bits,
                                                   int num_kv_splits, int max_query_len,
                                                   int max_blocks_per_seq, int page_size) {
-  if (num_requests <= 0 || num_tokens <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 ||
-      max_blocks_per_seq <= 0 || page_size <= 0 || num_heads % num_kv_heads != 0 || num_kv_splits < 0)
+  // whatever the inputs' type and the cache's strides: with the DMA kernels or without
+  auto need = [&](int io_dtype) {
+    return fxpr_attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
+                               max_query_len, max_blocks_per_seq, head_dim, head_dim, int_bits, num_kv_splits, nullptr);
+  };
+  return std::max(need(FXPR_DTYPE_BF16), need(FXPR_DTYPE_F32));
+}
+
+extern "C" int64_t fxpr_attention_plan(int io_dtype, int num_requests, int64_t num_tokens, int num_heads,
+                                       int num_kv_heads, int head_dim, int page_size, int max_query_len,
+                                       int max_blocks_per_seq, int64_t stride_k_slot, int64_t stride_v_slot,
+                                       int int_bits, int num_kv_splits, int32_t* plan) {
+  if (plan) std::fill(plan, plan + 4, 0);
+  if (!plan_args_ok(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size, max_blocks_per_seq,
+                    num_kv_splits))
     return 0;
-  const SplitPlan sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
-                                   max_query_len, max_blocks_per_seq, page_size, num_kv_splits);
-  const int64_t plain = ws_layout(num_tokens, num_heads, head_dim, int_bits, sp.splits > 1,
-                                  chunk_slots(max_blocks_per_seq, page_size))
-                            .total;
-  return std::max(plain, long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
-                                   max_blocks_per_seq, page_size, num_kv_splits)
-                             .ws.total);
+  const LaunchPlan p = attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
+                                      max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits,
+                                      num_kv_splits);
+  if (plan) {
+    const bool apart = p.lp.route == Route::kLongDma;
+    plan[0] = int(p.lp.route);
+    plan[1] = apart ? p.lp.pq_splits : p.sp.splits;
+    plan[2] = apart ? p.lp.splits : p.sp.splits;
+    plan[3] = p.lp.tok_cap;
+  }
+  return p.ws.total;
 }
 
 extern "C" int fxpr_unified_attention(
@@ -208,9 +260,6 @@ extern "C" int fxpr_unified_attention(
     return FXPR_E_SHAPE;
   if (num_requests == 0 || num_tokens == 0) return FXPR_OK;
   if (max_blocks_per_seq <= 0 || num_blocks <= 0) return FXPR_E_SHAPE;
-  const SplitPlan sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
-                                   max_query_len, max_blocks_per_seq, page_size, num_kv_splits);
-  const int num_splits = sp.splits;
   if (!q || !k_cache || !v_cache || !o || !query_start_loc || !seq_lens || !block_table) return FXPR_E_ARG;
   if (io_dtype != FXPR_DTYPE_BF16 && io_dtype != FXPR_DTYPE_F16 && io_dtype != FXPR_DTYPE_F32)
     return FXPR_E_DTYPE;
@@ -227,11 +276,10 @@ extern "C" int fxpr_unified_attention(
     if (sv < 0 || sv > int64_t(0xffffffff)) return FXPR_E_ARG;
   const int64_t slots = chunk_slots(max_blocks_per_seq, page_size);
   if (slots > 0x7fffffff) return FXPR_E_SHAPE;
-  const WsLayout wl = ws_layout(num_tokens, num_heads, head_dim, int_bits, num_splits > 1, slots);
-  LongLayout ll = long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
-                            max_blocks_per_seq, page_size, num_kv_splits);
-  const int64_t need = std::max(wl.total, ll.ws.total);
-  if (need > 0 && (!workspace || workspace_bytes < need)) return FXPR_E_WORKSPACE;
+  LaunchPlan plan = attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
+                                   max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits,
+                                   num_kv_splits);
+  if (plan.ws.total > 0 && (!workspace || workspace_bytes < plan.ws.total)) return FXPR_E_WORKSPACE;
 
   AttnArgs a{};
   a.q = q;
@@ -243,15 +291,11 @@ extern "C" int fxpr_unified_attention(
   a.bt = block_table;
   a.alibi = alibi_slopes;
   char* base = static_cast<char*>(workspace);
-  if (wl.crange >= 0) a.crange = reinterpret_cast<int*>(base + wl.crange);
-  if (wl.pmax >= 0) a.pmax = reinterpret_cast<float*>(base + wl.pmax);
-  if (wl.den >= 0) a.den_ws = base + wl.den;
-  if (wl.wv >= 0) a.wv_ws = base + wl.wv;
-  if (ll.ws.crange >= 0) {
-    ll.plan.crange = reinterpret_cast<int*>(base + ll.ws.crange);
-    ll.plan.pmax = reinterpret_cast<float*>(base + ll.ws.pmax);
-    ll.plan.den_ws = base + ll.ws.den;
-    ll.plan.wv_ws = base + ll.ws.wv;
+  if (plan.ws.total > 0) {
+    a.crange = reinterpret_cast<int*>(base + plan.ws.crange);
+    a.pmax = reinterpret_cast<float*>(base + plan.ws.pmax);
+    a.den_ws = base + plan.ws.den;
+    a.wv_ws = base + plan.ws.wv;
   }
   a.chunk_slots = int(slots);
   a.sq_t = stride_q_token;
@@ -270,8 +314,8 @@ extern "C" int fxpr_unified_attention(
   a.group = num_heads / num_kv_heads;
   a.head_dim = head_dim;
   a.page_size = page_size;
-  a.num_splits = num_splits;
-  a.chunks_per_split = sp.chunks_per_split;
+  a.num_splits = plan.sp.splits;
+  a.chunks_per_split = plan.sp.chunks_per_split;
   a.window = window_size > 0 ? window_size : 0;
   a.causal = is_causal ? 1 : 0;
   a.max_blocks = max_blocks_per_seq;
@@ -289,9 +333,9 @@ extern "C" int fxpr_unified_attention(
   const int max_qtiles = int(cdiv(int64_t(max_query_len > 1 ? max_query_len : 1) * a.group, QROWS));
   hipStream_t st = as_stream(stream);
   switch (io_dtype) {
-    case FXPR_DTYPE_BF16: return run_attn_bf16(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
-    case FXPR_DTYPE_F16: return run_attn_f16(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
-    default: return run_attn_f32(a, ll.plan, int_bits, num_requests, max_qtiles, num_tokens, st);
+    case FXPR_DTYPE_BF16: return run_attn_bf16(a, plan.lp, int_bits, num_requests, max_qtiles, num_tokens, st);
+    case FXPR_DTYPE_F16: return run_attn_f16(a, plan.lp, int_bits, num_requests, max_qtiles, num_tokens, st);
+    default: return run_attn_f32(a, plan.lp, int_bits, num_requests, max_qtiles, num_tokens, st);
   }
 }
 
@@ -359,8 +403,9 @@ extern "C" int fxpr_unified_attention_noalloc(
     int is_causal, float softmax_scale_log2, float softcap_log2, int window_size, int int_bits,
     int frac_bits, int num_kv_splits, void* stream) {
   auto ws_need = [&](int splits) {
-    return fxpr_attention_workspace_bytes(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
-                                          splits, max_query_len, max_blocks_per_seq, page_size);
+    return fxpr_attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
+                               max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits, splits,
+                               nullptr);
   };
   int64_t need = ws_need(num_kv_splits);
   if (need > 0 && num_kv_splits == 0) {

@@ -83,19 +83,23 @@ struct AttnArgs {
   float scale_log2, softcap_log2, fxp_scale, fxp_inv;
 };
 
-// Host plan of a launch that holds requests of kPrefillRows rows or more, for
-// shapes the DMA kernels take: key splits of the prefill workgroups and of the
-// short requests' 16-row ones, and the workspace records of the split rows.
+// The kernels that serve a launch.
+enum class Route : int {
+  kRows16 = 0,     // every row in 16-row workgroups, key tiles by register loads (attn_kernel)
+  kRows16Dma = 1,  // the same by LDS DMA (attn_dma_kernel)
+  kLong = 2,       // long requests in 64-row workgroups, unsplit, by register loads
+  kLongDma = 3,    // long requests in 64-row workgroups by LDS DMA, split as LongPlan says (launch_long)
+};
+
+// Host plan of a launch: its kernels, and for Route::kLongDma (requests of
+// kPrefillRows rows or more) the key splits of the prefill workgroups and of
+// the short requests' 16-row ones, and the workspace records of the split rows.
 struct LongPlan {
-  bool use = false;
+  Route route = Route::kRows16;
   int pq_splits = 1;       // prefill workgroups
   int splits = 1;          // short requests
   int chunks_per_split = 0;
   int tok_cap = 0;         // AttnArgs::tok_cap
-  float* pmax = nullptr;
-  void* den_ws = nullptr;
-  void* wv_ws = nullptr;
-  int* crange = nullptr;
 };
 
 template <int DT> struct Traits;
@@ -2490,19 +2494,16 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a, int64_t n
   }
 }
 
-// attn_dma_kernel serves a launch when each wave's 16 key rows of a tile lie
+// The DMA kernels serve a launch when each wave's 16 key rows of a tile lie
 // in one page and the rows are exactly DMAX wide.
-template <int DT, int DMAX> bool dma_ok(const AttnArgs& a) {
-  if constexpr (DT == FXPR_DTYPE_F32 || (DMAX != 64 && DMAX != 128)) {
-    return false;
-  } else {
-    // pages of 16, 32, ... keys; key strides below 2^20 elements (the prefill
-    // kernel's 32-bit lane offsets span 16 of them)
-    // and a page's K and V rows below 2^31 bytes (the prefill kernel's scalar
-    // offset to a wave's first row)
-    return a.head_dim == DMAX && a.ps_shift >= 4 && a.sk_s < (int64_t(1) << 20) && a.sv_s < (int64_t(1) << 20) &&
-           a.ps_shift < 31 && ((a.sk_s > a.sv_s ? a.sk_s : a.sv_s) << a.ps_shift) < (int64_t(1) << 30);
-  }
+inline bool dma_takes(int io_dtype, int head_dim, int page_size, int64_t sk_s, int64_t sv_s) {
+  if (io_dtype == FXPR_DTYPE_F32 || (head_dim != 64 && head_dim != 128)) return false;
+  // pages of 16, 32, ... keys; key strides below 2^20 elements (the prefill
+  // kernel's 32-bit lane offsets span 16 of them)
+  // and a page's K and V rows below 2^31 bytes (the prefill kernel's scalar
+  // offset to a wave's first row)
+  return page_size >= 16 && (page_size & (page_size - 1)) == 0 && sk_s < (int64_t(1) << 20) &&
+         sv_s < (int64_t(1) << 20) && std::max(sk_s, sv_s) * page_size < (int64_t(1) << 30);
 }
 
 template <int DT, int BITS, int DMAX, bool SPLIT, bool CAP = false>
@@ -2591,10 +2592,6 @@ int launch_long(AttnArgs a, const LongPlan& lp, int num_requests, int max_qtiles
   a.num_splits = lp.splits;
   a.chunks_per_split = lp.chunks_per_split;
   a.tok_cap = lp.tok_cap;
-  a.pmax = lp.pmax;
-  a.den_ws = lp.den_ws;
-  a.wv_ws = lp.wv_ws;
-  a.crange = lp.crange;
   const int64_t ptiles = cdiv(int64_t(max_qtiles) * QROWS, PQROWS);
   // a flat grid over the tokens where requests x the longest one's tiles
   // would be mostly empty (continuous batching: one prompt chunk, many
@@ -2634,10 +2631,11 @@ template <int DT, int BITS, int DMAX>
 int launch_attn(const AttnArgs& a, const LongPlan& lp, int num_requests, int max_qtiles, int64_t num_tokens,
                 hipStream_t st) {
   dim3 grid(unsigned(num_requests * a.num_kv_heads), unsigned(max_qtiles), unsigned(a.num_splits));
-  const bool dma = dma_ok<DT, DMAX>(a);
+  const bool dma = lp.route == Route::kRows16Dma;
   if constexpr (DT != FXPR_DTYPE_F32 && BITS <= 32 && DMAX <= 128) {
-    if (lp.use && dma) return launch_long<DT, BITS, DMAX>(a, lp, num_requests, max_qtiles, num_tokens, st);
-    if (a.num_splits <= 1 && int64_t(max_qtiles) * QROWS >= kPrefillRows) {
+    if (lp.route == Route::kLongDma)
+      return launch_long<DT, BITS, DMAX>(a, lp, num_requests, max_qtiles, num_tokens, st);
+    if (lp.route == Route::kLong) {
       // as launch_long, on the register-load kernels
       AttnArgs b = a;
       b.pq_rows = kPrefillRows;

@@ -288,9 +288,9 @@ void unified_attention(const Tensor& q_in, const Tensor& kv_cache, Tensor& o, co
   const float softcap_log2 = logit_softcap > 0.0 ? float(logit_softcap * kRcpLn2) : 0.0f;
   const int64_t max_blocks = bt.size(1);
   const int64_t window = std::max<int64_t>(0, window_size);
-  const int64_t n = fxpr_attention_workspace_bytes(int(num_requests), num_tokens, int(num_heads), int(num_kv_heads),
-                                                   int(head_dim), int(int_bits), int(num_kv_splits), int(max_query_len),
-                                                   int(max_blocks), int(page_size));
+  const int64_t n = fxpr_attention_plan(code_of(t), int(num_requests), num_tokens, int(num_heads), int(num_kv_heads),
+                                        int(head_dim), int(page_size), int(max_query_len), int(max_blocks),
+                                        k_cache.stride(1), v_cache.stride(1), int(int_bits), int(num_kv_splits), nullptr);
   Tensor ws = n > 0 ? bytes(n, q) : Tensor();
   check_rc(fxpr_unified_attention(
                q.const_data_ptr(), k_cache.const_data_ptr(), v_cache.const_data_ptr(), out.mutable_data_ptr(), code_of(t),

@@ -112,9 +112,10 @@ def unified_attention_fxp_run(
     if static_scratch:
         _hip.call("fxpr_unified_attention_noalloc", *common, _hip.stream_ptr(q.device))
     else:
-        ws_bytes = _hip.load().fxpr_attention_workspace_bytes(
-            num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int(fxp_int_bits),
-            int(num_kv_splits), int(max_query_len), max_blocks, page_size)
+        ws_bytes = _hip.load().fxpr_attention_plan(
+            _hip.DTYPE_CODE[q.dtype], num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
+            int(max_query_len), max_blocks, k_cache.stride(1), v_cache.stride(1), int(fxp_int_bits),
+            int(num_kv_splits), None)
         ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes > 0 else None
         _hip.call("fxpr_unified_attention", *common, _hip.ptr(ws), ws_bytes, _hip.stream_ptr(q.device))
     if out is not o:
