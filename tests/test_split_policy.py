@@ -133,6 +133,24 @@ def test_attention_workspace_is_the_running_launchs(lib):
     assert attn_plan(lib, 0, 128, 128, 8192) == (0, 0, 0, 0, 0)
 
 
+def test_attention_kernels_by_the_longest_requests_rows(lib):
+    # 64-row workgroups from 48 rows per kv head on; the 33 to 47 rows that fill
+    # three 16-row tiles as well stay on the 16-row kernels: by LDS DMA at
+    # head_dim 128 (or when split), by register loads at 64
+    for heads, kv_heads, below, first in ((32, 8, (9, 10, 11), 12), (16, 16, (33, 40, 47), 48), (24, 8, (11, 15), 16),
+                                          (28, 4, (5, 6), 7)):
+        for d in (64, 128):
+            shape = dict(heads=heads, kv_heads=kv_heads, d=d, keys=2048)
+            for n in (1, 32 * kv_heads // heads, *below):
+                want = ROWS16 if d == 64 and n in below else ROWS16_DMA
+                assert attn_plan(lib, 8, 8 * n, n, **shape)[0] == want, (heads, d, n)
+                assert attn_plan(lib, 8, 8 * n, n, requested=2, **shape)[0] == ROWS16_DMA, (heads, d, n)
+                assert attn_plan(lib, 8, 8 * n, n, bits=64, **shape)[0] == ROWS16_DMA, (heads, d, n)
+                assert attn_plan(lib, 8, 8 * n, n, page=8, **shape)[0] == ROWS16, (heads, d, n)
+            assert attn_plan(lib, 8, 8 * first, first, **shape)[0] == LONG_DMA, heads
+            assert attn_plan(lib, 8, 8 * first, first, page=8, **shape)[0] == LONG, heads
+
+
 BF16, F16, F32 = 1, 0, 2
 
 

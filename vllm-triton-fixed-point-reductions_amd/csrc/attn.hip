@@ -177,9 +177,11 @@ LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, in
   const bool dma = dma_takes(io_dtype, head_dim, page_size, stride_k_slot, stride_v_slot);
   const int group = num_heads / num_kv_heads;
   const int64_t max_rows = int64_t(max_query_len > 1 ? max_query_len : 1) * group;
-  // the 64-row workgroups: 16-bit inputs, 16- / 32-bit sums
-  const bool wide = io_dtype != FXPR_DTYPE_F32 && int_bits != 64 && head_dim <= 128;
-  if (wide && dma && max_rows >= kPrefillRows) {
+  // 64-row workgroups serve 16-bit inputs with 16- / 32-bit sums, and only
+  // requests of kPrefillRows rows or more
+  const bool narrow_sums = io_dtype != FXPR_DTYPE_F32 && int_bits != 64;
+  const bool wide = narrow_sums && head_dim <= 128 && max_rows >= kPrefillRows;
+  if (wide && dma) {
     const LongLayout l = long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
                                    max_blocks, page_size, requested);
     p.lp = l.plan;
@@ -190,10 +192,19 @@ LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, in
   p.sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len, max_blocks,
                      page_size, requested);
   p.ws = ws_layout(num_tokens, num_heads, head_dim, int_bits, p.sp.splits > 1, chunk_slots(max_blocks, page_size));
-  if (wide && p.sp.splits <= 1 && cdiv(max_rows, QROWS) * QROWS >= kPrefillRows)
+  // Just short of that, three 16-row tiles a request (33 to 47 rows), the DMA
+  // kernel is the faster one at head_dim 128 (us, register loads / DMA: 1 x 10
+  // tokens of group 4 over 1000 keys 30 / 27, 64 x 10 over 2000 296 / 262, 90
+  // decode steps up to 4000 keys beside 2 x 10 tokens 223 / 213; 64 x 10 over
+  // 500 69 / 76), register loads at 64 (4 x 40 tokens of group 1 over 500 keys
+  // 13.3 / 15.9, 64 x 40 over 1000 143 / 166, 90 decode steps up to 2000 beside
+  // 2 x 40 123 / 135; 64 x 40 over 2000 318 / 296).
+  const bool three_tiles = max_rows > 2 * QROWS && max_rows < kPrefillRows;
+  const bool by_registers = narrow_sums && head_dim == 64 && three_tiles && p.sp.splits <= 1;
+  if (wide && p.sp.splits <= 1)
     p.lp.route = Route::kLong;
   else
-    p.lp.route = dma ? Route::kRows16Dma : Route::kRows16;
+    p.lp.route = dma && !by_registers ? Route::kRows16Dma : Route::kRows16;
   return p;
 }
 
