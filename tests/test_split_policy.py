@@ -133,6 +133,17 @@ def test_attention_workspace_is_the_running_launchs(lib):
     assert attn_plan(lib, 0, 128, 128, 8192) == (0, 0, 0, 0, 0)
 
 
+def test_attention_batches_of_equal_long_requests_keep_no_short_records(lib):
+    # nothing for short requests where every request has the longest one's
+    # tokens; the prefill rows' own splits are not affected
+    assert attn_plan(lib, 4, 4 * 2048, 2048, 131072) == (LONG_DMA, 1, 1, 0, 0)
+    assert attn_plan(lib, 1, 512, 512, 131072) == (LONG_DMA, 1, 1, 0, 0)     # records of 512 tokens: 2 GiB
+    assert attn_plan(lib, 1, 64, 64, 32768) == (LONG_DMA, 64, 1, 0, record_bytes(64, 32768))
+    # one token less (some request is shorter), and one more (padding)
+    for tokens in (4 * 2048 - 1, 4 * 2048 + 1):
+        assert attn_plan(lib, 4, tokens, 2048, 131072) == (LONG_DMA, 1, 64, 11, record_bytes(4 * 11, 131072))
+
+
 def test_attention_kernels_by_the_longest_requests_rows(lib):
     # 64-row workgroups from 48 rows per kv head on; the 33 to 47 rows that fill
     # three 16-row tiles as well stay on the 16-row kernels: by LDS DMA at
