@@ -711,3 +711,14 @@ def test_launches_without_records_need_no_workspace(dtype, ps):
         128 ** -0.5 * 1.4426950408889634, 0.0, 0, 32, 16, 0, None, 0, _hip.stream_ptr(q.device))
     assert rc == 0, _hip.error_string(rc)
     assert torch.equal(o, _attend((q, kv, qsl, sl, bt, max_q), 3))
+
+
+@pytest.mark.parametrize("keys,new", [(131072, 128), (131072, 120), (65536, 256)])
+def test_prompt_chunk_over_a_wide_block_table(keys, new):
+    # around the record caps of the automatic split (128 x 131072: 520 MiB, split;
+    # 120 x 131072: just below 512 MiB, split; 256 x 65536: unsplit), the bits
+    # of the unsplit launch over a table that just holds the context
+    q, kv, qsl, sl, bt, max_q = _ragged([(new, 6000 + new)], 32, 8, 128, 16, torch.bfloat16, new)
+    wide = torch.zeros(1, keys // 16, dtype=torch.int32, device="cuda")
+    wide[:, :bt.shape[1]] = bt
+    assert torch.equal(_attend((q, kv, qsl, sl, wide, max_q), 0), _attend((q, kv, qsl, sl, bt, max_q), 1))

@@ -133,6 +133,35 @@ def test_attention_workspace_is_the_running_launchs(lib):
     assert attn_plan(lib, 0, 128, 128, 8192) == (0, 0, 0, 0, 0)
 
 
+def test_attention_long_requests_over_wide_tables_stay_split(lib):
+    # 512 MiB of records, 1 GiB with fewer than 128 prefill workgroups
+    half, full = 1 << 29, 1 << 30
+    for tokens, keys, splits in ((128, 131072, 32), (130, 131072, 32), (250, 131072, 17)):
+        n = record_bytes(tokens, keys)
+        assert half < n <= full
+        assert attn_plan(lib, 1, tokens, tokens, keys) == (LONG_DMA, splits, 1, 0, n), tokens
+        # (the register-load kernels: as many records, 64 splits)
+        assert attn_plan(lib, 1, tokens, tokens, keys, dt=F32) == (ROWS16, 64, 64, 0, n), tokens
+    assert attn_plan(lib, 1, 64, 64, 131072)[1] == 64                          # 260 MiB
+    for tokens, keys in ((256, 65536), (512, 32768)):
+        assert half < record_bytes(tokens, keys) <= full
+        assert attn_plan(lib, 1, tokens, tokens, keys) == (LONG_DMA, 1, 1, 0, 0), tokens
+    # past 1 GiB nothing of it is split
+    assert record_bytes(254, 262144) > full
+    assert attn_plan(lib, 1, 254, 254, 262144) == (LONG_DMA, 1, 1, 0, 0)
+    assert attn_plan(lib, 1, 256, 256, 131072) == (LONG_DMA, 1, 1, 0, 0)
+    assert attn_plan(lib, 1, 256, 256, 131072, dt=F32) == (ROWS16, 1, 1, 0, 0)
+    # and only where the 16-row kernels would split the batch as well
+    assert half < record_bytes(130, 131072) <= full
+    assert attn_plan(lib, 80, 130, 12, 131072)[1:] == (32, 64, 0, record_bytes(130, 131072))
+    assert attn_plan(lib, 90, 130, 12, 131072)[1:] == (1, 1, 0, 0)
+    # a chunk beside 31 decode steps; above the cap the decode steps keep
+    # records of their own tokens only
+    assert attn_plan(lib, 32, 543, 512, 28672) == (LONG_DMA, 8, 56, 0, record_bytes(543, 28672))
+    assert half < record_bytes(543, 30720) <= full
+    assert attn_plan(lib, 32, 543, 512, 30720) == (LONG_DMA, 1, 60, 11, record_bytes(32 * 11, 30720))
+
+
 def test_attention_batches_of_equal_long_requests_keep_no_short_records(lib):
     # nothing for short requests where every request has the longest one's
     # tokens; the prefill rows' own splits are not affected

@@ -113,8 +113,14 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
 //     no request, 179 MiB of records and a combine launch, 366 us; 340 without).
 // Explicit requests split both that many times. Records need a workspace: per
 // token when the prefill rows are split, else only for the short requests'
-// tokens; above kLongWsMax (explicit: kSplitWsMax) the launch runs unsplit.
-constexpr int64_t kFullWgs = 512, kLongWgs = 2048;
+// tokens. Above kLongWsMax the launch runs unsplit; above kSplitWsMax where the
+// split is explicit, or where there are so few prefill workgroups (kFewWgs) that
+// they lose to the 16-row kernels' split, which holds as many records (one
+// request, 32/8 heads of 128, over 30000 cached keys: 128 tokens, table of
+// 131072 keys 885 us unsplit, 462 split by 16 rows, 197 split here; 256 at 65536
+// 887 and 921. The wider cap at 256 and 512 tokens too would take 512 at 32768
+// from 897 to 697, but 512 without cached keys from 22 to 36).
+constexpr int64_t kFullWgs = 512, kLongWgs = 2048, kFewWgs = 128;
 constexpr int64_t kLongWsMax = int64_t(1) << 29;
 
 struct LongLayout {
@@ -128,11 +134,11 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
   const int group = num_heads / num_kv_heads;
   const int64_t slots = chunk_slots(max_blocks, page_size);
   const int64_t tiles = cdiv(int64_t(max_blocks > 0 ? max_blocks : 1) * page_size, TILE);
+  const int64_t wgs = std::max<int64_t>(cdiv(num_tokens * num_heads, PQROWS), 1);
   int64_t ps = 1, ds = 1;
   if (requested >= 1) {
     ps = ds = std::min<int64_t>({int64_t(requested), std::max<int64_t>(slots, 1), kMaxGridZ});
   } else {
-    const int64_t wgs = std::max<int64_t>(cdiv(num_tokens * num_heads, PQROWS), 1);
     if (wgs < kFullWgs && tiles > 32) ps = std::min<int64_t>(cdiv(kLongWgs, wgs), slots);
     const bool all_long = num_tokens == int64_t(num_requests) * max_query_len;
     if (tiles > 32 && int64_t(num_requests) * num_kv_heads <= 8 * 256 && !all_long)
@@ -140,9 +146,12 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
   }
   auto layout = [&](int64_t rows) { return ws_layout(rows, num_heads, head_dim, int_bits, true, slots); };
   const int64_t most = requested >= 1 ? kSplitWsMax : kLongWsMax;
+  const bool few = wgs < kFewWgs && launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits,
+                                                max_query_len, max_blocks, page_size, 0)
+                                            .splits > 1;
   if (ps > 1) {
     l.ws = layout(num_tokens);
-    if (l.ws.total > most) {
+    if (l.ws.total > (few ? kSplitWsMax : most)) {
       ps = 1;
       if (requested >= 1) ds = 1;
     }
