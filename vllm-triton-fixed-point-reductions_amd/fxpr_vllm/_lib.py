@@ -15,6 +15,8 @@ reference impls (_lib.py:36-129).
 
 from __future__ import annotations
 
+import logging
+
 import torch
 
 from . import _hip
@@ -24,6 +26,8 @@ from ._kernels import casts as _casts
 from ._kernels import gemm as _gemm
 from ._kernels import rows as _rows
 from ._kernels import sampling as _sampling
+
+logger = logging.getLogger("fxpr_vllm")
 
 _lib = torch.library.Library("fxpr", "DEF")
 
@@ -185,16 +189,25 @@ def _log_softmax_fxp_shard_finish_cuda(x, row_max, row_sum, fxp_frac_bits, out_d
 # The launchers of the hot ops are native (csrc/torch_ops.cpp, beside the
 # kernel library): they register themselves for the "CUDA" key when loaded. The
 # Python launchers below serve the remaining ops, and every op where the native
-# library has not been built (they raise without the kernel library).
+# ones are not built or do not load (a library that does not load has registered
+# nothing): the same kernels with more host time per call. Without the kernel
+# library the import still works and every op raises.
 _NATIVE_PATH = _hip.LIB_PATH.with_name("libfxpr_torch.so")
-_NATIVE = _NATIVE_PATH.exists()
-if _NATIVE:
+
+
+def _load_native() -> bool:
+    if not (_NATIVE_PATH.exists() and _hip.LIB_PATH.exists()):
+        return False
     try:
         torch.ops.load_library(str(_NATIVE_PATH))
     except OSError as e:
-        raise RuntimeError(
-            f"fxpr: {_NATIVE_PATH} does not load with this torch ({torch.__version__}): {e}; rebuild it "
-            "(`python build.py` in the package directory)") from e
+        logger.warning("fxpr: the native launchers (%s) do not load with torch %s, the Python ones serve the ops: %s; "
+                       "rebuild them (`python build.py` in the package directory)", _NATIVE_PATH, torch.__version__, e)
+        return False
+    return True
+
+
+_NATIVE = _load_native()
 
 # op -> Python launcher, native counterpart in csrc/torch_ops.cpp
 _WITH_NATIVE = {
