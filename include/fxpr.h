@@ -50,7 +50,9 @@ enum {
 /* Text for a return code of any entry point (static storage). */
 const char* fxpr_error_string(int code);
 
-/* ABI revision of this header; bumped on any signature change. */
+/* ABI revision of this header, and of the library: bumped when a signature
+ * changes or the bindings need a new entry point. */
+#define FXPR_ABI_VERSION 4
 int fxpr_abi_version(void);
 
 /*

@@ -4,8 +4,10 @@ package, with other library files beside it, in a process of its own."""
 
 from __future__ import annotations
 
+import importlib.util
 import os
 import pathlib
+import re
 import shutil
 import subprocess
 import sys
@@ -72,6 +74,49 @@ def test_native_launchers_that_do_not_load_are_reported(package):
     res = run(package, REPORT)
     assert "native False" in res.stdout and "kernels loaded" in res.stdout
     assert "native launchers" in res.stderr and "libfxpr_torch.so" in res.stderr
+
+
+def test_native_launchers_refuse_another_kernel_library(package):
+    # a kernel library of another ABI revision (stubs of what the launchers
+    # link to): nothing is registered, and the bindings refuse it per call
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    shutil.copy(PKG / "libfxpr_torch.so", package)
+    source = (PKG.parent / "csrc" / "torch_ops.cpp").read_text()
+    stubs = sorted(set(re.findall(r"\b(fxpr_[a-z0-9_]+)\(", source)) - {"fxpr_abi_version", "fxpr_torch_registered"})
+    assert "fxpr_gemm" in stubs
+    text = "int fxpr_abi_version(void) { return 999; }\n" + "".join(f"int {n}(void) {{ return 0; }}\n" for n in stubs)
+    (package / "stub.c").write_text(text)
+    subprocess.run([cc, "-shared", "-fPIC", "-Wl,-soname,libfxpr_hip.so", str(package / "stub.c"), "-o",
+                    str(package / "libfxpr_hip.so")], check=True)
+    res = run(package, REPORT)
+    assert "native False" in res.stdout and "ABI revision 999" in res.stdout
+    assert "another revision" in res.stderr
+
+
+def test_build_links_both_libraries_before_replacing_either(tmp_path, monkeypatch):
+    # a launcher library that does not link leaves the old pair in place
+    spec = importlib.util.spec_from_file_location("fxpr_build_test", PKG.parent / "build.py")
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    monkeypatch.setattr(build, "BUILD", tmp_path / "_build")
+    monkeypatch.setattr(build, "OUT", tmp_path / "libfxpr_hip.so")
+    monkeypatch.setattr(build, "TORCH_OUT", tmp_path / "libfxpr_torch.so")
+    monkeypatch.setattr(build, "_check_defined", lambda lib: None)
+    build.OUT.write_text("old kernels")
+    build.TORCH_OUT.write_text("old launchers")
+
+    def fake(cmd, verbose):
+        out = pathlib.Path(cmd[cmd.index("-o") + 1])
+        if "-shared" in cmd and "torch" in out.name:
+            raise RuntimeError("does not link")
+        out.write_text("new")
+
+    monkeypatch.setattr(build, "_run", fake)
+    with pytest.raises(RuntimeError, match="does not link"):
+        build.build(jobs=1)
+    assert build.OUT.read_text() == "old kernels" and build.TORCH_OUT.read_text() == "old launchers"
 
 
 @pytest.mark.gpu

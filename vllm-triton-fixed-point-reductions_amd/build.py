@@ -121,7 +121,8 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
     objs = [BUILD / (s.stem + ".o") for s in sources]
     jobs = jobs or min(8, len(sources) + 1)
     torch_obj, torch_tmp = BUILD / "torch_ops.o", TORCH_OUT.with_suffix(".so.tmp")
-    torch_cc, torch_ld = torch_commands(torch_obj, OUT, torch_tmp)
+    tmp = OUT.with_suffix(".so.tmp")
+    torch_cc, torch_ld = torch_commands(torch_obj, tmp, torch_tmp)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         futs = [
             ex.submit(_run, [cc, *COMMON_FLAGS, *FILE_FLAGS.get(s.name, []), "-c", str(s), "-o", str(o)], verbose)
@@ -130,13 +131,14 @@ def build(jobs: int | None = None, verbose: bool = False) -> Path:
         futs.append(ex.submit(_run, torch_cc, verbose))
         for f in futs:
             f.result()
-    tmp = OUT.with_suffix(".so.tmp")
     # (the soname is how libfxpr_torch.so finds it, beside itself)
     _run([cc, "-shared", f"--offload-arch={ARCH}", "-fPIC", f"-Wl,-soname,{OUT.name}", *map(str, objs), "-o", str(tmp)],
          verbose)
     _check_defined(tmp)
-    os.replace(tmp, OUT)
     _run(torch_ld, verbose)
+    # both linked: a failure leaves the old pair, not launchers beside a
+    # kernel library that they were not built for
+    os.replace(tmp, OUT)
     os.replace(torch_tmp, TORCH_OUT)
     return OUT
 

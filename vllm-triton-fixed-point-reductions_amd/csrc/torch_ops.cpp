@@ -339,7 +339,15 @@ void reshape_and_cache(const Tensor& key_in, const Tensor& value_in, Tensor& kv_
 
 }  // namespace
 
+// (set while the library is loaded: whether the launchers below were registered)
+static int launchers_registered = 0;
+extern "C" int fxpr_torch_registered() { return launchers_registered; }
+
 TORCH_LIBRARY_IMPL(fxpr, CUDA, m) {
+  // another kernel library than the one compiled against: its entry points may
+  // take other arguments. (No exception: none can pass the loader.)
+  if (fxpr_abi_version() != FXPR_ABI_VERSION) return;
+  launchers_registered = 1;
   m.impl("float_to_fixed", &float_to_fixed);
   m.impl("fixed_to_float", &fixed_to_float);
   m.impl("fixed_row_sum", &fixed_row_sum);

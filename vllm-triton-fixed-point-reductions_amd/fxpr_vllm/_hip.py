@@ -68,7 +68,7 @@ RESTYPES = {
 }
 
 # the ABI revision these signatures describe (include/fxpr.h, fxpr_abi_version)
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 _lib: ctypes.CDLL | None = None
 _lock = threading.Lock()

@@ -15,6 +15,7 @@ reference impls (_lib.py:36-129).
 
 from __future__ import annotations
 
+import ctypes
 import logging
 
 import torch
@@ -190,8 +191,9 @@ def _log_softmax_fxp_shard_finish_cuda(x, row_max, row_sum, fxp_frac_bits, out_d
 # kernel library): they register themselves for the "CUDA" key when loaded. The
 # Python launchers below serve the remaining ops, and every op where the native
 # ones are not built or do not load (a library that does not load has registered
-# nothing): the same kernels with more host time per call. Without the kernel
-# library the import still works and every op raises.
+# nothing, nor has one built for another revision of the kernel library): the
+# same kernels with more host time per call. Without the kernel library the
+# import still works and every op raises.
 _NATIVE_PATH = _hip.LIB_PATH.with_name("libfxpr_torch.so")
 
 
@@ -203,6 +205,10 @@ def _load_native() -> bool:
     except OSError as e:
         logger.warning("fxpr: the native launchers (%s) do not load with torch %s, the Python ones serve the ops: %s; "
                        "rebuild them (`python build.py` in the package directory)", _NATIVE_PATH, torch.__version__, e)
+        return False
+    if not ctypes.CDLL(str(_NATIVE_PATH)).fxpr_torch_registered():
+        logger.warning("fxpr: the native launchers (%s) are built for another revision of libfxpr_hip.so, the Python "
+                       "ones serve the ops; rebuild both (`python build.py` in the package directory)", _NATIVE_PATH)
         return False
     return True
 
