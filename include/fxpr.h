@@ -348,6 +348,15 @@ int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_tokens,
                                        int max_blocks_per_seq, int page_size);
 
 /*
+ * Test hook (no counterpart in the reference): adds to *count (device memory)
+ * the pairs of neighbouring fp32 values, over all of them, whose softcap
+ * softcap_log2 * tanh(x / softcap_log2) descends. The 64-row prefill kernels
+ * take a chunk's maximum before the softcap, which needs 0 of them.
+ */
+int fxpr_debug_softcap_descents(float softcap_log2, unsigned long long* count,
+                                void* stream);
+
+/*
  * Paged KV-cache write: for each token t with slot = slot_mapping[t] >= 0,
  * k_cache[slot / block_size, slot % block_size, h, :] = key[t, h, :] and the
  * same for value / v_cache (the two halves of a vLLM [num_blocks, 2,

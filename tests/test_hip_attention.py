@@ -722,3 +722,12 @@ def test_prompt_chunk_over_a_wide_block_table(keys, new):
     wide = torch.zeros(1, keys // 16, dtype=torch.int32, device="cuda")
     wide[:, :bt.shape[1]] = bt
     assert torch.equal(_attend((q, kv, qsl, sl, wide, max_q), 0), _attend((q, kv, qsl, sl, bt, max_q), 1))
+
+
+@pytest.mark.parametrize("softcap", [0.5, 30.0, 50.0, 1e-3, 1e4])
+def test_softcap_is_monotone_over_every_fp32_value(softcap):
+    # the prefill workgroups' chunk maximum is taken on the raw scores and
+    # capped once: no pair of neighbouring values may descend under the cap
+    count = torch.zeros(1, dtype=torch.int64, device="cuda")
+    _hip.call("fxpr_debug_softcap_descents", softcap * RCP_LN2, count.data_ptr(), _hip.stream_ptr(count.device))
+    assert int(count) == 0

@@ -268,6 +268,26 @@ extern "C" int64_t fxpr_attention_plan(int io_dtype, int num_requests, int64_t n
   return p.ws.total;
 }
 
+// Pairs of neighbouring fp32 values, from -inf to inf, whose softcap descends.
+namespace {
+__global__ __launch_bounds__(256) void softcap_descents_kernel(float softcap, unsigned long long* count) {
+  constexpr uint32_t kInf = 0x7f800000u;
+  auto value = [](uint64_t i) {  // the i-th from -inf: -inf .. -0 at 0 .. kInf, 0 .. inf after it
+    return __uint_as_float(i <= kInf ? 0x80000000u | (kInf - uint32_t(i)) : uint32_t(i - kInf - 1));
+  };
+  unsigned long long n = 0;
+  for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < 2 * uint64_t(kInf) + 1; i += uint64_t(gridDim.x) * 256)
+    n += !(softcapped(value(i), softcap) <= softcapped(value(i + 1), softcap));
+  if (n) atomicAdd(count, n);
+}
+}  // namespace
+
+extern "C" int fxpr_debug_softcap_descents(float softcap_log2, unsigned long long* count, void* stream) {
+  if (!count || !(softcap_log2 > 0.0f)) return FXPR_E_ARG;
+  softcap_descents_kernel<<<dim3(4096), 256, 0, as_stream(stream)>>>(softcap_log2, count);
+  return launch_status();
+}
+
 extern "C" int fxpr_unified_attention(
     const void* q, const void* k_cache, const void* v_cache, void* o, int io_dtype,
     const int32_t* query_start_loc, const int32_t* seq_lens, const int32_t* block_table,

@@ -148,6 +148,9 @@ __device__ __forceinline__ float tanh_approx(float x) {
   const float t = 1.0f - 2.0f / (e + 1.0f);
   return x < 0.0f ? -t : t;
 }
+// (every step of it is monotone in x: a correctly rounded division, exp2, sum,
+// quotient and product)
+__device__ __forceinline__ float softcapped(float x, float softcap) { return softcap * tanh_approx(x / softcap); }
 
 // Query-row bookkeeping for one of the workgroup's 16 rows.
 struct RowInfo {
@@ -359,7 +362,7 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float x = __fmul_rn(acc[e], a.scale_log2);
-      if (a.softcap_log2 > 0.0f) x = a.softcap_log2 * tanh_approx(x / a.softcap_log2);
+      if (a.softcap_log2 > 0.0f) x = softcapped(x, a.softcap_log2);
       if (a.alibi) x = x + slope[e] * static_cast<float>(key - srow[e].qpos);
       const bool ok = srow[e].valid && key >= srow[e].kstart && key < srow[e].kend;
       s[e] = ok ? x : -__builtin_inff();
@@ -1067,7 +1070,7 @@ __device__ __forceinline__ void attn_dma_body(const AttnArgs& a, const unsigned 
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             float x = __fmul_rn(acc[e], a.scale_log2);
-            if (a.softcap_log2 > 0.0f) x = a.softcap_log2 * tanh_approx(x / a.softcap_log2);
+            if (a.softcap_log2 > 0.0f) x = softcapped(x, a.softcap_log2);
             if (a.alibi) x = x + slope[e] * static_cast<float>(key - qp[e]);
             sc[u][e] = (key >= ks[e] && key < ke[e]) ? x : -__builtin_inff();
             mx[e] = fmaxf(mx[e], sc[u][e]);
@@ -1420,7 +1423,7 @@ __global__ __launch_bounds__(kPThreads, 2) void attn_prefill_kernel(AttnArgs a) 
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float x = __fmul_rn(acc[e], a.scale_log2);
-      if (a.softcap_log2 > 0.0f) x = a.softcap_log2 * tanh_approx(x / a.softcap_log2);
+      if (a.softcap_log2 > 0.0f) x = softcapped(x, a.softcap_log2);
       if (a.alibi) x = x + slope[e] * static_cast<float>(key - qp[e]);
       s[e] = (key >= ks[e] && key < ke[e]) ? x : -__builtin_inff();
     }
@@ -1996,8 +1999,8 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
   // its range, see fast_den); P is packed without the canonical-NaN rule (any
   // NaN weight yields a NaN weighted V either way, which quantises to 0).
   const bool fast_den = BITS != 64 && a.fxp_scale <= (BITS == 16 ? 16384.0f : 4194304.0f);
-  // With a softcap the same holds around it (CAP): tanh_approx is monotone
-  // (checked over every fp32 value), so the chunk maximum is the capped maximum
+  // With a softcap the same holds around it (CAP): softcapped is monotone
+  // (fxpr_debug_softcap_descents), so the chunk maximum is the capped maximum
   // of the raw scores, and only phase 1 computes a score's tanh and divisions
   // (3 x up to 1018 tokens after up to 5643, 32 heads: 1.24 -> 0.73 ms).
   const bool cap = a.softcap_log2 > 0.0f;
@@ -2005,7 +2008,7 @@ __device__ __forceinline__ void attn_prefill_dma_body(const AttnArgs& a, const u
   const float vlim = (BITS == 16 ? 32767.0f : 4194304.0f) / a.fxp_scale;  // 2^f: exact
   auto run = [&](auto fast_tag, auto cap_tag) __attribute__((always_inline)) {
     constexpr bool FAST = decltype(fast_tag)::value, CAP = decltype(cap_tag)::value;
-    auto capped = [&](float x) { return a.softcap_log2 * tanh_approx(x / a.softcap_log2); };
+    auto capped = [&](float x) { return softcapped(x, a.softcap_log2); };
     // A step consumes C ring entries (1: a K tile of phase 0; 2: a tile's K
     // and V in phase 1) and issues C more: the cursor stays NS - 2 entries
     // ahead, so the two slots a 2-entry step refills are free. Returns the

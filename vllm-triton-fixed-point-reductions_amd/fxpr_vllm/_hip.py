@@ -57,6 +57,8 @@ SIGNATURES: dict[str, list] = {
     "fxpr_debug_set_lsm_spin_limit": [_I, _I],
     "fxpr_debug_lsm_default_spin_limit": [],
     "fxpr_debug_lsm_fallbacks": [ctypes.POINTER(ctypes.c_ulonglong)],
+    # test hook of the softcap's monotonicity
+    "fxpr_debug_softcap_descents": [_F, _P, _P],
 }
 
 # entry points that return something other than an int status
