@@ -620,10 +620,10 @@ def _ragged(reqs, hq, hkv, d, ps, dtype, seed):
     return q, kv, qsl.cuda(), sl.cuda(), bt.cuda(), max(n for n, _ in reqs)
 
 
-def _attend(inp, splits, bits=32, frac=16, window=0, softcap=0.0, causal=True):
+def _attend(inp, splits, bits=32, frac=16, window=0, softcap=0.0, causal=True, alibi=None):
     q, kv, qsl, sl, bt, max_q = inp
     o = torch.full_like(q, 7.0)
-    KA.unified_attention_fxp_run(q, kv, o, qsl, sl, bt, max_q, None, causal, None, bits, frac, softcap, window, splits)
+    KA.unified_attention_fxp_run(q, kv, o, qsl, sl, bt, max_q, alibi, causal, None, bits, frac, softcap, window, splits)
     return o
 
 
@@ -731,3 +731,55 @@ def test_softcap_is_monotone_over_every_fp32_value(softcap):
     count = torch.zeros(1, dtype=torch.int64, device="cuda")
     _hip.call("fxpr_debug_softcap_descents", softcap * RCP_LN2, count.data_ptr(), _hip.stream_ptr(count.device))
     assert int(count) == 0
+
+
+def _alone_equal(inp, base, opts, which):
+    q, kv, qsl, sl, bt, _ = inp
+    at = qsl.tolist()
+    for i in which:
+        n = at[i + 1] - at[i]
+        one = (q[at[i]:at[i + 1]].contiguous(), kv, torch.tensor([0, n], dtype=torch.int32, device="cuda"),
+               sl[i:i + 1].contiguous(), bt[i:i + 1].contiguous(), n)
+        assert torch.equal(_attend(one, 0, **opts), base[at[i]:at[i + 1]]), i
+
+
+@pytest.mark.parametrize("d,hq,hkv,max_q,mix", [
+    (128, 16, 4, 512, False),    # two launches, the prefill one a flat grid
+    (64, 16, 8, 512, False),
+    (128, 8, 2, 512, True),      # both kinds in one grid, its prefill part flat
+    (128, 8, 2, 30000, True),    # flat because of a loose max_query_len
+])
+def test_flat_prefill_grid_unsplit(d, hq, hkv, max_q, mix):
+    # one prompt chunk among many decode steps, contexts of one block-table
+    # row of at most 2048 keys: nothing is split, and more than 4096 workgroups
+    # of a request-by-tile prefill grid would find no rows
+    reqs = ([(1, 30 + 17 * i) for i in range(60)] + [(min(max_q, 512), 1900), (70, 70), (3, 900)] +
+            [(1, 2000 - 40 * i) for i in range(40)]) if max_q == 512 else [(60, 200), (1, 300), (3, 50), (130, 700)]
+    inp = (*_ragged(reqs, hq, hkv, d, 16, torch.bfloat16, d + hq)[:5], max_q)
+    tokens, R, group = inp[0].shape[0], len(reqs), hq // hkv
+    empty = (R * -(-max_q * group // 64) - (tokens * group // 64 + R)) * hkv
+    assert empty > 4096 and (-(-tokens * hq // 64) + R * hkv <= 512) == mix
+    base = _attend(inp, 1)
+    assert torch.equal(_attend(inp, 0), base)
+    _alone_equal(inp, base, {}, range(0, R, 1 if R < 10 else 7))
+    if R > 10:
+        _alone_equal(inp, base, {}, (60, 61, 62))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("reqs", [
+    [(1, 700), (130, 2300), (1, 2600), (3, 513), (12, 40)],
+    [(64, 2100), (1, 64), (70, 70), (48, 2049)],
+])
+@pytest.mark.parametrize("opts", [dict(alibi=True), dict(causal=False), dict(alibi=True, causal=False, window=600),
+                                  dict(alibi=True, softcap=20.0)])
+def test_mixed_batch_with_alibi_and_non_causal(dtype, reqs, opts):
+    # the split prefill workgroups off their fast variant, and over keys after
+    # the row's own position
+    inp = _ragged(reqs, 8, 2, 128, 16, dtype, seed=len(reqs))
+    if opts.get("alibi"):
+        opts = {**opts, "alibi": torch.tensor([2.0 ** -i for i in range(1, 9)], device="cuda")}
+    base = _attend(inp, 1, **opts)
+    for splits in (0, 2, 5):
+        assert torch.equal(_attend(inp, splits, **opts), base), splits
+    _alone_equal(inp, base, opts, range(len(reqs)))
