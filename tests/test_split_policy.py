@@ -239,7 +239,8 @@ def test_gemm_auto_split_fills_the_gpu(lib):
     assert gemm_splits(lib, 32, 128256, 4096) == 1       # 501 tiles
     assert gemm_splits(lib, 8192, 128256, 4096) == 1
     assert gemm_splits(lib, 32, 4096, 256) == 2          # capped at the 2 K-tiles
-    # fp32 inputs keep the skinny tiles (16 / 32 / 64 x 256) and 64-wide K-tiles
+    # fp32 inputs up to M = 32 (tiles of 256 columns, 64-wide K-tiles), and a
+    # shape that fills the GPU unsplit
     assert gemm_splits(lib, 1, 4096, 4096, F32) == 16
     assert gemm_splits(lib, 32, 14336, 4096, F32) == 9   # 56 tiles
     assert gemm_splits(lib, 8192, 14336, 4096, F32) == 1

@@ -2578,16 +2578,16 @@ template <int DT, int BITS> int launch_combine(const AttnArgs& a, int64_t ws_row
 // would only start workgroups that exit at once
 constexpr int kShortTiles = (kPrefillRows - 1 + QROWS - 1) / QROWS;
 
-// Requests of at least kPrefillRows rows in 64-row workgroups, the others
-// (decode steps, short prompts) in 16-row ones; both kernels see the whole
-// batch and each skips the other's requests. Same bits per row either way.
-// empty workgroups of the request-by-tile prefill grid from which the flat one
+// Empty workgroups of the request-by-tile prefill grid from which the flat one
 // is taken: it costs a load of the token bounds per workgroup and the
 // longest-first order across requests (three prompts of 921 tokens among four
 // decode steps, 1500 empty workgroups: 53 us flat, 47 not; one of 512 among 31,
 // 7700 empty: the launch 8 us shorter)
 constexpr int64_t kFlatEmpty = 4096;
 
+// Requests of at least kPrefillRows rows in 64-row workgroups, the others
+// (decode steps, short prompts) in 16-row ones; both kernels see the whole
+// batch and each skips the other's requests. Same bits per row either way.
 template <int DT, int BITS, int DMAX>
 int launch_long(AttnArgs a, const LongPlan& lp, int num_requests, int max_qtiles, int64_t num_tokens, hipStream_t st) {
   a.pq_rows = kPrefillRows;
@@ -2639,7 +2639,7 @@ int launch_attn(const AttnArgs& a, const LongPlan& lp, int num_requests, int max
     if (lp.route == Route::kLongDma)
       return launch_long<DT, BITS, DMAX>(a, lp, num_requests, max_qtiles, num_tokens, st);
     if (lp.route == Route::kLong) {
-      // as launch_long, on the register-load kernels
+      // as launch_long, on the register-load kernels and unsplit
       AttnArgs b = a;
       b.pq_rows = kPrefillRows;
       const dim3 pgrid(grid.x, unsigned(cdiv(int64_t(max_qtiles) * QROWS, PQROWS)), 1);
