@@ -337,10 +337,12 @@ int64_t fxpr_attention_plan(int io_dtype, int num_requests, int64_t num_tokens,
                             int num_heads, int num_kv_heads, int head_dim,
                             int page_size, int max_query_len,
                             int max_blocks_per_seq, int64_t stride_k_slot,
-                            int64_t stride_v_slot, int int_bits,
-                            int num_kv_splits, int32_t* plan);
+                            int64_t stride_v_slot, int is_causal,
+                            int window_size, int int_bits, int num_kv_splits,
+                            int32_t* plan);
 
-/* The same without the input type and the cache's strides: enough for any. */
+/* The same without the input type, the cache's strides and the window: enough
+ * for any. */
 int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_tokens,
                                        int num_heads, int num_kv_heads,
                                        int head_dim, int int_bits,

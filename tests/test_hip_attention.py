@@ -783,3 +783,22 @@ def test_mixed_batch_with_alibi_and_non_causal(dtype, reqs, opts):
     for splits in (0, 2, 5):
         assert torch.equal(_attend(inp, splits, **opts), base), splits
     _alone_equal(inp, base, opts, range(len(reqs)))
+
+
+@pytest.mark.parametrize("dtype,d,hq,hkv", [(torch.bfloat16, 128, 8, 2), (torch.float16, 64, 4, 4)])
+@pytest.mark.parametrize("reqs", [
+    [(1, 700), (130, 2300), (1, 2600), (3, 513), (12, 40)],
+    [(20, 2300), (1, 900), (2, 4000)],              # few rows
+    [(1, 6000), (150, 3000)] + [(1, 3000 - 60 * i) for i in range(40)],
+])
+@pytest.mark.parametrize("opts", [dict(), dict(window=600), dict(window=1024, causal=False)])
+@pytest.mark.parametrize("keys", [8192, 16384, 40000])
+def test_automatic_plans_over_wide_tables(dtype, d, hq, hkv, reqs, opts, keys):
+    # every way the automatic plan takes with the table's width and the window
+    # (16-row split, runs of chunks, evenly dealt chunks, windows): the unsplit bits
+    q, kv, qsl, sl, bt, max_q = _ragged(reqs, hq, hkv, d, 16, dtype, seed=keys + len(reqs))
+    base = _attend((q, kv, qsl, sl, bt, max_q), 1, **opts)
+    wide = torch.zeros(len(reqs), keys // 16, dtype=torch.int32, device="cuda")
+    wide[:, :bt.shape[1]] = bt
+    for table in (bt, wide):
+        assert torch.equal(_attend((q, kv, qsl, sl, table, max_q), 0, **opts), base)

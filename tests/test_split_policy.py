@@ -88,12 +88,12 @@ ROWS16, ROWS16_DMA, LONG, LONG_DMA = range(4)
 
 
 def attn_plan(lib, requests, tokens, max_q, keys, dt=1, heads=32, kv_heads=8, d=128, page=16, bits=32, stride=None,
-              requested=0):
+              requested=0, window=0, causal=1):
     """(kernels, splits of long requests, of short ones, record rows per request, workspace bytes)"""
     plan = (ctypes.c_int32 * 4)()
     stride = kv_heads * d if stride is None else stride
     n = lib.fxpr_attention_plan(dt, requests, tokens, heads, kv_heads, d, page, max_q, -(-keys // page), stride, stride,
-                                bits, requested, plan)
+                                causal, window, bits, requested, plan)
     return (*plan, n)
 
 
@@ -136,13 +136,13 @@ def test_attention_workspace_is_the_running_launchs(lib):
 def test_attention_long_requests_over_wide_tables_stay_split(lib):
     # 512 MiB of records, 1 GiB with fewer than 128 prefill workgroups
     half, full = 1 << 29, 1 << 30
-    for tokens, keys, splits in ((128, 131072, 32), (130, 131072, 32), (250, 131072, 17)):
+    for tokens, keys, splits in ((128, 131072, 16), (130, 131072, 16), (250, 131072, 9)):
         n = record_bytes(tokens, keys)
         assert half < n <= full
         assert attn_plan(lib, 1, tokens, tokens, keys) == (LONG_DMA, splits, 1, 0, n), tokens
         # (the register-load kernels: as many records, 64 splits)
         assert attn_plan(lib, 1, tokens, tokens, keys, dt=F32) == (ROWS16, 64, 64, 0, n), tokens
-    assert attn_plan(lib, 1, 64, 64, 131072)[1] == 64                          # 260 MiB
+    assert attn_plan(lib, 1, 64, 64, 131072)[1] == 32                          # 260 MiB
     for tokens, keys in ((256, 65536), (512, 32768)):
         assert half < record_bytes(tokens, keys) <= full
         assert attn_plan(lib, 1, tokens, tokens, keys) == (LONG_DMA, 1, 1, 0, 0), tokens
@@ -153,13 +153,13 @@ def test_attention_long_requests_over_wide_tables_stay_split(lib):
     assert attn_plan(lib, 1, 256, 256, 131072, dt=F32) == (ROWS16, 1, 1, 0, 0)
     # and only where the 16-row kernels would split the batch as well
     assert half < record_bytes(130, 131072) <= full
-    assert attn_plan(lib, 80, 130, 12, 131072)[1:] == (32, 64, 0, record_bytes(130, 131072))
+    assert attn_plan(lib, 80, 130, 12, 131072)[1:] == (16, 1, 0, record_bytes(130, 131072))
     assert attn_plan(lib, 90, 130, 12, 131072)[1:] == (1, 1, 0, 0)
     # a chunk beside 31 decode steps; above the cap the decode steps keep
     # records of their own tokens only
-    assert attn_plan(lib, 32, 543, 512, 28672) == (LONG_DMA, 8, 56, 0, record_bytes(543, 28672))
+    assert attn_plan(lib, 32, 543, 512, 28672) == (LONG_DMA, 4, 2, 0, record_bytes(543, 28672))
     assert half < record_bytes(543, 30720) <= full
-    assert attn_plan(lib, 32, 543, 512, 30720) == (LONG_DMA, 1, 60, 11, record_bytes(32 * 11, 30720))
+    assert attn_plan(lib, 32, 543, 512, 30720) == (LONG_DMA, 1, 2, 11, record_bytes(32 * 11, 30720))
 
 
 def test_attention_batches_of_equal_long_requests_keep_no_short_records(lib):
@@ -167,10 +167,60 @@ def test_attention_batches_of_equal_long_requests_keep_no_short_records(lib):
     # tokens; the prefill rows' own splits are not affected
     assert attn_plan(lib, 4, 4 * 2048, 2048, 131072) == (LONG_DMA, 1, 1, 0, 0)
     assert attn_plan(lib, 1, 512, 512, 131072) == (LONG_DMA, 1, 1, 0, 0)     # records of 512 tokens: 2 GiB
-    assert attn_plan(lib, 1, 64, 64, 32768) == (LONG_DMA, 64, 1, 0, record_bytes(64, 32768))
+    assert attn_plan(lib, 1, 64, 64, 32768) == (LONG_DMA, 32, 1, 0, record_bytes(64, 32768))
     # one token less (some request is shorter), and one more (padding)
     for tokens in (4 * 2048 - 1, 4 * 2048 + 1):
-        assert attn_plan(lib, 4, tokens, 2048, 131072) == (LONG_DMA, 1, 64, 11, record_bytes(4 * 11, 131072))
+        assert attn_plan(lib, 4, tokens, 2048, 16384) == (LONG_DMA, 1, 32, 11, record_bytes(4 * 11, 16384))
+        # a wide table: long on average is taken for all long
+        assert attn_plan(lib, 4, tokens, 2048, 131072) == (LONG_DMA, 1, 1, 0, 0)
+    assert attn_plan(lib, 4, 500 + 599, 500, 16400)[1:3] == (1, 32)    # others of 199.7 tokens on average
+    assert attn_plan(lib, 4, 500 + 600, 500, 16400)[1:3] == (1, 1)     # of 200
+
+
+def test_attention_short_requests_splits(lib):
+    # a 100-token chunk beside decode steps, 7 chunks: runs of chunks while the
+    # short requests' workgroups number 512 or fewer, unsplit from there on
+    for requests, splits in ((2, 7), (16, 7), (64, 7), (65, 1), (300, 1)):
+        assert attn_plan(lib, requests, requests + 99, 100, 3584)[2] == splits, requests
+    assert attn_plan(lib, 64, 163, 100, 16384)[2] == 16                # 32 chunks, runs of two
+    # beyond 16384 keys: 512 workgroups (1024 for up to 64), at most 64 splits
+    for requests, splits in ((2, 64), (8, 16), (9, 8), (16, 4), (33, 2), (63, 2), (64, 1), (300, 1)):
+        assert attn_plan(lib, requests, requests + 99, 100, 65536)[2] == splits, requests
+
+
+def test_attention_few_rows_take_the_16_row_split(lib):
+    # up to 320 rows (tokens x group) and 3000 units over tables of up to 16384
+    # keys, where the plain policy splits: its launch, long requests included
+    assert attn_plan(lib, 3, 28, 26, 2528) == (ROWS16_DMA, 5, 5, 0, record_bytes(28, 2528))
+    assert attn_plan(lib, 1, 80, 80, 4096)[0] == ROWS16_DMA             # 320 rows
+    assert attn_plan(lib, 1, 81, 81, 4096)[0] == LONG_DMA
+    assert attn_plan(lib, 1, 80, 80, 8320)[0] == ROWS16_DMA             # 8 x 21 x 17 = 2856 units
+    assert attn_plan(lib, 1, 80, 80, 8704 + 16)[0] == LONG_DMA          # 18 chunks: 3024
+    assert attn_plan(lib, 3, 28, 26, 2048)[0] == LONG_DMA               # nothing splits
+    assert attn_plan(lib, 3, 28, 26, 32768)[0] == LONG_DMA              # wide
+    assert attn_plan(lib, 3, 28, 26, 2528, requested=2)[0] == LONG_DMA  # explicit
+
+
+def test_attention_small_windows(lib):
+    # windows of up to 2048 keys leave 3 chunks (of 1024 keys) per row: prefill
+    # rows split below 141 workgroups, short requests below 128
+    w = dict(window=1024)
+    assert attn_plan(lib, 1, 118, 118, 2112, **w) == (LONG_DMA, 3, 1, 0, record_bytes(118, 2112))
+    assert attn_plan(lib, 1, 280, 280, 8192, **w)[1:3] == (3, 1)        # 140 workgroups
+    assert attn_plan(lib, 1, 282, 282, 8192, **w)[1:3] == (1, 1)
+    assert attn_plan(lib, 15, 300, 250, 8192, **w)[2] == 3              # 120 short workgroups
+    assert attn_plan(lib, 16, 300, 250, 8192, **w)[2] == 1
+    # a table that splits nothing, a wider window, and one without causality
+    assert attn_plan(lib, 1, 118, 118, 2048, **w)[1:3] == (1, 1)
+    plain = attn_plan(lib, 2, 282, 281, 8192)
+    assert attn_plan(lib, 2, 282, 281, 8192, window=2049) == plain
+    assert attn_plan(lib, 2, 282, 281, 8192, causal=0, **w) == plain
+    # the bound without the window covers every plan
+    for requests, tokens, max_q in ((1, 118, 118), (3, 28, 26), (15, 300, 250), (40, 128, 89), (2, 282, 281)):
+        for keys in (2112, 8192, 16384, 65536, 131072):
+            bound = lib.fxpr_attention_workspace_bytes(requests, tokens, 32, 8, 128, 32, 0, max_q, -(-keys // 16), 16)
+            for kw in (dict(), w, dict(window=100), dict(window=4096), dict(causal=0, **w), dict(dt=F32)):
+                assert attn_plan(lib, requests, tokens, max_q, keys, **kw)[-1] <= bound, (requests, keys, kw)
 
 
 def test_attention_kernels_by_the_longest_requests_rows(lib):

@@ -102,15 +102,33 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
 
 // Launches that may hold requests of kPrefillRows rows or more, where the DMA
 // kernels can take them (Route::kLongDma): the two kinds of requests are split
-// apart from each other.
+// apart from each other, over tables of more than 32 key tiles. The host knows
+// the table's width and not the contexts, so every number of splits is paid for
+// by batches whose contexts are short: workgroups that find no keys (600 of them
+// start and exit in a microsecond), records and a combine launch.
 //   * Prefill workgroups (64 rows each): about tokens x heads / 64 of them.
-//     Below 512 (two per CU) their keys are split until there are about
+//     Below kFullWgs (two per CU) their keys are split until there are about
 //     kLongWgs; a chunk is the least a split can hold.
-//   * Short requests: one chunk per split, as in launches of their own, when
-//     their contexts can be long (more than 32 tiles) and there can be any:
-//     tokens that are just requests x the longest one's leave none (4 prompts
-//     of 2048 tokens, block table of 131072 keys: 6144 workgroups that found
-//     no request, 179 MiB of records and a combine launch, 366 us; 340 without).
+//   * Short requests, one workgroup per request and kv head (`rk` of them): up to
+//     kFullWgs split into equal runs of chunks, about kShortWgs in all. (Beyond
+//     it, 77 decode steps of up to 3000 keys beside 2 x 166 tokens, 16 heads of 64:
+//     133 us unsplit, 156 split by chunk, 202 in runs of two.)
+//   * Tables wider than kWideKeys say little about the contexts: the short
+//     requests' own chunks are dealt evenly to splits that make up kFullWgs
+//     workgroups (twice that for few), the prefill ones' to half as many, and a batch
+//     of long requests on average is taken to hold no short ones. (Split 64 ways,
+//     61 decode steps of up to 9300 keys beside 4 prompts of 22 tokens, 24/8 heads
+//     of 64, took 730 us at a table of 131072 keys; 192 now, 181 unsplit.)
+//   * A window of up to kSmallWindow keys leaves a few chunks per row whatever the
+//     table: split where the launch leaves the GPU nearly empty.
+//   * No short request is possible where the tokens are just requests x the
+//     longest one's (4 prompts of 2048 tokens, table of 131072 keys: 366 us with
+//     the short requests' split, 340 without).
+// Against the plan before requests were split apart (us before / now, geometric
+// mean): drawn batches with prompts, tables as wide as their longest context (up
+// to 12288 keys) 1.40x, 10 of 272 more than 3 % slower, the worst 1.18x; tables of
+// 8192 keys 1.52x, 9 of 78, 1.6x (83 decode steps under 300 keys beside 3 x 79
+// tokens, 36 -> 58); 32768 1.9x, 8 of 101, 1.34x; 131072 2.1x, 2 of 74, 1.06x.
 // Explicit requests split both that many times. Records need a workspace: per
 // token when the prefill rows are split, else only for the short requests'
 // tokens. Above kLongWsMax the launch runs unsplit; above kSplitWsMax where the
@@ -120,7 +138,9 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
 // 131072 keys 885 us unsplit, 462 split by 16 rows, 197 split here; 256 at 65536
 // 887 and 921. The wider cap at 256 and 512 tokens too would take 512 at 32768
 // from 897 to 697, but 512 without cached keys from 22 to 36).
-constexpr int64_t kFullWgs = 512, kLongWgs = 2048, kFewWgs = 128;
+constexpr int64_t kFullWgs = 512, kLongWgs = 2048, kShortWgs = 8192, kFewWgs = 128;
+constexpr int64_t kWideKeys = 16384, kSmallWindow = 2048, kWindowWgs = 140, kWindowShort = 128;
+constexpr int64_t kLongTokens = 200;  // tokens per request besides the longest that mean "long on average"
 constexpr int64_t kLongWsMax = int64_t(1) << 29;
 
 struct LongLayout {
@@ -129,20 +149,34 @@ struct LongLayout {
 };
 
 LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int num_kv_heads, int head_dim, int int_bits,
-                     int max_query_len, int max_blocks, int page_size, int requested) {
+                     int max_query_len, int max_blocks, int page_size, int64_t window, int requested) {
   LongLayout l;
   const int group = num_heads / num_kv_heads;
   const int64_t slots = chunk_slots(max_blocks, page_size);
-  const int64_t tiles = cdiv(int64_t(max_blocks > 0 ? max_blocks : 1) * page_size, TILE);
+  const int64_t keys = int64_t(max_blocks > 0 ? max_blocks : 1) * page_size;
   const int64_t wgs = std::max<int64_t>(cdiv(num_tokens * num_heads, PQROWS), 1);
-  int64_t ps = 1, ds = 1;
+  int64_t ps = 1, ds = 1, per = 0;  // per: chunks per split of the short requests (0: dealt evenly)
   if (requested >= 1) {
     ps = ds = std::min<int64_t>({int64_t(requested), std::max<int64_t>(slots, 1), kMaxGridZ});
-  } else {
-    if (wgs < kFullWgs && tiles > 32) ps = std::min<int64_t>(cdiv(kLongWgs, wgs), slots);
-    const bool all_long = num_tokens == int64_t(num_requests) * max_query_len;
-    if (tiles > 32 && int64_t(num_requests) * num_kv_heads <= 8 * 256 && !all_long)
-      ds = std::min<int64_t>(slots, kMaxSplits);
+  } else if (cdiv(keys, TILE) > 32) {
+    const int64_t rk = int64_t(num_requests) * num_kv_heads, others = num_tokens - max_query_len;
+    const bool wide = keys > kWideKeys;
+    bool shorts = num_tokens != int64_t(num_requests) * max_query_len;
+    if (window > 0) {
+      const int64_t chunks = std::min(slots, cdiv(window, TILE * CT) + 1);  // those a row's window can touch
+      if (wgs <= kWindowWgs) ps = chunks;
+      if (rk < kWindowShort) ds = chunks;
+    } else {
+      if (wgs < kFullWgs) ps = std::min(cdiv(wide ? kLongWgs / 2 : kLongWgs, wgs), slots);
+      if (wide) {
+        shorts = shorts && others < kLongTokens * (num_requests - 1);
+        if (rk < kFullWgs) ds = std::min<int64_t>({cdiv(rk <= 64 ? 2 * kFullWgs : kFullWgs, rk), slots, kMaxSplits});
+      } else if (rk <= kFullWgs) {
+        per = std::max<int64_t>(rk * slots / kShortWgs, 1);
+        ds = cdiv(slots, per);
+      }
+    }
+    if (!shorts) ds = 1;
   }
   auto layout = [&](int64_t rows) { return ws_layout(rows, num_heads, head_dim, int_bits, true, slots); };
   const int64_t most = requested >= 1 ? kSplitWsMax : kLongWsMax;
@@ -172,9 +206,12 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
   }
   l.plan.pq_splits = int(ps);
   l.plan.splits = int(ds);
-  l.plan.chunks_per_split = requested >= 1 || ds <= 1 ? 0 : int(cdiv(slots, ds));
+  l.plan.chunks_per_split = ds > 1 ? int(per) : 0;
   return l;
 }
+
+// rows (tokens x group) and 16-row chunk units up to which a batch counts as few
+constexpr int64_t kFewRows = 320, kFewChunks = 3000;
 
 // What a launch runs: its kernels, its splits and the records they need.
 struct LaunchPlan {
@@ -185,7 +222,7 @@ struct LaunchPlan {
 
 LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, int num_heads, int num_kv_heads,
                           int head_dim, int page_size, int max_query_len, int max_blocks, int64_t stride_k_slot,
-                          int64_t stride_v_slot, int int_bits, int requested) {
+                          int64_t stride_v_slot, int is_causal, int window_size, int int_bits, int requested) {
   LaunchPlan p;
   const bool dma = dma_takes(io_dtype, head_dim, page_size, stride_k_slot, stride_v_slot);
   const int group = num_heads / num_kv_heads;
@@ -194,16 +231,30 @@ LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, in
   // requests of kPrefillRows rows or more
   const bool narrow_sums = io_dtype != FXPR_DTYPE_F32 && int_bits != 64;
   const bool wide = narrow_sums && head_dim <= 128 && max_rows >= kPrefillRows;
-  if (wide && dma) {
+  // a window that leaves few keys per row (and bounds them on both sides)
+  const int64_t keys = int64_t(max_blocks) * page_size;
+  const int64_t window =
+      is_causal && window_size > 0 && window_size <= kSmallWindow && window_size < keys ? window_size : 0;
+  p.sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len, max_blocks,
+                     page_size, requested);
+  // A few tokens in all, over tables that are not wide: one split launch of
+  // 16-row workgroups spreads them further than 64-row ones, and takes two
+  // launches instead of three. Both sides, us: 28 tokens in 3 requests over up to
+  // 2500 keys (32/8 heads of 128) 23 against 42 apart; 79 in 8 with a softcap 45
+  // and 69; 140 of 24/8 heads of 64 over 2400 47 and 38 (420 rows: apart).
+  const int64_t rows = num_tokens * group;
+  const int64_t chunks = cdiv(window > 0 ? std::min<int64_t>(keys, window + max_query_len) : keys, TILE * CT);
+  const bool few_rows = requested == 0 && p.sp.splits > 1 && keys <= kWideKeys && rows <= kFewRows &&
+                        num_kv_heads * (cdiv(rows, QROWS) + num_requests) * chunks <= kFewChunks;
+  if (wide && dma && !few_rows) {
     const LongLayout l = long_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len,
-                                   max_blocks, page_size, requested);
+                                   max_blocks, page_size, window, requested);
+    p.sp = SplitPlan{1, 0};
     p.lp = l.plan;
     p.lp.route = Route::kLongDma;
     p.ws = l.ws;
     return p;
   }
-  p.sp = launch_plan(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, int_bits, max_query_len, max_blocks,
-                     page_size, requested);
   p.ws = ws_layout(num_tokens, num_heads, head_dim, int_bits, p.sp.splits > 1, chunk_slots(max_blocks, page_size));
   // Just short of that, three 16-row tiles a request (33 to 47 rows), the DMA
   // kernel is the faster one at head_dim 128 (us, register loads / DMA: 1 x 10
@@ -239,25 +290,27 @@ extern "C" int64_t fxpr_attention_workspace_bytes(int num_requests, int64_t num_
                                                   int num_kv_heads, int head_dim, int int_bits,
                                                   int num_kv_splits, int max_query_len,
                                                   int max_blocks_per_seq, int page_size) {
-  // whatever the inputs' type and the cache's strides: with the DMA kernels or without
-  auto need = [&](int io_dtype) {
+  // whatever the inputs' type, the cache's strides and the window: with the DMA
+  // kernels or without, and the widest and the narrowest window
+  auto need = [&](int io_dtype, int window) {
     return fxpr_attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
-                               max_query_len, max_blocks_per_seq, head_dim, head_dim, int_bits, num_kv_splits, nullptr);
+                               max_query_len, max_blocks_per_seq, head_dim, head_dim, 1, window, int_bits,
+                               num_kv_splits, nullptr);
   };
-  return std::max(need(FXPR_DTYPE_BF16), need(FXPR_DTYPE_F32));
+  return std::max({need(FXPR_DTYPE_BF16, 0), need(FXPR_DTYPE_BF16, 1), need(FXPR_DTYPE_F32, 0)});
 }
 
 extern "C" int64_t fxpr_attention_plan(int io_dtype, int num_requests, int64_t num_tokens, int num_heads,
                                        int num_kv_heads, int head_dim, int page_size, int max_query_len,
                                        int max_blocks_per_seq, int64_t stride_k_slot, int64_t stride_v_slot,
-                                       int int_bits, int num_kv_splits, int32_t* plan) {
+                                       int is_causal, int window_size, int int_bits, int num_kv_splits, int32_t* plan) {
   if (plan) std::fill(plan, plan + 4, 0);
   if (!plan_args_ok(num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size, max_blocks_per_seq,
                     num_kv_splits))
     return 0;
   const LaunchPlan p = attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
-                                      max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits,
-                                      num_kv_splits);
+                                      max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, is_causal,
+                                      window_size, int_bits, num_kv_splits);
   if (plan) {
     const bool apart = p.lp.route == Route::kLongDma;
     plan[0] = int(p.lp.route);
@@ -276,7 +329,8 @@ __global__ __launch_bounds__(256) void softcap_descents_kernel(float softcap, un
     return __uint_as_float(i <= kInf ? 0x80000000u | (kInf - uint32_t(i)) : uint32_t(i - kInf - 1));
   };
   unsigned long long n = 0;
-  for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < 2 * uint64_t(kInf) + 1; i += uint64_t(gridDim.x) * 256)
+  const uint64_t step = uint64_t(gridDim.x) * 256;
+  for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < 2 * uint64_t(kInf) + 1; i += step)
     n += !(softcapped(value(i), softcap) <= softcapped(value(i + 1), softcap));
   if (n) atomicAdd(count, n);
 }
@@ -321,8 +375,8 @@ extern "C" int fxpr_unified_attention(
   const int64_t slots = chunk_slots(max_blocks_per_seq, page_size);
   if (slots > 0x7fffffff) return FXPR_E_SHAPE;
   LaunchPlan plan = attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
-                                   max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits,
-                                   num_kv_splits);
+                                   max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, is_causal,
+                                   window_size, int_bits, num_kv_splits);
   if (plan.ws.total > 0 && (!workspace || workspace_bytes < plan.ws.total)) return FXPR_E_WORKSPACE;
 
   AttnArgs a{};
@@ -448,8 +502,8 @@ extern "C" int fxpr_unified_attention_noalloc(
     int frac_bits, int num_kv_splits, void* stream) {
   auto ws_need = [&](int splits) {
     return fxpr_attention_plan(io_dtype, num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
-                               max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, int_bits, splits,
-                               nullptr);
+                               max_query_len, max_blocks_per_seq, stride_k_slot, stride_v_slot, is_causal, window_size,
+                               int_bits, splits, nullptr);
   };
   int64_t need = ws_need(num_kv_splits);
   if (need > 0 && num_kv_splits == 0) {

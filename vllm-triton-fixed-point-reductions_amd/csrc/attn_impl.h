@@ -714,14 +714,19 @@ constexpr int kCpolNT = 2;
 // a radix select over the length bits finds the (k + 1)-th largest length T
 // (31 steps of kOrderMax / 64 ballots), then the requests of length T are
 // taken in index order. Launches whose workgroups hold at most one chunk
-// each keep the launch order (the order gains nothing there).
-constexpr int kOrderMax = 256;
+// each keep the launch order (the order gains nothing there), and so do those
+// with chunks dealt evenly to many splits (most hold none or one, and the select
+// costs a workgroup that exits more than anything else it does: three prompts of
+// 57 tokens over a table of 32768 keys, 43 splits for short requests: 31 us with
+// it).
+constexpr int kOrderMax = 256, kOrderSplits = 8;
 __device__ __forceinline__ int request_by_length(const AttnArgs& a, int k) {
   const int R = a.num_requests;
   const int per_max = a.num_splits <= 1 ? a.chunk_slots + 1
                       : a.chunks_per_split > 0 ? a.chunks_per_split
                                                : (a.chunk_slots + a.num_splits - 1) / a.num_splits;
   if (R <= 1 || R > kOrderMax || k >= R || per_max <= 1) return k;
+  if (a.chunks_per_split <= 0 && a.num_splits > kOrderSplits) return k;
   constexpr int NB = kOrderMax / 64;
   const int lane = threadIdx.x & 63;
   int len[NB];

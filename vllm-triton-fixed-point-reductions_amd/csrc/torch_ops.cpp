@@ -290,7 +290,8 @@ void unified_attention(const Tensor& q_in, const Tensor& kv_cache, Tensor& o, co
   const int64_t window = std::max<int64_t>(0, window_size);
   const int64_t n = fxpr_attention_plan(code_of(t), int(num_requests), num_tokens, int(num_heads), int(num_kv_heads),
                                         int(head_dim), int(page_size), int(max_query_len), int(max_blocks),
-                                        k_cache.stride(1), v_cache.stride(1), int(int_bits), int(num_kv_splits), nullptr);
+                                        k_cache.stride(1), v_cache.stride(1), is_causal ? 1 : 0, int(window), int(int_bits),
+                                        int(num_kv_splits), nullptr);
   Tensor ws = n > 0 ? bytes(n, q) : Tensor();
   check_rc(fxpr_unified_attention(
                q.const_data_ptr(), k_cache.const_data_ptr(), v_cache.const_data_ptr(), out.mutable_data_ptr(), code_of(t),

@@ -64,7 +64,8 @@ SIGNATURES: dict[str, list] = {
 # entry points that return something other than an int status
 RESTYPES = {
     "fxpr_gemm_workspace_bytes": ([_L, _L, _L, _I, _I, _I], _L),
-    "fxpr_attention_plan": ([_I, _I, _L, _I, _I, _I, _I, _I, _I, _L, _L, _I, _I, ctypes.POINTER(ctypes.c_int32)], _L),
+    "fxpr_attention_plan": ([_I, _I, _L, _I, _I, _I, _I, _I, _I, _L, _L, _I, _I, _I, _I,
+                             ctypes.POINTER(ctypes.c_int32)], _L),
     "fxpr_attention_workspace_bytes": ([_I, _L, _I, _I, _I, _I, _I, _I, _I, _I], _L),
     "fxpr_sample_greedy_workspace_bytes": ([_L, _I], _L),
 }

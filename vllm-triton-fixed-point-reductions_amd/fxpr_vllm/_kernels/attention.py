@@ -114,8 +114,8 @@ def unified_attention_fxp_run(
     else:
         ws_bytes = _hip.load().fxpr_attention_plan(
             _hip.DTYPE_CODE[q.dtype], num_requests, num_tokens, num_heads, num_kv_heads, head_dim, page_size,
-            int(max_query_len), max_blocks, k_cache.stride(1), v_cache.stride(1), int(fxp_int_bits),
-            int(num_kv_splits), None)
+            int(max_query_len), max_blocks, k_cache.stride(1), v_cache.stride(1), int(bool(is_causal)),
+            max(0, int(window_size)), int(fxp_int_bits), int(num_kv_splits), None)
         ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes > 0 else None
         _hip.call("fxpr_unified_attention", *common, _hip.ptr(ws), ws_bytes, _hip.stream_ptr(q.device))
     if out is not o:
