@@ -232,3 +232,22 @@ def test_ragged_widths_equal_element_loads(dtype, bits, frac, cols):
     for k in {0, min(5, cols), min(64, cols)}:
         for a, b in zip(*(torch.ops.fxpr.sample_greedy_fxp(t, k, bits, frac) for t in (x, off))):
             assert torch.equal(a.double().nan_to_num(7.0), b.double().nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bits,frac", [(32, 16), (64, 32)])
+@pytest.mark.parametrize("cols", [255, 4001, 16001, 33001, 71049, 100003])
+def test_ragged_widths_one_workgroup_per_row(dtype, bits, frac, cols):
+    # more rows than the sampler spreads over workgroups: rows whose vectors a
+    # thread keeps in registers all of, some of and few of, against element loads
+    rows = 131
+    x = (torch.randn(rows, cols, generator=torch.Generator("cpu").manual_seed(cols)) * 4)
+    x[1], x[2, 7], x[130, cols - 1] = float("-inf"), float("nan"), float("inf")
+    x = x.to(dtype).cuda()
+    off = torch.empty(rows * cols + 1, dtype=dtype, device="cuda")[1:].view(rows, cols).copy_(x)
+    assert off.data_ptr() % 16 and x.data_ptr() % 16 == 0
+    a, b = (torch.ops.fxpr.log_softmax_fxp(t, bits, frac, torch.float32) for t in (x, off))
+    assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)) and torch.equal(a.isnan(), b.isnan())
+    for k in (0, 5):
+        for a, b in zip(*(torch.ops.fxpr.sample_greedy_fxp(t, k, bits, frac) for t in (x, off))):
+            assert torch.equal(a.double().nan_to_num(7.0), b.double().nan_to_num(7.0))

@@ -709,13 +709,14 @@ bool try_lsm_split(const void* x, void* y, int64_t rows, int64_t cols, int frac,
   return true;
 }
 
-template <int XDT, int YDT, int VEC, bool RAG>
+// (SHORT: rag_is_short)
+template <int XDT, int YDT, int VEC, bool RAG, bool SHORT = false>
 int launch_lsm_vec(const void* x, void* y, int64_t rows, int64_t cols, int bits, int frac,
                    hipStream_t st) {
   using XT = typename Io<XDT>::T;
   using YT = typename Io<YDT>::T;
-  constexpr int NREG = VEC == 1 ? 8 : 32;
-  const LseShape sh = lse_shape(cols, VEC, NREG, bits, frac);
+  constexpr int NREG = lse_regs(VEC, SHORT);
+  const LseShape sh = lse_shape(cols, VEC, lse_vectors(VEC, SHORT), bits, frac);
   // (128-bit sums, for near-flat rows at large f, keep the one-workgroup kernel)
   if constexpr (VEC > 1 && !RAG) {
     int rc = FXPR_OK;
@@ -748,6 +749,7 @@ int launch_lsm(const void* x, void* y, int64_t rows, int64_t cols, int bits, int
   constexpr int VEC = 16 / sizeof(XT);
   if (aligned(x, 16) && aligned(y, sizeof(YT) * VEC)) {
     if (cols % VEC == 0) return launch_lsm_vec<XDT, YDT, VEC, false>(x, y, rows, cols, bits, frac, st);
+    if (rag_is_short(rows, cols, VEC)) return launch_lsm_vec<XDT, YDT, VEC, true, true>(x, y, rows, cols, bits, frac, st);
     return launch_lsm_vec<XDT, YDT, VEC, true>(x, y, rows, cols, bits, frac, st);
   }
   return launch_lsm_vec<XDT, YDT, 1, false>(x, y, rows, cols, bits, frac, st);

@@ -310,10 +310,26 @@ inline bool lse_fast_sum(int bits, int frac, double lane_elems) {
   return bits != 64 && term_max < 4194304.0 && term_max < qmax && lane_elems * term_max < 4294967296.0;
 }
 
-inline LseShape lse_shape(int64_t cols, int vec, int nreg, int bits, int frac) {
+// One-workgroup kernels: vectors a thread keeps in registers (later ones are
+// read again, from cache), and how many of them the thread count is chosen for.
+// Rows of whole vectors keep up to 32, with few threads for narrow ones. Rows
+// that share vectors (RAG) have no form of several workgroups beside this one,
+// so occupancy decides: 8 kept, a thread for every 4. Kept and shaped like the
+// others they took, against element loads / against this, us: sampler 129 x
+// 16001 bf16 62, 21, 16; 2000 x 33001 f32 244, 173, 110; log-softmax 16 x 16001
+// bf16 27, 15, 8. Few long ones keep 32 as well, one workgroup to a CU either
+// way (129 x 100003 f32 log-softmax 47 us, 64 with 8; at 600 rows 8 is no slower).
+constexpr int64_t kRagLongVectors = 10000, kRagLongRows = 256;
+constexpr int lse_regs(int vec, bool rag_short) { return vec == 1 || rag_short ? 8 : 32; }
+constexpr int lse_vectors(int vec, bool rag_short) { return rag_short ? 4 : lse_regs(vec, rag_short); }
+inline bool rag_is_short(int64_t rows, int64_t cols, int vec) {
+  return rows > kRagLongRows || cols / vec < kRagLongVectors;
+}
+
+inline LseShape lse_shape(int64_t cols, int vec, int per_thread, int bits, int frac) {
   LseShape s;
   const int64_t nchunks = cols / vec + (cols % vec ? 2 : 0);  // (RowVecs: partial vectors at both ends)
-  s.threads = threads_for(nchunks, nreg, kLsmThreads);
+  s.threads = threads_for(nchunks, per_thread, kLsmThreads);
   const double term_max = std::fmin(1.4143 * std::ldexp(1.0, frac) + 1.0, double(qmax_for_bits(bits)));
   s.fast_sum = lse_fast_sum(bits, frac, double(cdiv(nchunks, s.threads)) * vec);
   s.wide = double(cols) * term_max >= 18446744073709551616.0;

@@ -383,7 +383,8 @@ bool try_sample_multi(const void* x, int64_t rows, int64_t cols, int k, int bits
   return true;
 }
 
-template <int XDT, int VEC, bool RAG>
+// (SHORT: rag_is_short)
+template <int XDT, int VEC, bool RAG, bool SHORT = false>
 int launch_sample_vec(const void* x, int64_t rows, int64_t cols, int k, int bits, int frac, int64_t* sampled,
                       float* sampled_lp, int64_t* topk_ids, float* topk_lp, void* ws, int64_t ws_bytes,
                       hipStream_t st) {
@@ -392,8 +393,8 @@ int launch_sample_vec(const void* x, int64_t rows, int64_t cols, int k, int bits
                                  st, &rc))
     return rc;
   using XT = typename Io<XDT>::T;
-  constexpr int NREG = VEC == 1 ? 8 : 32;
-  const LseShape sh = lse_shape(cols, VEC, NREG, bits, frac);
+  constexpr int NREG = lse_regs(VEC, SHORT);
+  const LseShape sh = lse_shape(cols, VEC, lse_vectors(VEC, SHORT), bits, frac);
   const float inv = pow2f(-frac);
   const int rounds = k > 1 ? k : 1;
   dim3 grid(static_cast<unsigned>(rows));
@@ -419,6 +420,9 @@ int launch_sample(const void* x, int64_t rows, int64_t cols, int k, int bits, in
     if (cols % VEC == 0)
       return launch_sample_vec<XDT, VEC, false>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp,
                                                 ws, ws_bytes, st);
+    if (rag_is_short(rows, cols, VEC))
+      return launch_sample_vec<XDT, VEC, true, true>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids,
+                                                     topk_lp, ws, ws_bytes, st);
     return launch_sample_vec<XDT, VEC, true>(x, rows, cols, k, bits, frac, sampled, sampled_lp, topk_ids, topk_lp, ws,
                                              ws_bytes, st);
   }
