@@ -670,3 +670,19 @@ def test_gemm_partial_last_k_tile(dtype, b_layout, M, N, K, bits, frac):
     for split_k in (0, 1, 2):
         got = KG.gemm_fxp_run(wide[:, :K], bd, None, bits, frac, split_k=split_k).cpu()
         assert torch.equal(got, want), mismatch_report(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 264, 128), (16, 8200, 136), (5, 256, 392), (17, 136, 256), (64, 264, 520), (130, 392, 72)])
+def test_gemm_row_major_b_exact_rounding(dtype, M, N, K):
+    # 64-bit sums at f = 32, rounded exactly at every K-tile: the register-staged
+    # tiles, skinny up to M = 16, unsplit, split and with the automatic count of
+    # the native launchers; random values against the K-contiguous kernel
+    g = torch.Generator("cpu").manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).to(dtype)
+    b = (torch.randn(K, N, generator=g) * 0.05).to(dtype)
+    want = _run(a, b, bits=64, frac=32, b_layout="nk")
+    for split_k in (0, 1, 2):
+        assert torch.equal(_run(a, b, bits=64, frac=32, split_k=split_k, b_layout="kn"), want), split_k
+    got = torch.ops.fxpr.gemm_fxp(a.to(DEV), b.to(DEV), None, 64, 32)
+    assert torch.equal(got.cpu(), want)

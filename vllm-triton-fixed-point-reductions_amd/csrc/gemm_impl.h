@@ -1438,7 +1438,7 @@ inline F32Plan f32_plan(int64_t M, int64_t N, int ktiles, int requested) {
 }
 
 // Instantiation matrix of the register-staged tiles: the vectorised paths get
-// a skinny and a square tile; misaligned / ragged operands (scalar loads) use
+// a skinny (row-major B: 64-bit sums only) and a square tile; misaligned / ragged operands (scalar loads) use
 // the square tile only. Tile choice never changes bits.
 template <int DT, int BITS>
 int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipStream_t st) {
@@ -1475,6 +1475,21 @@ int dispatch_tile(const GemmArgs& a, bool b_ncontig, bool vec, int splits, hipSt
         return launch_big<DT, BITS, TB2, BNC>(a, splits, st);
       }
     };
+    // 64-bit sums at f > 20: no K-tile stays in the rounding constant's range, and
+    // the kernel computes each twice. A row-major B then runs faster on the
+    // register-staged tiles, which round exactly at once, from two K-tiles a split
+    // on (bf16, f = 32, us, DMA kernel / these: 1000 x 4096 x 4096 480 / 391, 64 x
+    // 4096 x 4096 95 / 73, 256 x 512 x 14336 94 / 76; one K-tile a split, 64 x 4096
+    // x 2048 45 / 49), and few rows on the skinny tile where its columns fill the
+    // GPU (16 x 4096 x 14336 198 / 131, 16 x 4096 x 4096 71 / 46, 62 on the square
+    // one; 16 x 4096 x 1024 37 / 42, 34 on the square one).
+    if constexpr (BITS == 64) {
+      if (vec && b_ncontig && a.fast_lim < 4.0f) {
+        if (a.M <= 16 && (a.N > 8192 ? a.ktiles >= 4 : a.N > 2048 && a.ktiles >= 16))
+          return launch_cfg<DT, BITS, T16, true, true>(a, splits, st);
+        if (a.tiles_per_split >= 2) return launch_cfg<DT, BITS, TBig, true, true>(a, splits, st);
+      }
+    }
     if (big_ok) return b_ncontig ? big(std::true_type{}) : big(std::false_type{});
   }
   if constexpr (DT == FXPR_DTYPE_F32) {

@@ -231,8 +231,11 @@ Tensor gemm(const Tensor& a_in, const Tensor& b_in, const std::optional<Tensor>&
   }
   const int code = code_of(t), bits = int(int_bits);
   // a row-major B runs on the large-M kernel's tiles at every M: the split
-  // count its policy gives a row of them, not the streaming kernel's (none)
-  const int split_k = M <= 16 && b.stride(0) != 1 && K > 1 ? fxpr_gemm_splits(17, N, K, code, bits, 0) : 0;
+  // count its policy gives a row of them, not the streaming kernel's (none).
+  // (64-bit sums at f > 20 run the skinny tile, whose own count is the automatic
+  // one where the streaming kernel's columns end)
+  const bool own_count = bits == 64 && frac_bits > 20 && N > 8192;
+  const int split_k = M <= 16 && b.stride(0) != 1 && K > 1 && !own_count ? fxpr_gemm_splits(17, N, K, code, bits, 0) : 0;
   const int64_t n = fxpr_gemm_workspace_bytes(M, N, K, code, bits, split_k);
   Tensor ws = n > 0 ? bytes(n, a) : Tensor();
   check_rc(fxpr_gemm(a.const_data_ptr(), b.const_data_ptr(), bias32.defined() ? bias32.const_data_ptr<float>() : nullptr,
