@@ -238,6 +238,14 @@ int fxpr_gemm_finish(const void* acc, const float* bias, void* c,
 int fxpr_gemm_splits(int64_t m, int64_t n, int64_t k, int io_dtype,
                      int int_bits, int split_k);
 
+/* The split count that suits operands with these strides (elements), to be
+ * passed to fxpr_gemm and fxpr_gemm_workspace_bytes: fxpr_gemm's automatic
+ * choice knows the shape only, and is another one for a row-major B at
+ * m <= 16 and for fp32 operands whose strides are no multiple of 4. */
+int fxpr_gemm_layout_splits(int64_t m, int64_t n, int64_t k, int io_dtype,
+                            int int_bits, int frac_bits, int64_t stride_am,
+                            int64_t stride_bk, int64_t stride_bn);
+
 /* Workspace bytes fxpr_gemm needs for this shape and request (0 = none).
  * Replaces the persistent scratch of gemm.py:61-107. */
 int64_t fxpr_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k,

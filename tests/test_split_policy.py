@@ -317,6 +317,35 @@ def test_gemm_f32_split_fills_whole_rounds(lib):
     assert gemm_splits(lib, 130, 4096, 100, F32) <= 2        # 2 K-tiles
 
 
+def test_gemm_layout_splits(lib):
+    def layout(m, n, k, dt=BF16, bits=32, frac=16, lda=None, row_major=False, ldb=None):
+        lda, ldb = lda or k, ldb or (n if row_major else k)
+        bk, bn = (ldb, 1) if row_major else (1, ldb)
+        return lib.fxpr_gemm_layout_splits(m, n, k, dt, bits, frac, lda, bk, bn)
+
+    # K-contiguous operands: the shape's own count
+    for m, n, k in ((1, 4096, 4096), (16, 8193, 4096), (32, 28672, 4096), (130, 4096, 14336)):
+        for dt in (BF16, F32):
+            assert layout(m, n, k, dt) == gemm_splits(lib, m, n, k, dt)
+    # a row-major B at M <= 16: a row of the large-M kernel's tiles (32 of them)
+    assert layout(1, 4096, 4096, row_major=True) == 16 and gemm_splits(lib, 1, 4096, 4096) == 1
+    assert layout(16, 28672, 4096, row_major=True) == 4
+    assert layout(17, 4096, 4096, row_major=True) == gemm_splits(lib, 17, 4096, 4096)
+    # 64-bit sums at f = 32 beyond 8192 columns: the skinny tile's (56 tiles of 256)
+    assert layout(16, 14336, 4096, bits=64, frac=32, row_major=True) == 9
+    assert layout(16, 14336, 4096, bits=64, frac=16, row_major=True) == 4
+    assert layout(16, 8192, 4096, bits=64, frac=32, row_major=True) == 8
+    # fp32: the DMA kernel's plan, or 512 / (tiles of 128 x 128) where rows cannot
+    # be 16-byte aligned
+    assert layout(1852, 500, 856, F32, row_major=True) == gemm_splits(lib, 1852, 500, 856, F32)
+    assert layout(1852, 499, 856, F32, row_major=True) == 8          # 60 tiles
+    assert layout(1852, 500, 856, F32, row_major=True, ldb=501) == 8
+    assert layout(1852, 499, 856, F32, ldb=857) == 8
+    assert layout(1852, 499, 856, F32, lda=858) == 8
+    assert layout(1852, 499, 856, F32) == gemm_splits(lib, 1852, 499, 856, F32)
+    assert layout(0, 4, 4) == 1
+
+
 def test_gemm_auto_decode_shapes_with_a_k_tail(lib):
     # the streaming kernel takes whole K-tiles only; other K split the skinny tile
     assert gemm_splits(lib, 1, 4096, 4096 + 16) == 16     # 16 tiles of 16 x 256

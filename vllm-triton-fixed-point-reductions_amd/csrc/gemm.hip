@@ -10,6 +10,12 @@ extern "C" int fxpr_gemm_splits(int64_t m, int64_t n, int64_t k, int io_dtype, i
   return resolve_splits(m, n, k, io_dtype, int_bits, split_k);
 }
 
+extern "C" int fxpr_gemm_layout_splits(int64_t m, int64_t n, int64_t k, int io_dtype, int int_bits, int frac_bits,
+                                       int64_t stride_am, int64_t stride_bk, int64_t stride_bn) {
+  if (m <= 0 || n <= 0 || k < 0) return 1;
+  return layout_splits(m, n, k, io_dtype, int_bits, frac_bits, stride_am, stride_bk, stride_bn);
+}
+
 extern "C" int64_t fxpr_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int io_dtype,
                                              int int_bits, int split_k) {
   if (m <= 0 || n <= 0 || k < 0) return 0;

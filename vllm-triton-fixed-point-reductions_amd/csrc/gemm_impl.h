@@ -1523,7 +1523,9 @@ inline int ktile_for(int io_dtype) { return io_dtype == FXPR_DTYPE_F32 ? 64 : 12
 // N <= 8192), and elsewhere a split only when the output tiles (of the
 // kernel the shape and accumulator width take) cannot fill the 256 CUs about
 // twice: 512 / tiles splits, at most 16.
-inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int_bits, int requested) {
+// (f32_dma: fp32 operands that the DMA kernel takes, as far as the caller knows)
+inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int_bits, int requested,
+                          bool f32_dma = true) {
   const int ktiles = int(cdiv(K, ktile_for(io_dtype)));
   if (ktiles <= 1) return 1;
   int s;
@@ -1536,7 +1538,7 @@ inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int
     if (io_dtype != FXPR_DTYPE_F32 && stream_shape(M, N) && K % 128 == 0) return 1;
     // fp32 beyond M = 32 (K a multiple of a chunk: other rows cannot be
     // 16-byte aligned and take the register-staged tiles)
-    if (io_dtype == FXPR_DTYPE_F32 && M > 32 && K % 4 == 0) return f32_plan(M, N, ktiles, 0).splits;
+    if (io_dtype == FXPR_DTYPE_F32 && M > 32 && K % 4 == 0 && f32_dma) return f32_plan(M, N, ktiles, 0).splits;
     int bm = 128, bn = 128;  // TB2, TB64, TBig
     if (io_dtype != FXPR_DTYPE_F32 && ts64_rows(M, int_bits)) {
       bm = TS64::BM;
@@ -1551,6 +1553,26 @@ inline int resolve_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int
   }
   if (s > ktiles) s = ktiles;
   return s < 1 ? 1 : s;
+}
+
+// The automatic count for operands laid out like this.
+//   * A row-major 16-bit B at M <= 16 runs on the large-M kernel's tiles: the
+//     count of a row of them, not the streaming kernel's (none). 64-bit sums at
+//     f > 20 run on the skinny tile there, whose own count is the automatic one
+//     where the streaming kernel's columns end.
+//   * fp32 operands that cannot be 16-byte aligned take the register-staged tiles:
+//     512 / (output tiles), not the DMA kernel's plan (row-major 1852 x 856 x 499:
+//     130 us with its count, 56; 2318 x 1696 x 825, 64-bit sums 301 and 216).
+inline int layout_splits(int64_t M, int64_t N, int64_t K, int io_dtype, int int_bits, int frac_bits, int64_t stride_am,
+                         int64_t stride_bk, int64_t stride_bn) {
+  const bool row_major = stride_bk != 1 && K > 1;
+  if (row_major && M <= 16) {
+    const bool own_count = io_dtype != FXPR_DTYPE_F32 && int_bits == 64 && frac_bits > 20 && N > 8192;
+    return resolve_splits(own_count ? M : 17, N, K, io_dtype, int_bits, 0);
+  }
+  const bool f32_dma = (stride_am % 4 == 0 || M == 1) &&
+                       (row_major ? N % 4 == 0 && stride_bk % 4 == 0 : stride_bn % 4 == 0 || N == 1);
+  return resolve_splits(M, N, K, io_dtype, int_bits, 0, f32_dma);
 }
 
 inline int64_t ws_bytes_for(int64_t M, int64_t N, int int_bits, int splits) {

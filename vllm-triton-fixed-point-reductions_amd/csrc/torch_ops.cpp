@@ -230,12 +230,8 @@ Tensor gemm(const Tensor& a_in, const Tensor& b_in, const std::optional<Tensor>&
     bias32 = bias->reshape({N}).to(at::kFloat).contiguous();
   }
   const int code = code_of(t), bits = int(int_bits);
-  // a row-major B runs on the large-M kernel's tiles at every M: the split
-  // count its policy gives a row of them, not the streaming kernel's (none).
-  // (64-bit sums at f > 20 run the skinny tile, whose own count is the automatic
-  // one where the streaming kernel's columns end)
-  const bool own_count = bits == 64 && frac_bits > 20 && N > 8192;
-  const int split_k = M <= 16 && b.stride(0) != 1 && K > 1 && !own_count ? fxpr_gemm_splits(17, N, K, code, bits, 0) : 0;
+  const int split_k =
+      fxpr_gemm_layout_splits(M, N, K, code, bits, int(frac_bits), a.stride(0), b.stride(0), b.stride(1));
   const int64_t n = fxpr_gemm_workspace_bytes(M, N, K, code, bits, split_k);
   Tensor ws = n > 0 ? bytes(n, a) : Tensor();
   check_rc(fxpr_gemm(a.const_data_ptr(), b.const_data_ptr(), bias32.defined() ? bias32.const_data_ptr<float>() : nullptr,

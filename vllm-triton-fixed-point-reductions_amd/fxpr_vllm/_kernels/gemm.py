@@ -59,14 +59,9 @@ def gemm_fxp_run(a: torch.Tensor, b: torch.Tensor, bias: torch.Tensor | None, in
 
     lib = _hip.load()
     code = _hip.DTYPE_CODE[a.dtype]
-    own_count = int(int_bits) == 64 and int(fxp_frac_bits) > 20 and N > 8192
-    if split_k == 0 and M <= 16 and b.stride(0) != 1 and K > 1 and not own_count:
-        # a row-major B runs on the large-M kernel's tiles at every M: the
-        # split count its policy gives a row of them, not the streaming
-        # kernel's (none). (64-bit sums at f > 20 run the skinny tile, whose
-        # own count is the automatic one where the streaming kernel's columns
-        # end)
-        split_k = lib.fxpr_gemm_splits(17, N, K, code, int(int_bits), 0)
+    if split_k == 0:
+        split_k = lib.fxpr_gemm_layout_splits(M, N, K, code, int(int_bits), int(fxp_frac_bits), a.stride(0), b.stride(0),
+                                              b.stride(1))
     ws_bytes = lib.fxpr_gemm_workspace_bytes(M, N, K, code, int(int_bits), int(split_k))
     ws = torch.empty(ws_bytes, device=a.device, dtype=torch.uint8) if ws_bytes > 0 else None
     _hip.call(
