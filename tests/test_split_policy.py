@@ -189,13 +189,13 @@ def test_attention_short_requests_splits(lib):
 
 
 def test_attention_few_rows_take_the_16_row_split(lib):
-    # up to 320 rows (tokens x group) and 3000 units over tables of up to 16384
+    # up to 256 rows (tokens x group) and 3000 units over tables of up to 16384
     # keys, where the plain policy splits: its launch, long requests included
     assert attn_plan(lib, 3, 28, 26, 2528) == (ROWS16_DMA, 5, 5, 0, record_bytes(28, 2528))
-    assert attn_plan(lib, 1, 80, 80, 4096)[0] == ROWS16_DMA             # 320 rows
-    assert attn_plan(lib, 1, 81, 81, 4096)[0] == LONG_DMA
-    assert attn_plan(lib, 1, 80, 80, 8320)[0] == ROWS16_DMA             # 8 x 21 x 17 = 2856 units
-    assert attn_plan(lib, 1, 80, 80, 8704 + 16)[0] == LONG_DMA          # 18 chunks: 3024
+    assert attn_plan(lib, 1, 64, 64, 4096)[0] == ROWS16_DMA             # 256 rows
+    assert attn_plan(lib, 1, 65, 65, 4096)[0] == LONG_DMA
+    assert attn_plan(lib, 1, 64, 64, 11264)[0] == ROWS16_DMA            # 8 x 17 x 22 = 2992 units
+    assert attn_plan(lib, 1, 64, 64, 11264 + 16)[0] == LONG_DMA         # 23 chunks: 3128
     assert attn_plan(lib, 3, 28, 26, 2048)[0] == LONG_DMA               # nothing splits
     assert attn_plan(lib, 3, 28, 26, 32768)[0] == LONG_DMA              # wide
     assert attn_plan(lib, 3, 28, 26, 2528, requested=2)[0] == LONG_DMA  # explicit

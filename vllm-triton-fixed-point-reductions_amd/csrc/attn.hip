@@ -126,9 +126,9 @@ SplitPlan launch_plan(int num_requests, int64_t num_tokens, int num_heads, int n
 //     the short requests' split, 340 without).
 // Against the plan before requests were split apart (us before / now, geometric
 // mean): drawn batches with prompts, tables as wide as their longest context (up
-// to 12288 keys) 1.40x, 10 of 272 more than 3 % slower, the worst 1.18x; tables of
-// 8192 keys 1.52x, 9 of 78, 1.6x (83 decode steps under 300 keys beside 3 x 79
-// tokens, 36 -> 58); 32768 1.9x, 8 of 101, 1.34x; 131072 2.1x, 2 of 74, 1.06x.
+// to 12288 keys) 1.40x, 7 of 272 more than 3 % slower, the worst 1.24x; tables of
+// 8192 keys 1.53x, 8 of 78, 1.6x (83 decode steps under 300 keys beside 3 x 79
+// tokens, 36 -> 58); 32768 1.9x, 7 of 101, 1.35x; 131072 2.1x, 1 of 74, 1.06x.
 // Explicit requests split both that many times. Records need a workspace: per
 // token when the prefill rows are split, else only for the short requests'
 // tokens. Above kLongWsMax the launch runs unsplit; above kSplitWsMax where the
@@ -211,7 +211,7 @@ LongLayout long_plan(int num_requests, int64_t num_tokens, int num_heads, int nu
 }
 
 // rows (tokens x group) and 16-row chunk units up to which a batch counts as few
-constexpr int64_t kFewRows = 320, kFewChunks = 3000;
+constexpr int64_t kFewRows = 256, kFewChunks = 3000;
 
 // What a launch runs: its kernels, its splits and the records they need.
 struct LaunchPlan {
@@ -240,8 +240,10 @@ LaunchPlan attention_plan(int io_dtype, int num_requests, int64_t num_tokens, in
   // A few tokens in all, over tables that are not wide: one split launch of
   // 16-row workgroups spreads them further than 64-row ones, and takes two
   // launches instead of three. Both sides, us: 28 tokens in 3 requests over up to
-  // 2500 keys (32/8 heads of 128) 23 against 42 apart; 79 in 8 with a softcap 45
-  // and 69; 140 of 24/8 heads of 64 over 2400 47 and 38 (420 rows: apart).
+  // 2500 keys (32/8 heads of 128) 23 against 42 apart; 45 in 14 beside 4096 cached
+  // ones under a window of 1024 26 and 43; 77 in 3 over 6000 59 and 38 (308 rows:
+  // apart). Over 348 drawn batches of up to 500 rows the rule is within 2 % of the
+  // better of the two on average, always apart 7 %.
   const int64_t rows = num_tokens * group;
   const int64_t chunks = cdiv(window > 0 ? std::min<int64_t>(keys, window + max_query_len) : keys, TILE * CT);
   const bool few_rows = requested == 0 && p.sp.splits > 1 && keys <= kWideKeys && rows <= kFewRows &&
